@@ -340,38 +340,64 @@ __device__ __forceinline__ double rec_coef_col(const RecArgs &a, int p, int pp) 
   return (k - 1) * a.lnxi - a.beta * E - ln_n;
 }
 
-// rec_coef without branches (ok false: NEG), so that unrolled callers issue
-// their loads together.
+// rec_coef_col for the columns pp0 + j, j < min(n, 16), of row p: E and ln n
+// loaded by rec_load16, all loads issued before any is used (clamped indices
+// instead of branches, which would make each load wait for the one before),
+// and made coefficients by rec_conv16, so that callers can keep the loads in
+// flight across other work.  act false or j >= n: NEG.  pp0 is wave-uniform,
+// so that the address of a column is scalar work and a load one vector
+// instruction: with per-lane 64-bit addresses the solver's loop body outgrew
+// the instruction cache (60 KB of code per block, every phase three times its
+// issue time).
+struct RecRaw {
+  double E[16], ln;  // ln: forward ln p, the same for every column; backward ln of column pp0 + (lane mod 16)
+};
+
 template <bool FWD>
-__device__ __forceinline__ double rec_coef_nb(const RecArgs &a, int p, int pp, bool ok) {
-  const int k = p - pp;
-  ok = ok && !(a.xi0 && k != 1);
-  const size_t idx = ok ? (FWD ? tri_row(p) : col_off(a.N - p, a.N)) + k - 1 : 0;
-  const double E = FWD ? a.ENk[idx] : a.ET[idx];
-  const double ln_n = a.lnn[ok ? (FWD ? p : a.N - pp) : 0];
-  return ok ? (k - 1) * a.lnxi - a.beta * E - ln_n : NEG;
+__device__ __forceinline__ void rec_load16(const RecArgs &a, int p, int pp0, RecRaw &x) {
+  const int N = a.N, pn = min(p, N);
+  // element (p, pp) sits at base[d + p], d >= 0 the column's offset from the
+  // lowest-addressed column of the 16 (the first forward, the last backward);
+  // columns past N - 1 read column N - 1, rows above the diagonal the
+  // column's first element
+  const int pf = min(FWD ? pp0 : pp0 + 15, N - 1);
+  const double *base = (FWD ? a.ET + col_off(pf, N) : a.ENk + tri_row(N - pf)) - (pf + 1);
+  int d = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int j = FWD ? i : 15 - i, pp = min(pp0 + j, N - 1);
+    x.E[j] = base[(unsigned)(max(pn, pp + 1) + d)];
+    if (FWD)
+      d += pp0 + j < N - 1 ? N - pp - 1 : 0;
+    else
+      d += pp0 + j - 1 < N - 1 ? N - pp0 - j + 1 : 0;
+  }
+  x.ln = a.lnn[FWD ? pn : max(0, N - pp0 - (int)(threadIdx.x & 15))];
 }
 
-// rec_coef_col for the 16 columns pp0 .. pp0+15 of row p, all loads issued
-// before any is used (clamped indices instead of branches, which would make
-// each load wait for the one before); act false: every coefficient NEG.
+template <bool FWD>
+__device__ __forceinline__ void rec_conv16(const RecArgs &a, int p, int pp0, int n, bool act, const RecRaw &x,
+                                           double *c) {
+  // coefficients exist for jlo <= j < jlo + cnt (xi = 0: only the column with k = 1)
+  const int jlo = a.xi0 ? p - 1 - pp0 : 0;
+  const unsigned cnt = !act ? 0 : a.xi0 ? (jlo < n ? 1 : 0) : max(0, n);
+  const int k0 = p - pp0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int k = k0 - j;
+    const double ln = FWD ? x.ln : readlane_d(x.ln, j);
+    // the contraction hipcc picks for rec_coef's expression, spelled out so
+    // that every copy of a coefficient is the same to the last bit
+    const double v = fma((double)(k - 1), a.lnxi, -(a.beta * x.E[j])) - ln;
+    c[j] = (unsigned)(j - jlo) < cnt ? v : NEG;
+  }
+}
+
 template <bool FWD>
 __device__ __forceinline__ void rec_coef_col16(const RecArgs &a, int p, int pp0, bool act, double *c) {
-  double E[16], ln[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int pp = pp0 + j, k = p - pp;
-    const bool ok = act && !(a.xi0 && k != 1);
-    const size_t idx = ok ? (FWD ? col_off(pp, a.N) : tri_row(a.N - pp)) + k - 1 : 0;
-    E[j] = FWD ? a.ET[idx] : a.ENk[idx];
-    ln[j] = a.lnn[ok ? (FWD ? p : a.N - pp) : 0];
-  }
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int pp = pp0 + j, k = p - pp;
-    const bool ok = act && !(a.xi0 && k != 1);
-    c[j] = ok ? (k - 1) * a.lnxi - a.beta * E[j] - ln[j] : NEG;
-  }
+  RecRaw x;
+  rec_load16<FWD>(a, p, pp0, x);
+  rec_conv16<FWD>(a, p, pp0, 16, act, x, c);
 }
 
 // DIRECT: coefficients from positions and prefix sums (rec_coef_direct, e
@@ -530,15 +556,31 @@ __device__ __forceinline__ void lse_pair(double &M, double &S, double m, double 
   }
 }
 
-// Two-pass log-sum-exp of 16 terms held by this lane.
-__device__ __forceinline__ void lse16(const double *t, double &M, double &S) {
+// exp of an exponent that may be absent (ok false: 0 exactly), without the
+// branch a conditional exp becomes.
+__device__ __forceinline__ double exp_if(bool ok, double x) { return exp(ok ? x : -2000.0); }
+
+// Log-sum-exp of 16 terms t_j of this lane, kept at buf[64 j] (LDS): the
+// exponentials run in a rolled loop, whose constants stay in registers (26
+// instead of 46 instructions each when unrolled).
+__device__ __forceinline__ void lse16(const double *t, double *buf, double &M, double &S) {
   M = NEG;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) M = fmax(M, t[j]);
+  for (int j = 0; j < 16; ++j) {
+    M = fmax(M, t[j]);
+    buf[RB * j] = t[j];
+  }
   S = 0.0;
-  if (M > NEG) {
+  const bool any = M > NEG;
+#pragma unroll 1
+  for (int j = 0; j < 16; j += 4) {
+    double e[4];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) S += (t[j] > M - LSE_SKIP) ? exp(t[j] - M) : 0.0;
+    for (int i = 0; i < 4; ++i) e[i] = buf[RB * (j + i)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[i] = exp_if(any && e[i] > M - LSE_SKIP, e[i] - M);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S += e[i];
   }
 }
 
@@ -603,12 +645,13 @@ __device__ __forceinline__ void rec_poll(const double *p, const double *q, int n
 // workgroup solved the blocks (its barriers order those stores before these
 // plain loads).  The next block's coefficients are in flight while a block
 // is folded; the four partials of a block merge in wave 0 through
-// double-buffered LDS (one barrier per block).
+// double-buffered LDS (one barrier per block); scr: 64 x 64 doubles of LDS
+// scratch.
 template <bool FWD, bool POLL>
 __device__ __forceinline__ void rec_fold_rows(const RecArgs &a, int dir, int G, double (*pm)[4][RB],
-                                              double (*ps)[4][RB], double &Ma, double &Sa) {
+                                              double (*ps)[4][RB], double *scr, double &Ma, double &Sa) {
   const int N = a.N;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   int *err = a.sync + 4 * a.nblk;
   const double *val = a.val2 + (size_t)dir * (N + 1);
   const double *AM = a.accM + (size_t)dir * (N + 1), *AS = a.accS + (size_t)dir * (N + 1);
@@ -638,7 +681,7 @@ __device__ __forceinline__ void rec_fold_rows(const RecArgs &a, int dir, int G, 
       t[j] = c[j] > NEG ? c[j] + vj : NEG;
     }
     double M, S;
-    lse16(t, M, S);
+    lse16(t, scr + 16 * wv * RB + lane, M, S);
     const int buf = b & 1;
     pm[buf][wv][lane] = M;
     ps[buf][wv][lane] = S;
@@ -652,11 +695,22 @@ __device__ __forceinline__ void rec_fold_rows(const RecArgs &a, int dir, int G, 
   }
 }
 
+struct alignas(16) RecLds {
+  double dg[2][RSQ];            // in-block coefficients [r][q] (ping-pong)
+  double la[RSQ];               // look-ahead weights [r][q] of the next block's rows
+  double sg[RB];                // per-row shifts of an exact block solve
+  double wl[RB];                // W of the block solved last
+  double lv[RB];                // its values L
+  double tacc[4][RB], sacc[4][RB];  // look-ahead partials of the four waves (an exact fold: M and S)
+  int fast;                     // the block's chain-frame solve stayed in range
+  double nm[RB], ns[RB];        // next block's accumulators, loaded by wave 1
+  double pm[2][4][RB], ps[2][4][RB];  // fold partials (updater, or a self-fold in SOLO)
+};
+
 template <bool FWD>
-__device__ __forceinline__ void rec_updater(const RecArgs &a, int dir, int G, double (*pm)[4][RB],
-                                            double (*ps)[4][RB]) {
+__device__ __forceinline__ void rec_updater(const RecArgs &a, int dir, int G, RecLds &S) {
   double Ma, Sa;
-  rec_fold_rows<FWD, true>(a, dir, G, pm, ps, Ma, Sa);
+  rec_fold_rows<FWD, true>(a, dir, G, S.pm, S.ps, S.dg[0], Ma, Sa);
   const int p = 1 + G * RB + (threadIdx.x & 63);
   if (threadIdx.x < 64 && p <= a.N) {
     st_handoff(a.finM + (size_t)dir * (a.N + 1) + p, Ma);
@@ -664,55 +718,66 @@ __device__ __forceinline__ void rec_updater(const RecArgs &a, int dir, int G, do
   }
 }
 
-struct RecLds {
-  double dg[2][RSQ];            // in-block coefficients [r][q] (ping-pong)
-  double sg[RB];                // per-row shifts of an exact block solve
-  double wl[RB];                // W of the block solved last
-  double lv[RB];                // its values L
-  double tacc[4][RB];           // look-ahead partial sums of the four waves
-  double nm[RB], ns[RB];        // next block's accumulators, loaded by wave 1
-  double pm[2][4][RB], ps[2][4][RB];  // fold partials (updater, or a self-fold in SOLO)
-};
-
-// LDS written by some lanes of a wave and read by others of the same wave:
-// the fence keeps the compiler from forwarding or reordering across it.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // Upper end of the chain frame's range (RecArgs::big, lowered only by a
 // test hook): W up to e^575, so no sum of non-negative terms overflows, and
 // a term that underflows is below e^-133 of its row's W (>= 1).
 constexpr double REC_BIG = 1e250;
 
-// Exact solve of row block b by wave 0 alone, without the chain frame:
-// coefficients from the tables, per-row shifts sigma_q = max(M_q, max_{r<q}
-// c(q,r) + sigma_r) by a (max,+) scan (no transcendental on its chain), the
-// scaled exps a(q,r) = exp(c(q,r) + sigma_r - sigma_q) and the substitution
-// W_q = b_q + sum_{r<q} a(q,r) W_r, W_q = exp(L(q) - sigma_q) (every term
-// obeys c(q,r) + L(r) <= L(q) <= sigma_q + (rows) ln N).  Returns L of the
-// lane's row (lane = row, accumulators (M, Sm)).
-template <bool FWD>
-__device__ __forceinline__ double rec_block_exact(const RecArgs &a, int p0, int nrows, double M, double Sm,
-                                                  double *dg, double *sg) {
-  const int lane = threadIdx.x & 63;
-  // lane = row q, element [r][q] = c(q, r) for r < q (NEG otherwise)
-#pragma unroll 16
-  for (int r = 0; r < RB - 1; ++r) dg[r * RB + lane] = rec_coef_nb<FWD>(a, p0 + lane, p0 + r, r < lane && lane < nrows);
-  double sig = lane < nrows ? M : NEG;
-  for (int r = 0; r < RB - 1; ++r) sig = fmax(sig, dg[r * RB + lane] + readlane_d(sig, r));
-  sg[lane] = lane < nrows ? sig : NEG;
-  wave_lds_sync();
-  for (int r = 0; r < RB - 1; ++r) {
-    const double x = dg[r * RB + lane];
-    dg[r * RB + lane] = x > NEG ? exp(x + sg[r] - sig) : 0.0;
-  }
-  double W = 0.0;
-  if (lane < nrows && M > NEG && M > sig - 745.0) W = Sm * exp(M - sig);
-  for (int r = 0; r < RB - 1; ++r) W = fma(dg[r * RB + lane], readlane_d(W, r), W);
-  return sig + log(W);
+// Forward substitution and (max,+) scan of a block by one wave, lane = row q,
+// coefficients at dg[r * RB + q] (0 or NEG unless r < q), columns r in order:
+//   W_q += A(q, r) W_r          until W leaves `big` (NaN too; false then)
+//   sig_q = max(sig_q, c(q, r) + sig_r)
+// The chain per column is one broadcast (two v_readlane) and one or two FP64
+// operations, about 30 cycles, when its operands wait in registers: each
+// group of 16 columns is read from LDS while the group before it is worked off
+// (a read per column at its use costs 85 cycles a column).
+struct RecCols {
+  double d[16];
+};
+
+__device__ __forceinline__ void rec_cols(const double *dg, int r0, RecCols &x) {
+#pragma unroll
+  for (int j = 0; j < 16; ++j) x.d[j] = dg[(r0 + j) * RB + (threadIdx.x & 63)];
 }
+
+__device__ __forceinline__ bool rec_subst(const double *dg, int ncol, double big, double &W) {
+  RecCols x, n;
+  rec_cols(dg, 0, x);
+#pragma unroll 1
+  for (int r0 = 0; r0 < ncol; r0 += 16) {
+    if (!__all(W <= big)) return false;
+    rec_cols(dg, min(r0 + 16, RB - 16), n);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) W = fma(x.d[j], readlane_d(W, r0 + j), W);
+    x = n;
+  }
+  return __all(W <= big);
+}
+
+__device__ __forceinline__ void rec_shift(const double *dg, int ncol, double &sig) {
+  RecCols x, n;
+  rec_cols(dg, 0, x);
+#pragma unroll 1
+  for (int r0 = 0; r0 < ncol; r0 += 16) {
+    rec_cols(dg, min(r0 + 16, RB - 16), n);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sig = fmax(sig, x.d[j] + readlane_d(sig, r0 + j));
+    x = n;
+  }
+}
+
+// Copies a 64 x 64 tile from global memory into LDS by the direct path, 16
+// bytes per lane (a wave's 64 lanes fill 1 KB in lane order), chunk c of 32 by
+// wave c mod 3 of three; rec_copy_wait: this wave's copies have arrived (the
+// caller's barrier then publishes them).
+__device__ __forceinline__ void rec_copy_tile(const double *src, double *dst, int wave) {
+  typedef const __attribute__((address_space(1))) void *gptr;
+  typedef __attribute__((address_space(3))) void *lptr;
+  for (int c = wave; c < RSQ / 128; c += 3)
+    __builtin_amdgcn_global_load_lds((gptr)(src + c * 128 + 2 * (threadIdx.x & 63)), (lptr)(dst + c * 128), 16, 0, 0);
+}
+
+__device__ __forceinline__ void rec_copy_wait() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // The solver walks the blocks in order.  Block b is solved in the frame of
 // its k = 1 chain: row q's unknown is W_q = exp(L(q) - sigma - E(q)), with
@@ -732,16 +797,30 @@ __device__ __forceinline__ double rec_block_exact(const RecArgs &a, int p0, int 
 //           (E', Delta: block b+1's offsets and the step into it, so this is
 //           the log-sum-exp of c(q', r) + L(r) over block b).
 // A block whose W leaves [0, REC_BIG] (a row more than ~575 above its
-// chain, or an overflowed coefficient) fails a wave vote; wave 0 then solves
-// it with rec_block_exact and folds it into block b+1 from its values, as it
-// also does for a row whose look-ahead sum left the range.
+// chain, or an overflowed coefficient) fails a wave vote after the 16 columns
+// that show it (W only grows).  It is then solved exactly, without the chain
+// frame: coefficients from the tables, per-row shifts sigma_q = max(M_q,
+// max_{r<q} c(q,r) + sigma_r) by a (max,+) scan (no transcendental on its
+// chain), the scaled exps a(q,r) = exp(c(q,r) + sigma_r - sigma_q) and the
+// substitution W_q = b_q + sum_{r<q} a(q,r) W_r, W_q = exp(L(q) - sigma_q)
+// (every term obeys c(q,r) + L(r) <= L(q) <= sigma_q + (rows) ln N); and it
+// is folded into block b+1 from its values, as a row whose look-ahead sum
+// left the range also is.  Thermal states take this path in nearly every
+// block (each particle inside a longer cycle lies its ring-closing energy
+// above the chain, 48 at P = 32), so its coefficients are prefetched like the
+// frame's and the four waves share the exps of the solve (16 columns each)
+// and of the fold (its four 16-term log-sum-exps).  What bounds it is the
+// instruction issue of single waves (FP64 at about 6 cycles an instruction,
+// an exp 30 of them) and the serial scan and substitution.  Both directions
+// at UEG N=1024 P=32 with cycles: 755 -> 200 us, 42 -> 11.6 us per block,
+// against one wave loading and exponentiating all of a block.
 // SOLO: no updater workgroups; the solver folds blocks 0 .. b-1 into block
 // b+1 itself (same order and arithmetic as an updater), so it waits on no
 // other workgroup.
 template <bool FWD, bool SOLO = false>
 __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S) {
   const int N = a.N;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   int *err = a.sync + 4 * a.nblk;
   // Test hook: while sync[4 nblk + 1] (set by the host, never by a normal
   // run) is positive, a forward solve takes one from it and its first poll
@@ -760,13 +839,14 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
   const double *DGd = a.dg + (size_t)dir * a.nblk * RSQ;
   const double *LAd = a.la + (size_t)dir * a.nblk * (RB * RB);
   const double *ECd = a.ech + (size_t)dir * a.nblk * (RB + 1);
-  constexpr int DPT = RSQ / 256;           // in-block coefficients per thread
   constexpr int LPW = RB / 4;              // look-ahead columns per lane
   // block 0: coefficients, accumulators (column 0 only), chain offsets
-  for (int w = tid; w < RSQ; w += 256) S.dg[0][w] = DGd[w];
+  const int nr0 = min(RB, N);
+  for (int w = tid; w < (nr0 + 15) / 16 * 16 * RB; w += 256) S.dg[0][w] = DGd[w];
+  RecRaw xd;  // this wave's 16 columns of the block on itself, for an exact solve
+  rec_load16<FWD>(a, 1 + lane, 1 + 16 * wv, xd);
   double M = NEG, Sm = 0.0, E = 0.0, Dl = 0.0;
   if (wv == 0) {
-    const int nr0 = min(RB, N);
     M = lane < nr0 ? AM[1 + lane] : NEG;
     Sm = lane < nr0 ? AS[1 + lane] : 0.0;
     E = ECd[lane];
@@ -777,34 +857,9 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
     const int p0 = 1 + b * RB, nrows = min(RB, N - p0 + 1);
     const bool more = b + 1 < a.nblk;
     const int p1 = p0 + RB, nrows1 = more ? min(RB, N - p1 + 1) : 0;
-    __syncthreads();
-    // block b+1's coefficients, in flight during this block's solve
-    double dgr[DPT], lar[LPW], En = 0.0, Dn = 0.0;
-    if (more) {
-#pragma unroll
-      for (int k = 0; k < DPT; ++k) {
-        const int w = tid + 256 * k;
-        dgr[k] = DGd[(size_t)(b + 1) * RSQ + w];
-      }
-#pragma unroll
-      for (int k = 0; k < LPW; ++k) lar[k] = LAd[(size_t)(b + 1) * (RB * RB) + (wv + 4 * k) * RB + lane];
-      if (wv == 0) {
-        En = ECd[(size_t)(b + 1) * (RB + 1) + lane];
-        Dn = ECd[(size_t)(b + 1) * (RB + 1) + RB];
-      }
-    }
     double *dg = S.dg[cur];
-    double sigma = 0.0;
-    bool fast = true;
-    if (wv == 0) {
-      sigma = readlane_d(M, 0) + log(readlane_d(Sm, 0));
-      double W = lane < nrows ? Sm * exp(M - sigma - E) : 0.0;
-      // column r of dg holds A(q, r) at row q = lane (0 unless r < q)
-#pragma unroll
-      for (int r = 0; r < RB - 1; ++r) W = fma(dg[r * RB + lane], readlane_d(W, r), W);
-      fast = __all(W <= a.big);  // NaN fails too
-      const double v = fast ? sigma + E + log(W) : rec_block_exact<FWD>(a, p0, nrows, M, Sm, dg, S.sg);
-      S.wl[lane] = W;
+    // publishes the block's values: lane = row
+    auto publish = [&](double v) {
       S.lv[lane] = v;
       if (lane < nrows) {
         const int p = p0 + lane;
@@ -816,36 +871,121 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
           a.Rb[N - p] = v;
         }
       }
-    } else if (wv == 1 && !SOLO && more) {
-      // block b+1's accumulators: column 0 (set-up) for block 1, blocks
-      // 0 .. b-1 from its updater otherwise
+    };
+    __syncthreads();
+    // block b+1's frame coefficients into LDS (copied there without passing
+    // registers, by waves 1-3: wave 0's own LDS reads would wait for copies
+    // it had issued), in flight during this block's attempt
+    double En = 0.0, Dn = 0.0;
+    if (more) {
+      if (wv != 0) {
+        rec_copy_tile(DGd + (size_t)(b + 1) * RSQ, S.dg[cur ^ 1], wv - 1);
+        rec_copy_tile(LAd + (size_t)(b + 1) * RSQ, S.la, wv - 1);
+      } else {
+        En = ECd[(size_t)(b + 1) * (RB + 1) + lane];
+        Dn = ECd[(size_t)(b + 1) * (RB + 1) + RB];
+      }
+    }
+    double sigma = 0.0;
+    // block b+1's accumulators (wave 1): column 0 (set-up) for block 1,
+    // blocks 0 .. b-1 from its updater otherwise, waited for beside wave 0's
+    // substitution
+    bool have = SOLO || !more;
+    auto next_acc = [&](bool wait) {
+      if (have || wv != 1) return;
       double m = NEG, sv = 0.0;
-      if (b + 1 >= 2) {
+      if (b + 1 < 2) {
+        if (lane < nrows1) {
+          m = AM[p1 + lane];
+          sv = AS[p1 + lane];
+        }
+      } else if (wait) {
         rec_poll(FM + p1, FS + p1, nrows1, err, spin, m, sv);
         spin = REC_SPIN_MAX;
-      } else if (lane < nrows1) {
-        m = AM[p1 + lane];
-        sv = AS[p1 + lane];
+      } else {
+        if (lane < nrows1) {
+          m = ld_handoff(FM + p1 + lane);
+          sv = ld_handoff(FS + p1 + lane);
+        }
+        if (spin < 0 || __any(m != m || sv != sv)) return;
       }
+      have = true;
       S.nm[lane] = lane < nrows1 ? m : NEG;
       S.ns[lane] = lane < nrows1 ? sv : 0.0;
+    };
+    if (wv == 0) {
+      sigma = readlane_d(M, 0) + log(readlane_d(Sm, 0));
+      double W = lane < nrows ? Sm * exp(M - sigma - E) : 0.0;
+      // column r of dg holds A(q, r) at row q = lane (0 unless r < q); NaN
+      // and overflow fail the vote too
+      const bool in = rec_subst(dg, nrows, a.big, W);
+      S.wl[lane] = W;
+      if (lane == 0) S.fast = in ? 1 : 0;
+      if (in) publish(sigma + E + log(W));
+    } else {
+      next_acc(false);
+      rec_copy_wait();
     }
     __syncthreads();
+    const bool fast = S.fast != 0;
+    RecRaw xl;  // block b+1's rows on this block
+    if (fast) {
+      next_acc(true);
+    } else {
+      double c[16];
+      rec_conv16<FWD>(a, p0 + lane, p0 + 16 * wv, lane - 16 * wv, lane < nrows, xd, c);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) dg[(16 * wv + j) * RB + lane] = c[j];
+      rec_load16<FWD>(a, p1 + lane, p0 + 16 * wv, xl);
+      __syncthreads();
+      double sig = lane < nrows ? M : NEG;
+      if (wv == 0) {
+        rec_shift(dg, nrows, sig);
+        S.sg[lane] = lane < nrows ? sig : NEG;
+      }
+      __syncthreads();
+      const double sq = S.sg[lane];
+#pragma unroll 1
+      for (int r = 16 * wv; r < 16 * wv + 16; r += 4) {  // rolled: see lse16
+        double e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = dg[(r + i) * RB + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = exp_if(e[i] > NEG, e[i] + S.sg[r + i] - sq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dg[(r + i) * RB + lane] = e[i];
+      }
+      __syncthreads();
+      if (wv == 0) {
+        double W = 0.0;
+        if (lane < nrows && M > NEG && M > sig - 745.0) W = Sm * exp(M - sig);
+        rec_subst(dg, nrows, HUGE_VAL, W);
+        publish(sig + log(W));
+      } else {
+        next_acc(true);
+      }
+      __syncthreads();
+    }
     if (!more) break;
-    {
+    if (fast) {
       double acc = 0.0;
 #pragma unroll
-      for (int k = 0; k < LPW; ++k) acc = fma(lar[k], S.wl[wv + 4 * k], acc);
+      for (int k = 0; k < LPW; ++k) acc = fma(S.la[(wv + 4 * k) * RB + lane], S.wl[wv + 4 * k], acc);
       S.tacc[wv][lane] = acc;
-    }
+    } else {
+      // block b folded into row q' = lane from its values (block b is full)
+      double c[16], t[16], m16, s16;
+      rec_conv16<FWD>(a, p1 + lane, p0 + 16 * wv, 16, lane < nrows1, xl, c);
 #pragma unroll
-    for (int k = 0; k < DPT; ++k) {
-      const int w = tid + 256 * k;
-      S.dg[cur ^ 1][w] = dgr[k];
+      for (int j = 0; j < 16; ++j) t[j] = c[j] > NEG ? c[j] + S.lv[16 * wv + j] : NEG;
+      lse16(t, dg + 16 * wv * RB + lane, m16, s16);
+      S.tacc[wv][lane] = m16;
+      S.sacc[wv][lane] = s16;
     }
     // SOLO: block b+1's accumulators over blocks 0 .. b-1, folded here
     double Mf = NEG, Sf = 0.0;
-    if (SOLO && b + 1 >= 2) rec_fold_rows<FWD, false>(a, dir, b + 1, S.pm, S.ps, Mf, Sf);
+    if (SOLO && b + 1 >= 2) rec_fold_rows<FWD, false>(a, dir, b + 1, S.pm, S.ps, dg, Mf, Sf);
+    rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
     __syncthreads();
     if (wv == 0) {
       double Mn, Sn;
@@ -856,24 +996,28 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
         Mn = S.nm[lane];
         Sn = S.ns[lane];
       }
-      const double Y = (S.tacc[0][lane] + S.tacc[1][lane]) + (S.tacc[2][lane] + S.tacc[3][lane]);
-      if (lane < nrows1) {
-        if (fast && Y <= a.big) {
-          if (Y > 0.0) lse_pair(Mn, Sn, sigma + Dl + En + log(Y), 1.0);
-        } else {
-          // block b folded into row q' from its values (block b is full)
-          const int p = p1 + lane;
+      if (fast) {
+        const double Y = (S.tacc[0][lane] + S.tacc[1][lane]) + (S.tacc[2][lane] + S.tacc[3][lane]);
+        const bool out = lane < nrows1 && !(Y <= a.big);
+        if (lane < nrows1 && !out && Y > 0.0) lse_pair(Mn, Sn, sigma + Dl + En + log(Y), 1.0);
+        if (__any(out)) {  // whole wave: the loads below use every lane
           double m = NEG, s = 0.0;
+#pragma unroll 1
           for (int r0 = 0; r0 < RB; r0 += 16) {
             double c[16], t[16], m16, s16;
-            rec_coef_col16<FWD>(a, p, p0 + r0, true, c);
+            rec_coef_col16<FWD>(a, p1 + lane, p0 + r0, out, c);
 #pragma unroll
             for (int j = 0; j < 16; ++j) t[j] = c[j] > NEG ? c[j] + S.lv[r0 + j] : NEG;
-            lse16(t, m16, s16);
+            lse16(t, dg + lane, m16, s16);
             lse_pair(m, s, m16, s16);
           }
-          lse_pair(Mn, Sn, m, s);
+          if (out) lse_pair(Mn, Sn, m, s);
         }
+      } else if (lane < nrows1) {
+        double m = NEG, s = 0.0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) lse_pair(m, s, S.tacc[w][lane], S.sacc[w][lane]);
+        lse_pair(Mn, Sn, m, s);
       }
       M = Mn;
       Sm = Sn;
@@ -895,9 +1039,9 @@ __global__ __launch_bounds__(256) void k_rec_persist(RecArgs a, int dir0) {
       rec_solver<false>(a, 1, S);
   } else {
     if (dir == 0)
-      rec_updater<true>(a, 0, role + 1, S.pm, S.ps);
+      rec_updater<true>(a, 0, role + 1, S);
     else
-      rec_updater<false>(a, 1, role + 1, S.pm, S.ps);
+      rec_updater<false>(a, 1, role + 1, S);
   }
 }
 
@@ -1522,7 +1666,7 @@ constexpr size_t NA_ET = 0;
 constexpr size_t NA_LNN = NA_ET + (size_t)NA_NMAX * (NA_NMAX + 1) / 2;
 constexpr size_t NA_LF = NA_LNN + (NA_NMAX + 1);
 constexpr size_t NA_RB = NA_LF + (NA_NMAX + 1);
-constexpr size_t NA_REC = NA_RB + (NA_NMAX + 1);
+constexpr size_t NA_REC = (NA_RB + (NA_NMAX + 1) + 1) / 2 * 2;  // the coefficient tiles are 16-byte aligned
 constexpr size_t NA_SYNC = NA_REC + 10 * (size_t)(NA_NMAX + 1) + 2 * (size_t)NA_NBLK * (2 * RSQ + RB + 1);
 constexpr int NA_NSYNC = 4 * NA_NBLK + 2;  // flags of N_max, error word, injected-timeout count (unused here)
 constexpr size_t NA_DOUBLES = NA_SYNC + (NA_NSYNC + 1) / 2;
