@@ -1331,60 +1331,138 @@ __global__ __launch_bounds__(256) void k_box_virial(const double *__restrict__ X
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// Sign-tracked forward recursion at |xi'| (md_pimd_x.c:4675-4701): one
-// workgroup, one n at a time (a per-sample estimator, not per step).
-// One workgroup per xi' of a grid: out[b] = sign * exp(-beta V'(N) + beta V_B(N)).
-__global__ __launch_bounds__(256) void k_vi_sign(RecArgs a, const double *__restrict__ vi2s,
-                                                 double *__restrict__ outs) {
+// Sign-tracked forward recursion at xi' (md_pimd_x.c:4675-4701), one workgroup
+// per xi' of a grid: with c'(n, m) = (n-m-1) ln|xi'| - beta E_n^(n-m) - ln n
+// and s = sign(xi'), Z(n) = sum_{m<n} s^(n-m-1) exp(c'(n, m)) Z(m) is solved
+// as (sign, L' = ln |Z|) in blocks of 64 rows:
+//   columns of earlier blocks: a wave takes four rows, lanes the columns, in
+//     chunks of 64 from the nearest backwards; a chunk without a term within
+//     LSE_SKIP of the row's largest so far costs six instructions a row and
+//     no exponential (cycles end near their last particle, so that is most of
+//     them), the others rescale the row's sum to their maximum;
+//   the block itself: shifts sigma_q >= L'(q) by the (max,+) scan, signed
+//     scaled coefficients a(q, r) = +-exp(c' + sigma_r - sigma_q) on all waves,
+//     and the substitution W_q += a(q, r) W_r, L'(q) = sigma_q + ln |W_q|.
+// The instruction issue of the one compute unit per xi' (its 16 waves share
+// four SIMDs) and the serial scan and substitution (3.3 us per block) bound
+// it: 16 values at N=1024 3065 -> 202 us, at N=150 336 -> 31 us, against one
+// row at a time with two tree reductions each.
+constexpr int SIGN_NMAX = 4094;
+constexpr int SIGN_WG = 1024;
+
+__global__ __launch_bounds__(SIGN_WG) void k_vi_sign(RecArgs a, const double *__restrict__ vi2s,
+                                                     double *__restrict__ outs) {
+  __shared__ double Lp[SIGN_NMAX + 2], tile[RSQ], rM[RB], rS[RB], sg[RB];
+  __shared__ signed char sgn[SIGN_NMAX + 2];
   const double vi2 = vi2s[blockIdx.x];
-  double *out = outs + blockIdx.x;
-  __shared__ double red[256];
-  extern __shared__ double lds[];
-  const int N = a.N;
-  double *V2 = lds, *sg = lds + N + 1;
-  const double av = fabs(vi2), sv = vi2 < 0 ? -1.0 : 1.0;
-  const double lv = av > 0 ? log(av) : 0.0;
-  if (threadIdx.x == 0) {
-    V2[0] = 0;
-    sg[0] = 1;
+  const int N = a.N, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool neg = vi2 < 0.0, x0 = vi2 == 0.0;
+  const double lv = x0 ? 0.0 : log(fabs(vi2));
+  if (tid == 0) {
+    Lp[0] = 0.0;
+    sgn[0] = 1;
   }
   __syncthreads();
-  for (int n = 1; n <= N; ++n) {
-    double mn = 1e10;
-    if (vi2 == 0.0) {
-      mn = a.beta * (a.ENk[tri_row(n)] + V2[n - 1]);
-    } else {
-      for (int k = 1 + threadIdx.x; k <= n; k += 256) mn = fmin(mn, -(k - 1) * lv + a.beta * (a.ENk[tri_row(n) + k - 1] + V2[n - k]));
-      red[threadIdx.x] = mn;
-      __syncthreads();
-      for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + w]);
-        __syncthreads();
+  for (int p0 = 1; p0 <= N; p0 += RB) {
+    const int nrows = min(RB, N - p0 + 1);
+    // c'(p0 + q, p0 + r) at tile[r][q], r < q
+    {
+      double E[RSQ / SIGN_WG];
+      const double lnq = a.lnn[min(p0 + lane, N)];
+#pragma unroll
+      for (int i = 0; i < RSQ / SIGN_WG; ++i) {  // r = wv + 16 i, q = lane
+        const int r = wv + 16 * i, pc = min(p0 + r, N - 1);
+        E[i] = a.ET[col_off(pc, N) + max(min(p0 + lane, N) - pc - 1, 0)];
       }
-      mn = red[0];
-      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < RSQ / SIGN_WG; ++i) {
+        const int r = wv + 16 * i, k = lane - r;
+        const bool ok = k >= 1 && lane < nrows && !(x0 && k != 1);
+        tile[r * RB + lane] = ok ? (k - 1) * lv - a.beta * E[i] - lnq : NEG;
+      }
     }
-    double s = 0;
-    for (int k = 1 + threadIdx.x; k <= n; k += 256) {
-      if (vi2 == 0.0 && k != 1) continue;
-      double sk = ((k - 1) % 2 == 1) ? sv : 1.0;
-      double arg = (vi2 == 0.0 ? 0.0 : (k - 1) * lv) - a.beta * (a.ENk[tri_row(n) + k - 1] + V2[n - k]) + mn;
-      s += sg[n - k] * sk * exp(arg);
+    // columns m < p0 of rows n_i = p0 + wv + 16 i: exponents less ln n_i
+    constexpr int NR = RB / (SIGN_WG / 64);
+    double M[NR], S[NR], En[NR];
+    const double *row[NR];
+    auto load = [&](int i, int m) { return row[i][-min(max(m, 0), p0 - 1)]; };
+    int m = p0 - 64 + lane;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int n = min(p0 + wv + 16 * i, N);
+      row[i] = a.ENk + tri_row(n) + n - 1;  // E_n^(n-m) at row[-m]
+      En[i] = load(i, m);
+      M[i] = NEG;
+      S[i] = 0.0;
     }
-    red[threadIdx.x] = s;
+    for (int m0 = p0 - 64; m0 > -64; m0 -= 64, m -= 64) {
+      double E[NR];
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        E[i] = En[i];
+        En[i] = load(i, m - 64);
+      }
+      const int k = p0 + wv - m;
+      const bool on = m >= 0;
+      const double base = on ? fma((double)(k - 1), lv, Lp[m]) : NEG;
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        double t = fma(-a.beta, E[i], base + (16 * i) * lv);
+        if (x0 && k + 16 * i != 1) t = NEG;
+        if (!__any(t > M[i] - LSE_SKIP)) continue;
+        const double mx = wave_max_dpp(t);
+        if (mx > M[i]) {
+          if (M[i] > NEG) S[i] *= exp(M[i] - mx);
+          M[i] = mx;
+        }
+        const bool in = on && t > M[i] - LSE_SKIP;
+        const double e = exp_if(in, t - M[i]);
+        S[i] += (neg && ((k - 1) & 1)) != (in && sgn[m] < 0) ? -e : e;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if (M[i] > 0.5 * NEG) M[i] -= a.lnn[min(p0 + wv + 16 * i, N)];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      S[i] = wave_sum_dpp(S[i]);
+      if (lane == 0) {
+        rM[wv + 16 * i] = M[i];
+        rS[wv + 16 * i] = S[i];
+      }
+    }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
+    double sig = NEG;
+    if (wv == 0) {
+      sig = lane < nrows ? rM[lane] : NEG;
+      rec_shift(tile, nrows, sig);
+      sg[lane] = sig;
     }
-    if (threadIdx.x == 0) {
-      double t = red[0];
-      sg[n] = t >= 0 ? 1 : -1;
-      V2[n] = (mn - log(fabs(t)) + log((double)n)) / a.beta;
+    __syncthreads();
+    // columns j and 63 - j share a wave's lanes: rows q > j of the one, rows
+    // q > 63 - j of the other; the upper triangle becomes 0
+    for (int j = wv; j < RB / 2; j += SIGN_WG / 64) {
+      const int r = lane > j ? j : RB - 1 - j, q = lane > j ? lane : RB - 1 - lane;
+      const bool below = q > r;
+      const double c = below ? tile[r * RB + q] : NEG;
+      const double e = exp_if(c > NEG, c + sg[r] - sg[q]);
+      if (below) tile[r * RB + q] = neg && ((q - r - 1) & 1) ? -e : e;
+      if (lane <= j) tile[j * RB + lane] = 0.0;
+      if (lane <= RB - 1 - j) tile[(RB - 1 - j) * RB + lane] = 0.0;
+    }
+    __syncthreads();
+    if (wv == 0) {
+      double W = 0.0;
+      if (lane < nrows && rM[lane] > NEG) W = rS[lane] * exp(rM[lane] - sig);
+      rec_subst(tile, nrows, HUGE_VAL, W);
+      if (lane < nrows) {
+        Lp[p0 + lane] = sig + log(fabs(W));
+        sgn[p0 + lane] = W >= 0.0 ? 1 : -1;
+      }
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = sg[N] * exp(-a.beta * V2[N] - a.Lf[N]);
+  if (tid == 0) outs[blockIdx.x] = sgn[N] * exp(Lp[N] - a.Lf[N]);
 }
 
 // ------------------------------------------------- batched replicas
@@ -2250,8 +2328,8 @@ int md_pimd_calc_vi_virial_pressure_x(md_pimd_t_x *pimd, md_stats_t_x *stats, in
 // each): out[i] = sign_{xi'_i}(N) exp(-beta V_{|xi'_i|}(N) + beta V_B(N)).
 static int vi_sign_grid(DevPimd *p, int n, const double *vi2, double *out) {
   if (n <= 0) return 0;
-  if (2 * (p->N + 1) * sizeof(double) > 65536) {
-    fprintf(stderr, "xmd: sign reweighting supports N <= 4094\n");
+  if (p->N > SIGN_NMAX) {
+    fprintf(stderr, "xmd: sign reweighting supports N <= %d\n", SIGN_NMAX);
     return -1;
   }
   if (n > 512) {
@@ -2262,7 +2340,7 @@ static int vi_sign_grid(DevPimd *p, int n, const double *vi2, double *out) {
   double *d_vi = p->work + 4 * (p->N + 1) + 8, *d_out = d_vi + 512;
   hipStream_t st = rt().s0;
   XMD_CHECK(hipMemcpyAsync(d_vi, vi2, n * sizeof(double), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_vi_sign, dim3(n), dim3(256), 2 * (p->N + 1) * sizeof(double), st, a, d_vi, d_out);
+  hipLaunchKernelGGL(k_vi_sign, dim3(n), dim3(SIGN_WG), 0, st, a, d_vi, d_out);
   XMD_CHECK(hipGetLastError());
   XMD_CHECK(hipMemcpyAsync(out, d_out, n * sizeof(double), hipMemcpyDeviceToHost, st));
   XMD_CHECK(hipStreamSynchronize(st));

@@ -52,6 +52,35 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Whole-wave reductions through DPP moves (row shifts, then row broadcasts),
+// every lane active: the result in every lane, lanes combined in ascending
+// order.  About 20 cycles a step against 80-120 for a shuffle through LDS.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or(double v, double other) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(other), __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(other), __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+template <class Op>
+__device__ __forceinline__ double wave_reduce_dpp(double v, double neutral, Op op) {
+  v = op(dpp_or<0x111, 0xf>(v, neutral), v);  // row_shr 1, 2, 4, 8: lane 15 of each row holds the row
+  v = op(dpp_or<0x112, 0xf>(v, neutral), v);
+  v = op(dpp_or<0x114, 0xf>(v, neutral), v);
+  v = op(dpp_or<0x118, 0xf>(v, neutral), v);
+  v = op(dpp_or<0x142, 0xa>(v, neutral), v);  // row_bcast 15 into rows 1 and 3
+  v = op(dpp_or<0x143, 0xc>(v, neutral), v);  // row_bcast 31 into rows 2 and 3
+  return readlane_d(v, 63);
+}
+
+__device__ __forceinline__ double wave_max_dpp(double v) {
+  return wave_reduce_dpp(v, -__builtin_inf(), [](double a, double b) { return fmax(a, b); });
+}
+
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  return wave_reduce_dpp(v, 0.0, [](double a, double b) { return a + b; });
+}
+
 // Double-double arithmetic (Knuth TwoSum / Dekker) for prefix sums whose
 // differences must keep full double precision.
 struct dd {
