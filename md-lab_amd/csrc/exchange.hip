@@ -1218,69 +1218,113 @@ __global__ __launch_bounds__(256) void k_enk2_fill(const double *__restrict__ X,
 
 // res(n) = sum_{m<n} w(n,m) (res(m) - B(n,m)) / sum_{m<n} w(n,m) with
 // w(n,m) = exp(c(n,m) + L(m) - L(n)), B = ENk or ENk2
-// (md_pimd_x.c:1273-1288, 4294-4319).  Linear recursion: blocked like the
-// forward pass, the diagonal is a 64-step forward substitution.
-__global__ __launch_bounds__(RT) void k_estimator(RecArgs a, const double *__restrict__ Bm, double *__restrict__ out) {
-  extern __shared__ double lds[];
-  const int N = a.N;
-  double *wd = lds;                       // RB*(RB-1)/2 weights
-  double *bd = wd + RB * (RB - 1) / 2;    // RB*(RB-1)/2 matrix values
-  double *ao = bd + RB * (RB - 1) / 2;    // RB
-  double *wo = ao + RB;                   // RB
-  double *res = wo + RB;                  // N+1
-  double *Ls = res + N + 1;               // N+1
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int p = tid; p <= N; p += RT) Ls[p] = a.Lf[p];
-  if (tid == 0) res[0] = 0.0;
+// (md_pimd_x.c:1273-1288, 4294-4319), in two kernels: the row-normalised
+// weights P(n,m) and the rows' sums of P B, which do not depend on res (every
+// row its own workgroup: all of the exponentials), then the linear
+// recursion res(n) = sum_m P(n,m) res(m) - bn(n) on one workgroup, blocked
+// like the forward pass.  Normalising each row keeps the rounding of its
+// exponents (differences of numbers of size beta V_B) out of the total; the
+// unnormalised sum over cycle probabilities exp(c + L(m) + R(n) - L(N)) would
+// be one parallel pass, but is 20 times less accurate.  Weights below e^-80
+// of their row are 0 and 64-column chunks without any other are skipped (a
+// bit mask per row).  What bounds it is the serial substitution (1.7 us per
+// block): N=1024 507 -> 66 us, N=150 41 -> 17 us, against one workgroup doing
+// both.
+constexpr int EST_NMAX = 2015;                       // rows of a workgroup's chunk mask and LDS
+constexpr int EST_PER = (EST_NMAX + 255) / 256;      // weights per thread
+
+struct EstArgs {
+  double *P;       // [tri_row(n) + m], columns before row n's block only
+  double *dg;      // [nblk][RB][RB] in-block weights [r][q] (0 unless r < q)
+  double *bn;      // [N]
+  unsigned *mask;  // [N] chunks of 64 columns with a weight
+};
+
+__global__ __launch_bounds__(256) void k_est_weights(RecArgs a, const double *__restrict__ Bm, EstArgs o) {
+  __shared__ double red[2][4], dgr[RB];
+  __shared__ unsigned mask;
+  const int N = a.N, n = blockIdx.x + 1, tid = threadIdx.x;
+  const int blk = (n - 1) / RB, q = (n - 1) % RB, p0 = 1 + blk * RB;
+  if (tid < RB) dgr[tid] = 0.0;
+  if (tid == 0) mask = 0;
   __syncthreads();
-  for (int p0 = 1; p0 <= N; p0 += RB) {
-    const int nrows = min(RB, N - p0 + 1);
-    for (int r = wv; r < nrows; r += RT / 64) {
-      const int n = p0 + r;
-      double acc = 0, sw = 0;
-      for (int m = lane; m < p0; m += 64) {
-        double c = rec_coef<true>(a, n, m);
-        if (c > NEG) {
-          double w = exp(c + Ls[m] - Ls[n]);
-          acc += w * (res[m] - Bm[tri_row(n) + (n - m) - 1]);
-          sw += w;
-        }
-      }
-      acc = wave_sum(acc);
-      sw = wave_sum(sw);
-      if (lane == 0) {
-        ao[r] = acc;
-        wo[r] = sw;
-      }
+  if (n <= N) {
+    const double *row = a.ENk + tri_row(n), *brow = Bm + tri_row(n);
+    const double ln = a.lnn[n], Ln = a.Lf[n];
+    double w[EST_PER], s0 = 0.0, s1 = 0.0;
+#pragma unroll
+    for (int i = 0; i < EST_PER; ++i) {
+      const int k = 1 + tid + 256 * i;
+      const bool ok = k <= n && !(a.xi0 && k != 1);
+      const double x = ok ? ((k - 1) * a.lnxi - a.beta * row[k - 1] - ln) + (a.Lf[n - k] - Ln) : NEG;
+      w[i] = 0.0;
+      if (__any(x > -80.0)) w[i] = exp_if(x > -80.0, x);
+      s0 += w[i];
+      if (w[i] != 0.0) s1 += w[i] * brow[k - 1];
     }
-    for (int w = tid; w < RB * (RB - 1) / 2; w += RT) {
-      int q = (int)((1.0 + sqrt(1.0 + 8.0 * w)) / 2.0);
-      while (q * (q - 1) / 2 > w) --q;
-      while ((q + 1) * q / 2 <= w) ++q;
-      int r = w - q * (q - 1) / 2;
-      double wt = 0, bv = 0;
-      if (q < nrows) {
-        const int n = p0 + q, m = p0 + r;
-        double c = rec_coef<true>(a, n, m);
-        if (c > NEG) wt = exp(c + Ls[m] - Ls[n]);
-        bv = Bm[tri_row(n) + (n - m) - 1];
-      }
-      wd[w] = wt;
-      bd[w] = bv;
+    s0 = wave_sum_dpp(s0);
+    s1 = wave_sum_dpp(s1);
+    if ((tid & 63) == 0) {
+      red[0][tid >> 6] = s0;
+      red[1][tid >> 6] = s1;
     }
     __syncthreads();
-    if (wv == 0) {
-      double acc = lane < nrows ? ao[lane] : 0.0;
-      double sw = lane < nrows ? wo[lane] : 0.0;
-      for (int r = 0; r < nrows; ++r) {
-        const double rr = readlane_d(acc, r) / readlane_d(sw, r);
-        if (lane > r && lane < nrows) {
-          const int w = lane * (lane - 1) / 2 + r;
-          acc += wd[w] * (rr - bd[w]);
-          sw += wd[w];
-        }
+    s0 = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    s1 = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    const double inv = 1.0 / s0;
+    unsigned bits = 0;
+#pragma unroll
+    for (int i = 0; i < EST_PER; ++i) {
+      const int m = n - 1 - tid - 256 * i;
+      if (m < 0) break;
+      const double p = w[i] * inv;
+      if (m >= p0) {
+        dgr[m - p0] = p;
+      } else {
+        o.P[tri_row(n) + m] = p;
+        if (p != 0.0) bits |= 1u << (m >> 6);
       }
-      if (lane < nrows) res[p0 + lane] = acc / sw;
+    }
+    if (bits) atomicOr(&mask, bits);
+    if (tid == 0) o.bn[n - 1] = s1 * inv;
+  }
+  __syncthreads();
+  if (tid < RB) o.dg[(size_t)blk * RSQ + tid * RB + q] = dgr[tid];
+  if (tid == 0 && n <= N) o.mask[n - 1] = mask;
+}
+
+__global__ __launch_bounds__(RT) void k_est_solve(int N, EstArgs o, double *__restrict__ out) {
+  __shared__ alignas(16) double tile[2][RSQ];
+  __shared__ double res[EST_NMAX + RB + 1], acc[RB];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int NR = RB / (RT / 64);  // rows per wave
+  const int nblk = (N + RB - 1) / RB;
+  if (tid == 0) res[0] = 0.0;
+  for (int w = tid; w < RSQ; w += RT) tile[0][w] = o.dg[w];
+  __syncthreads();
+  for (int b = 0; b < nblk; ++b) {
+    const int p0 = 1 + b * RB, nrows = min(RB, N - p0 + 1);
+    // the next block's tile, by three waves that do not substitute
+    if (b + 1 < nblk && wv >= 13) rec_copy_tile(o.dg + (size_t)(b + 1) * RSQ, tile[(b + 1) & 1], wv - 13);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int n = p0 + wv + 16 * i;
+      double s = 0.0;
+      if (n <= N) {
+        for (unsigned mk = o.mask[n - 1]; mk; mk &= mk - 1) {
+          const int m = 64 * (__ffs(mk) - 1) + lane;
+          if (m < p0) s = fma(o.P[tri_row(n) + m], res[m], s);
+        }
+        s = wave_sum_dpp(s) - o.bn[n - 1];
+      }
+      if (lane == 0) acc[wv + 16 * i] = s;
+    }
+    rec_copy_wait();
+    __syncthreads();
+    if (wv == 0) {
+      double W = acc[lane];
+      rec_subst(tile[b & 1], nrows, HUGE_VAL, W);
+      res[p0 + lane] = W;
     }
     __syncthreads();
   }
@@ -1970,16 +2014,23 @@ static int ensure_vbn(DevPimd *p) {
   return 0;
 }
 
-static size_t est_lds(int N) { return (size_t)(RB * (RB - 1) + 2 * RB + 2 * (N + 1)) * sizeof(double); }
-
 static int run_estimator(DevPimd *p, const double *Bm, double *out) {
-  if (est_lds(p->N) > 65536) {
-    fprintf(stderr, "xmd: estimator recursion supports N <= 2015\n");
+  const int N = p->N, nblk = (N + RB - 1) / RB;
+  if (N > EST_NMAX) {
+    fprintf(stderr, "xmd: estimator recursion supports N <= %d\n", EST_NMAX);
     return -1;
   }
+  const size_t tri = (size_t)N * (N + 1) / 2;
+  if (!p->est) XMD_CHECK(hipMalloc(&p->est, ((size_t)nblk * RSQ + tri + 2 * (size_t)N) * sizeof(double)));
   RecArgs a = rec_args(p);
-  double *d_out = p->work + 4 * (p->N + 1);
-  hipLaunchKernelGGL(k_estimator, dim3(1), dim3(RT), est_lds(p->N), rt().s0, a, Bm, d_out);
+  EstArgs o;
+  o.dg = p->est;
+  o.P = o.dg + (size_t)nblk * RSQ;
+  o.bn = o.P + tri;
+  o.mask = (unsigned *)(o.bn + N);
+  double *d_out = p->work + 4 * (N + 1);
+  hipLaunchKernelGGL(k_est_weights, dim3(nblk * RB), dim3(256), 0, rt().s0, a, Bm, o);
+  hipLaunchKernelGGL(k_est_solve, dim3(1), dim3(RT), 0, rt().s0, N, o, d_out);
   XMD_CHECK(hipGetLastError());
   XMD_CHECK(hipMemcpyAsync(out, d_out, sizeof(double), hipMemcpyDeviceToHost, rt().s0));
   XMD_CHECK(hipStreamSynchronize(rt().s0));

@@ -101,6 +101,7 @@ struct DevPimd {
   double *Rb = nullptr;     // backward R(m) = -beta Vt^(m),  N+1
   double *Gm = nullptr;     // optional connection matrix (debug/tests), N*N
   double *work = nullptr;   // estimator scratch
+  double *est = nullptr;    // estimator weights (exchange.hip EstArgs), made on first use
   double *Fx = nullptr;     // exchange forces of the end beads, [slice P-1, slice 0][dim][particle] (6N)
   double *rec = nullptr;    // recursion state: values, accumulators, block coefficients
   int *recsync = nullptr;   // recursion sync words: 4*nblk unused, error word, injected-timeout count
