@@ -175,15 +175,19 @@ void batch_table_free(BatchTable &t) {
   t = BatchTable();
 }
 
-int device_sum(const double *src, int n, double *out) {
+int device_sums(const double *const *src, const int *n, int count, double *out) {
   static double *d_out = nullptr;
-  if (!d_out) XMD_CHECK(hipMalloc(&d_out, sizeof(double)));
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, rt().s0, src, n, d_out);
+  if (count > 4) return -1;
+  if (!d_out) XMD_CHECK(hipMalloc(&d_out, 4 * sizeof(double)));
+  for (int k = 0; k < count; ++k)
+    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, rt().s0, src[k], n[k], d_out + k);
   XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipMemcpyAsync(out, d_out, sizeof(double), hipMemcpyDeviceToHost, rt().s0));
+  XMD_CHECK(hipMemcpyAsync(out, d_out, count * sizeof(double), hipMemcpyDeviceToHost, rt().s0));
   XMD_CHECK(hipStreamSynchronize(rt().s0));
   return 0;
 }
+
+int device_sum(const double *src, int n, double *out) { return device_sums(&src, &n, 1, out); }
 
 // -------------------------------------------------------- upload/download
 

@@ -1,5 +1,6 @@
 """Generates ewald_table.h: piecewise polynomials of the Ewald real-space
-force kernel h(x) = erfc(x) + 2x/sqrt(pi) exp(-x^2) on 0 <= x < 53/8.
+kernels on 0 <= x < 53/8, h(x) = erfc(x) + 2x/sqrt(pi) exp(-x^2) of the force
+and erfc(x) of the energy.
 
 Interval i covers [i/8, (i+1)/8); inside it h = sum_k c[i][k] y^k with
 y = 16 x - (2 i + 1) in [-1, 1].  The coefficients interpolate h at the 10
@@ -19,7 +20,7 @@ def h(x):
     return mp.erfc(x) + 2 * x / mp.sqrt(mp.pi) * mp.exp(-x * x)
 
 
-def main():
+def table(h):
     nodes = [mp.cos(mp.pi * (k + mp.mpf(1) / 2) / (DEG + 1)) for k in range(DEG + 1)]
     V = mp.matrix([[t ** j for j in range(DEG + 1)] for t in nodes])
     rows = []
@@ -36,17 +37,24 @@ def main():
                 acc = acc * t + cd[j]
             worst = max(worst, abs(acc - float(h(a + (mp.mpf(t) + 1) / (2 * INV_W)))))
         rows.append(cd)
+    return rows, worst
+
+
+def main():
+    force, ef = table(h)
+    energy, ee = table(mp.erfc)
     print("// Generated by gen_ewald_table.py -- do not edit.")
-    print(f"// h(x) = erfc(x) + 2x/sqrt(pi) exp(-x^2), {NINT} intervals of width 1/{INV_W}, degree {DEG};")
-    print(f"// max abs error of the FP64 Horner evaluation {worst:.2e}.")
+    print(f"// h(x) = erfc(x) + 2x/sqrt(pi) exp(-x^2) (kEwTab) and erfc(x) (kEwTabE), {NINT} intervals of width 1/{INV_W}, degree {DEG};")
+    print(f"// max abs errors of the FP64 Horner evaluation {ef:.2e} and {ee:.2e}.")
     print("#pragma once")
     print(f"constexpr int kEwTabIntervals = {NINT};")
     print(f"constexpr int kEwTabStride = {DEG + 1};")
     print(f"constexpr double kEwTabInvWidth = {INV_W}.0;")
-    print(f"__device__ __constant__ double kEwTab[{NINT * (DEG + 1)}] = {{")
-    for cd in rows:
-        print("    " + ", ".join(repr(v) for v in cd) + ",")
-    print("};")
+    for name, rows in (("kEwTab", force), ("kEwTabE", energy)):
+        print(f"__device__ __constant__ double {name}[{NINT * (DEG + 1)}] = {{")
+        for cd in rows:
+            print("    " + ", ".join(repr(v) for v in cd) + ",")
+        print("};")
 
 
 if __name__ == "__main__":

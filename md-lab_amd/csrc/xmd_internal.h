@@ -127,6 +127,8 @@ int download_pimd(DevPimd *p);
 
 // reductions: sum of n doubles on device into *out (host), deterministic
 int device_sum(const double *src, int n, double *out);
+// up to four such sums with one wait for the results
+int device_sums(const double *const *src, const int *n, int count, double *out);
 
 inline double box_L(const md_simulation_t_x *sim, int d) {
   if (sim->box && sim->box->type == MD_ND_RECT_BOX_X && sim->box->box)
