@@ -175,6 +175,20 @@ void batch_table_free(BatchTable &t) {
   t = BatchTable();
 }
 
+double *host_scratch(size_t n) {
+  static double *buf = nullptr;
+  static size_t cap = 0;
+  if (n > cap) {
+    if (buf) (void)hipHostFree(buf);
+    buf = nullptr;
+    cap = 0;
+    n = n < 1024 ? 1024 : n;
+    if (hipHostMalloc((void **)&buf, n * sizeof(double), hipHostMallocDefault) != hipSuccess) return nullptr;
+    cap = n;
+  }
+  return buf;
+}
+
 int device_sums(const double *const *src, const int *n, int count, double *out) {
   static double *d_out = nullptr;
   if (count > 4) return -1;

@@ -6,13 +6,16 @@
 // (md_pimd_x.c:4958-5450, md_statistics_x.c:104-161).
 //
 // Histograms: the kernels count samples per bin with integer atomics (exact,
-// order independent); the host then adds the reference's increment (1/P or
-// 1/norm) once per count into stats->fxs[stats->N-1][bin].  Every bin only
-// ever receives that one increment value, so the result equals the
-// reference's sequential accumulation bit for bit.
+// order independent), each workgroup in LDS first (kLdsBins bins; 490,000
+// pairs into 200 bins took 148 us as global atomics, whose bins are shared by
+// all, 12 us this way), and k_hist_add adds the reference's increment (1/P or
+// 1/norm) once per count to stats->fxs[stats->N-1][bin], which it reads and
+// writes in pinned host memory.  Every bin only ever receives that one
+// increment value, so the result equals the reference's sequential
+// accumulation bit for bit.
 #include <algorithm>
 #include <cmath>
-#include <vector>
+#include <cstring>
 
 #include "xmd_device.h"
 #include "xmd_internal.h"
@@ -35,13 +38,69 @@ struct ObsGeo {
   int points, image;
 };
 
+// A workgroup's counts: in LDS (LDS true; points <= kLdsBins, dynamic shared
+// memory of that many words), added to the global counts at the end, or
+// straight into the global counts.
+constexpr int kLdsBins = 12288;
+constexpr int kHistWork = 4096;  // samples per workgroup of the pair histograms, about 20 per bin at 200 bins
+
+template <bool LDS>
+struct Hist {
+  unsigned *lds;
+  unsigned long long *cnt;
+  int points;
+  __device__ Hist(unsigned *l, unsigned long long *c, int n) : lds(l), cnt(c), points(n) {
+    if (!LDS) return;
+    for (int b = threadIdx.x; b < points; b += blockDim.x) lds[b] = 0;
+    __syncthreads();
+  }
+  // bins below 0 or beyond the last are dropped
+  __device__ void add(int b) {
+    if ((unsigned)b >= (unsigned)points) return;
+    if (LDS)
+      atomicAdd(&lds[b], 1u);
+    else
+      atomicAdd(&cnt[b], 1ull);
+  }
+  __device__ void flush() {
+    if (!LDS) return;
+    __syncthreads();
+    for (int b = threadIdx.x; b < points; b += blockDim.x)
+      if (lds[b]) atomicAdd(&cnt[b], (unsigned long long)lds[b]);
+  }
+};
+
+// Row and column of this workgroup's samples of a row-major (.. x n) matrix,
+// thread tid taking samples tid, tid + 256, ... of [begin, begin + kHistWork).
+struct RowCol {
+  long row;
+  int col, n, dr, dc;
+  __device__ RowCol(long t, int n_) : row(t / n_), n(n_) {
+    col = (int)(t - row * n);
+    dr = 256 / n;
+    dc = 256 - dr * n;
+  }
+  __device__ void next() {
+    row += dr;
+    col += dc;
+    if (col >= n) {
+      col -= n;
+      ++row;
+    }
+  }
+};
+
 // md_pimd_x.c:1947-1962: every bead's distance to the center.
-__global__ void k_density_hist(const double *__restrict__ X, int nb, ObsGeo g, unsigned long long *__restrict__ cnt) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nb) return;
-  const double r = obs_dist(X[s] - g.c[0], X[nb + s] - g.c[1], X[2 * nb + s] - g.c[2], g.L, g.image);
-  const int b = (int)(r / g.incre);
-  if (b < g.points) atomicAdd(&cnt[b], 1ull);
+template <bool LDS>
+__global__ __launch_bounds__(256) void k_density_hist(const double *__restrict__ X, int nb, ObsGeo g,
+                                                      unsigned long long *__restrict__ cnt) {
+  extern __shared__ unsigned bins[];
+  Hist<LDS> h(bins, cnt, g.points);
+  for (int s = blockIdx.x * 256 + threadIdx.x; s < nb; s += gridDim.x * 256) {
+    const double r = obs_dist(X[s] - g.c[0], X[nb + s] - g.c[1], X[2 * nb + s] - g.c[2], g.L, g.image);
+    h.add((int)(r / g.incre));
+  }
+  h.flush();
 }
 
 // Bead sets of a pair histogram: bead slots slot0 + l (l < N) of one
@@ -75,53 +134,101 @@ __device__ __forceinline__ int clamp_bin(int i1, int i2, int n, int points) {
 //  HM_RADIAL (md_pimd_x.c:3019-3036, 3125-3136): bin (int)(r / incre), dropped beyond the last bin;
 //  HM_AXES2D (md_pimd_x.c:4889-4909): bins (int)(|dx| / incre), (int)(|dy| / incre), clamped;
 //  HM_ITCF   (md_pimd_x.c:2731-2746, 2851-2870): bins of (x - rmin) / incre along dimension 0, clamped.
+template <bool LDS>
 __global__ __launch_bounds__(256) void k_pair_hist(PairHist h, unsigned long long *__restrict__ cnt) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)h.a.N * h.b.N) return;
-  const int l = (int)(t / h.b.N), j = (int)(t - (long)l * h.b.N);
-  if (h.same && l == j) return;
-  const int sa = h.a.slot0 + l, sb = h.b.slot0 + j;
+  extern __shared__ unsigned bins[];
+  Hist<LDS> H(bins, cnt, h.points);
+  const long begin = (long)blockIdx.x * kHistWork, end = min(begin + kHistWork, (long)h.a.N * h.b.N);
   const double *XA = h.a.X, *XB = h.b.X;
   const int na = h.a.nb, nb = h.b.nb;
-  if (h.mode == HM_RADIAL) {
-    const double r =
-        obs_dist(XA[sa] - XB[sb], XA[na + sa] - XB[nb + sb], XA[2 * na + sa] - XB[2 * nb + sb], h.L, h.image);
-    const int bin = (int)(r / h.incre);
-    if (bin < h.points) atomicAdd(&cnt[bin], 1ull);
-  } else if (h.mode == HM_AXES2D) {
-    double dx = XA[sa] - XB[sb], dy = XA[na + sa] - XB[nb + sb];
-    if (h.image) {
-      dx = dv_min_image(dx, h.L[0]);
-      dy = dv_min_image(dy, h.L[1]);
+  RowCol at(begin + threadIdx.x, h.b.N);
+  for (long t = begin + threadIdx.x; t < end; t += 256, at.next()) {
+    const int l = (int)at.row, j = at.col;
+    if (h.same && l == j) continue;
+    const int sa = h.a.slot0 + l, sb = h.b.slot0 + j;
+    if (h.mode == HM_RADIAL) {
+      const double r =
+          obs_dist(XA[sa] - XB[sb], XA[na + sa] - XB[nb + sb], XA[2 * na + sa] - XB[2 * nb + sb], h.L, h.image);
+      H.add((int)(r / h.incre));
+    } else if (h.mode == HM_AXES2D) {
+      double dx = XA[sa] - XB[sb], dy = XA[na + sa] - XB[nb + sb];
+      if (h.image) {
+        dx = dv_min_image(dx, h.L[0]);
+        dy = dv_min_image(dy, h.L[1]);
+      }
+      const int i1 = (int)(fabs(dx) / h.incre), i2 = (int)(fabs(dy) / h.incre);
+      H.add(clamp_bin(i1, i2, h.n, h.points));
+    } else {
+      const int i1 = (int)((XA[sa] - h.rmin) / h.incre), i2 = (int)((XB[sb] - h.rmin) / h.incre);
+      H.add(clamp_bin(i1, i2, h.n, h.points));
+      if (h.two) H.add(clamp_bin(i2, i1, h.n, h.points));
     }
-    const int i1 = (int)(fabs(dx) / h.incre), i2 = (int)(fabs(dy) / h.incre);
-    atomicAdd(&cnt[clamp_bin(i1, i2, h.n, h.points)], 1ull);
-  } else {
-    const int i1 = (int)((XA[sa] - h.rmin) / h.incre), i2 = (int)((XB[sb] - h.rmin) / h.incre);
-    atomicAdd(&cnt[clamp_bin(i1, i2, h.n, h.points)], 1ull);
-    if (h.two) atomicAdd(&cnt[clamp_bin(i2, i1, h.n, h.points)], 1ull);
   }
+  H.flush();
 }
 
 // md_pimd_x.c:3248-3278: in-plane distance of beads l != j of one slice,
 // both inside the window box = {x0, x1, y0, y1}.
+template <bool LDS>
 __global__ __launch_bounds__(256) void k_paircorr_box2d(const double *__restrict__ X, int N, int nb, int P, double x0,
                                                         double x1, double y0, double y1, double incre, int points,
                                                         unsigned long long *__restrict__ cnt) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)P * N * N) return;
-  const int slice = (int)(t / ((long)N * N));
-  const int rem = (int)(t - (long)slice * N * N);
-  const int l = rem / N, j = rem - l * N;
-  if (l == j) return;
-  const int sa = slice * N + l, sb = slice * N + j;
-  const double ax = X[sa], ay = X[nb + sa], bx = X[sb], by = X[nb + sb];
-  if (ax < x0 || ax > x1 || ay < y0 || ay > y1) return;
-  if (bx < x0 || bx > x1 || by < y0 || by > y1) return;
-  const double dx = ax - bx, dy = ay - by;
-  const double r = sqrt(dx * dx + dy * dy);
-  const int bin = (int)(r / incre);
-  if (bin < points) atomicAdd(&cnt[bin], 1ull);
+  extern __shared__ unsigned bins[];
+  Hist<LDS> H(bins, cnt, points);
+  const long begin = (long)blockIdx.x * kHistWork, end = min(begin + kHistWork, (long)P * N * N);
+  RowCol at(begin + threadIdx.x, N);
+  for (long t = begin + threadIdx.x; t < end; t += 256, at.next()) {
+    const int sa = (int)at.row, slice = sa / N, sb = slice * N + at.col;  // row: bead slot slice * N + l
+    if (sa == sb) continue;
+    const double ax = X[sa], ay = X[nb + sa], bx = X[sb], by = X[nb + sb];
+    if (ax < x0 || ax > x1 || ay < y0 || ay > y1) continue;
+    if (bx < x0 || bx > x1 || by < y0 || by > y1) continue;
+    const double dx = ax - bx, dy = ay - by;
+    const double r = sqrt(dx * dx + dy * dy);
+    H.add((int)(r / incre));
+  }
+  H.flush();
+}
+
+// x + c, n times, each sum rounded (n repeated additions, bit for bit).
+// While x stays in one binade every addition moves it by the same multiple of
+// its last place (unless c lies midway between two, which rounds by parity),
+// so all additions up to the binade's end are one product.
+__host__ __device__ inline double add_repeated(double x, double c, unsigned long long n) {
+  while (n) {
+    const double y = x + c;
+    if (!(c > 0.0) || !(x >= c) || !(y < 1e300) || n < 4) {  // the general case: one at a time
+      if (y == x || y != y) return y;
+      x = y;
+      --n;
+      continue;
+    }
+    const double d = y - x;  // exact, x <= y <= 2x
+    if (d == 0.0) return x;
+    int e;
+    (void)frexp(x, &e);                                       // x in [2^(e-1), 2^e)
+    const double top = ldexp(1.0, e), half = ldexp(1.0, e - 54);  // half of x's last place
+    double k = floor((top - x) / d);
+    if (k * d > top - x) k -= 1.0;
+    if (k < 1.0 || fabs(c - d) == half) {
+      x = y;
+      --n;
+      continue;
+    }
+    if (k > (double)n) k = (double)n;
+    x += k * d;
+    n -= (unsigned long long)k;
+  }
+  return x;
+}
+
+// fx[b] += incr, cnt[b] times; the counts are left zero for the next call.
+__global__ __launch_bounds__(256) void k_hist_add(unsigned long long *__restrict__ cnt, double *__restrict__ fx,
+                                                  int points, double incr) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= points) return;
+  fx[b] = add_repeated(fx[b], incr, cnt[b]);
+  cnt[b] = 0;
 }
 
 // S(q) of two bead sets (each the union of up to two BeadSets):
@@ -193,41 +300,45 @@ static int obs_geo(md_simulation_t_x *sim, ObsGeo &g) {
   return 0;
 }
 
-// counts -> stats->fxs[N-1][b] += incr, once per count
-static int add_counts(md_stats_t_x *stats, const unsigned long long *dcnt, int points, double incr) {
-  std::vector<unsigned long long> h(points);
-  XMD_CHECK(hipMemcpy(h.data(), dcnt, points * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-  double *fx = stats->fxs[stats->N - 1];
-  for (int b = 0; b < points; ++b)
-    for (unsigned long long c = 0; c < h[b]; ++c) fx[b] += incr;
-  return 0;
+// Device counts of at least `points` bins, all zero between calls (k_hist_add
+// clears what it has read; a call that failed in between drops the buffer).
+static unsigned long long *g_counts = nullptr;
+static int g_counts_cap = 0;
+
+static void obs_counts_drop() {
+  if (g_counts) (void)hipFree(g_counts);
+  g_counts = nullptr;
+  g_counts_cap = 0;
 }
 
 static unsigned long long *obs_counts(int points) {
-  static unsigned long long *buf = nullptr;
-  static int cap = 0;
-  if (points > cap) {
-    if (buf) (void)hipFree(buf);
-    buf = nullptr;
-    cap = 0;
-    if (hipMalloc(&buf, points * sizeof(unsigned long long)) != hipSuccess) return nullptr;
-    cap = points;
+  if (points > g_counts_cap) {
+    obs_counts_drop();
+    if (hipMalloc(&g_counts, points * sizeof(unsigned long long)) != hipSuccess) return nullptr;
+    if (hipMemset(g_counts, 0, points * sizeof(unsigned long long)) != hipSuccess) {
+      obs_counts_drop();
+      return nullptr;
+    }
+    g_counts_cap = points;
   }
-  return buf;
+  return g_counts;
 }
 
-// Device scratch of n doubles for S(q) outputs and q vectors (grown on demand, kept).
-static double *obs_doubles(int slot, int n) {
-  static double *buf[2] = {nullptr, nullptr};
-  static int cap[2] = {0, 0};
-  if (n > cap[slot]) {
-    if (buf[slot]) (void)hipFree(buf[slot]);
-    buf[slot] = nullptr;
-    cap[slot] = 0;
-    if (hipMalloc(&buf[slot], n * sizeof(double)) != hipSuccess) return nullptr;
-    cap[slot] = n;
+// counts -> stats->fxs[N-1][b] += incr, once per count
+static int add_counts(md_stats_t_x *stats, int points, double incr) {
+  double *fx = stats->fxs[stats->N - 1], *h = host_scratch(points);
+  const hipStream_t st = rt().s0;
+  if (h) {
+    memcpy(h, fx, points * sizeof(double));
+    hipLaunchKernelGGL(k_hist_add, dim3((points + 255) / 256), dim3(256), 0, st, g_counts, h, points, incr);
   }
-  return buf[slot];
+  if (!h || hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
+    fprintf(stderr, "xmd: histogram accumulation failed\n");
+    obs_counts_drop();
+    return -1;
+  }
+  memcpy(fx, h, points * sizeof(double));
+  return 0;
 }
 
 // Bead slice `bead` (1-based) of every particle of a system.
@@ -248,15 +359,15 @@ static DevPimd *obs_pimd(md_pimd_t_x *pimd) {
 static int run_pair_hist(PairHist &h, md_stats_t_x *stats, double incr) {
   unsigned long long *cnt = obs_counts(h.points);
   if (!cnt) return -1;
-  hipStream_t st = rt().s0;
-  XMD_CHECK(hipMemsetAsync(cnt, 0, h.points * sizeof(unsigned long long), st));
   const long work = (long)h.a.N * h.b.N;
   if (work > 0) {
-    hipLaunchKernelGGL(k_pair_hist, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, st, h, cnt);
-    XMD_CHECK(hipGetLastError());
+    const dim3 grid((unsigned)((work + kHistWork - 1) / kHistWork));
+    if (h.points <= kLdsBins)
+      hipLaunchKernelGGL(k_pair_hist<true>, grid, dim3(256), h.points * sizeof(unsigned), rt().s0, h, cnt);
+    else
+      hipLaunchKernelGGL(k_pair_hist<false>, grid, dim3(256), 0, rt().s0, h, cnt);
   }
-  XMD_CHECK(hipStreamSynchronize(st));
-  return add_counts(stats, cnt, h.points, incr);
+  return add_counts(stats, h.points, incr);
 }
 
 static PairHist pair_hist(DevPimd *a, int bead_a, DevPimd *b, int bead_b, md_simulation_t_x *box_sim, int mode,
@@ -280,21 +391,17 @@ static PairHist pair_hist(DevPimd *a, int bead_a, DevPimd *b, int bead_b, md_sim
 static int run_sk(SkArgs &a, md_stats_t_x *stats, int npts, const double *qis_host) {
   if (npts <= 0) return 0;
   hipStream_t st = rt().s0;
-  double *out = obs_doubles(0, npts);
+  double *out = host_scratch(4 * (size_t)npts);  // results, then q vectors
   if (!out) return -1;
   a.qis = nullptr;
   if (a.sphere) {
-    double *q = obs_doubles(1, 3 * npts);
-    if (!q) return -1;
-    XMD_CHECK(hipMemcpyAsync(q, qis_host, 3 * npts * sizeof(double), hipMemcpyHostToDevice, st));
-    a.qis = q;
+    memcpy(out + npts, qis_host, 3 * npts * sizeof(double));
+    a.qis = out + npts;
   }
   hipLaunchKernelGGL(k_sk, dim3(npts), dim3(256), 0, st, a, 0, out);
   XMD_CHECK(hipGetLastError());
-  std::vector<double> h(npts);
-  XMD_CHECK(hipMemcpyAsync(h.data(), out, npts * sizeof(double), hipMemcpyDeviceToHost, st));
   XMD_CHECK(hipStreamSynchronize(st));
-  for (int j = 0; j < npts; ++j) stats->fxs[stats->N - 1][j] += h[j];
+  for (int j = 0; j < npts; ++j) stats->fxs[stats->N - 1][j] += out[j];
   return 0;
 }
 
@@ -317,13 +424,13 @@ int md_pimd_calc_density_distribution_x(md_pimd_t_x *pimd, md_stats_t_x *stats, 
   g.image = image;
   unsigned long long *cnt = obs_counts(g.points);
   if (!cnt) return -1;
-  hipStream_t st = rt().s0;
-  XMD_CHECK(hipMemsetAsync(cnt, 0, g.points * sizeof(unsigned long long), st));
   const int nb = p->ds->nb;
-  hipLaunchKernelGGL(k_density_hist, dim3((nb + 255) / 256), dim3(256), 0, st, p->ds->X, nb, g, cnt);
-  XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipStreamSynchronize(st));
-  return add_counts(stats, cnt, g.points, 1.0 / pimd->P);
+  const dim3 grid(std::min((nb + 255) / 256, 128));
+  if (g.points <= kLdsBins)
+    hipLaunchKernelGGL(k_density_hist<true>, grid, dim3(256), g.points * sizeof(unsigned), rt().s0, p->ds->X, nb, g, cnt);
+  else
+    hipLaunchKernelGGL(k_density_hist<false>, grid, dim3(256), 0, rt().s0, p->ds->X, nb, g, cnt);
+  return add_counts(stats, g.points, 1.0 / pimd->P);
 }
 
 int md_pimd_calc_pair_correlation_x(md_pimd_t_x *pimd, md_stats_t_x *stats, md_num_t_x rmax, md_num_t_x norm,
@@ -352,16 +459,18 @@ int md_pimd_calc_pair_correlation_2d_x(md_pimd_t_x *pimd, md_stats_t_x *stats, m
                                        md_num_t_x *box) {
   DevPimd *p = obs_pimd(pimd);
   if (!p || !stats || stats->points <= 0 || !box) return -1;
-  unsigned long long *cnt = obs_counts(stats->points);
+  const int points = stats->points;
+  unsigned long long *cnt = obs_counts(points);
   if (!cnt) return -1;
-  hipStream_t st = rt().s0;
-  XMD_CHECK(hipMemsetAsync(cnt, 0, stats->points * sizeof(unsigned long long), st));
   const long work = (long)p->P * p->N * p->N;
-  hipLaunchKernelGGL(k_paircorr_box2d, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, st, p->ds->X, p->N,
-                     p->ds->nb, p->P, box[0], box[1], box[2], box[3], rmax / stats->points, stats->points, cnt);
-  XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipStreamSynchronize(st));
-  return add_counts(stats, cnt, stats->points, 1.0 / norm);
+  const dim3 grid((unsigned)((work + kHistWork - 1) / kHistWork));
+  if (points <= kLdsBins)
+    hipLaunchKernelGGL(k_paircorr_box2d<true>, grid, dim3(256), points * sizeof(unsigned), rt().s0, p->ds->X, p->N,
+                       p->ds->nb, p->P, box[0], box[1], box[2], box[3], rmax / points, points, cnt);
+  else
+    hipLaunchKernelGGL(k_paircorr_box2d<false>, grid, dim3(256), 0, rt().s0, p->ds->X, p->N, p->ds->nb, p->P, box[0],
+                       box[1], box[2], box[3], rmax / points, points, cnt);
+  return add_counts(stats, points, 1.0 / norm);
 }
 
 int md_pimd_calc_2d_pair_correlation_x(md_pimd_t_x *pimd, md_stats_t_x *stats, md_num_t_x rmax, md_num_t_x norm,

@@ -125,6 +125,11 @@ int ensure_pimd_device(md_pimd_t_x *pimd);
 int download_sim(DevSim *d);                         // device -> host mirror
 int download_pimd(DevPimd *p);
 
+// Pinned host memory of at least n doubles that kernels read and write
+// directly (grown on demand, kept; used by one call at a time, which waits
+// for its kernels before it returns); nullptr on failure.
+double *host_scratch(size_t n);
+
 // reductions: sum of n doubles on device into *out (host), deterministic
 int device_sum(const double *src, int n, double *out);
 // up to four such sums with one wait for the results
