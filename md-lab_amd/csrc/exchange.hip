@@ -2028,12 +2028,13 @@ static int run_estimator(DevPimd *p, const double *Bm, double *out) {
   o.P = o.dg + (size_t)nblk * RSQ;
   o.bn = o.P + tri;
   o.mask = (unsigned *)(o.bn + N);
-  double *d_out = p->work + 4 * (N + 1);
+  double *h = host_scratch(1);
+  if (!h) return -1;
   hipLaunchKernelGGL(k_est_weights, dim3(nblk * RB), dim3(256), 0, rt().s0, a, Bm, o);
-  hipLaunchKernelGGL(k_est_solve, dim3(1), dim3(RT), 0, rt().s0, N, o, d_out);
+  hipLaunchKernelGGL(k_est_solve, dim3(1), dim3(RT), 0, rt().s0, N, o, h);
   XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipMemcpyAsync(out, d_out, sizeof(double), hipMemcpyDeviceToHost, rt().s0));
   XMD_CHECK(hipStreamSynchronize(rt().s0));
+  *out = *h;
   return 0;
 }
 
@@ -2388,13 +2389,14 @@ static int vi_sign_grid(DevPimd *p, int n, const double *vi2, double *out) {
     return -1;
   }
   RecArgs a = rec_args(p);
-  double *d_vi = p->work + 4 * (p->N + 1) + 8, *d_out = d_vi + 512;
+  double *h = host_scratch(2 * (size_t)n);  // xi', then the factors
+  if (!h) return -1;
+  for (int i = 0; i < n; ++i) h[i] = vi2[i];
   hipStream_t st = rt().s0;
-  XMD_CHECK(hipMemcpyAsync(d_vi, vi2, n * sizeof(double), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_vi_sign, dim3(n), dim3(SIGN_WG), 0, st, a, d_vi, d_out);
+  hipLaunchKernelGGL(k_vi_sign, dim3(n), dim3(SIGN_WG), 0, st, a, h, h + n);
   XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipMemcpyAsync(out, d_out, n * sizeof(double), hipMemcpyDeviceToHost, st));
   XMD_CHECK(hipStreamSynchronize(st));
+  for (int i = 0; i < n; ++i) out[i] = h[n + i];
   return 0;
 }
 
