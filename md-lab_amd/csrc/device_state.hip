@@ -5,8 +5,12 @@
 // md_pimd_sync_host_x copy the device state back into the reference-layout
 // host mirrors (read_only = 0 also returns authority to the host, as in
 // md_util_x.c:481-551 / md_pimd_x.c:271-328).
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <mutex>
+#include <thread>
 #include <unordered_map>
 
 #include "xmd_internal.h"
@@ -131,11 +135,14 @@ __global__ void k_chains_to_device(const md_nhc_t_x *__restrict__ in, double *th
   }
 }
 
-__global__ void k_chains_to_host(md_nhc_t_x *__restrict__ out, const double *th, const double *vth,
+// up: the records of the upload, for the fields the device does not keep
+// (the host's own records are not sent up again).
+__global__ void k_chains_to_host(md_nhc_t_x *out, const md_nhc_t_x *up, const double *th, const double *vth,
                                  const double *Q, int Nf, int nb, int N, int P, int massive, int M) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= Nf) return;
   int e = massive ? (i % 3) * nb + slot_of(i / 3, N, P) : i;
+  out[i].f = up[i].f;
   for (int k = 0; k < M; ++k) {
     out[i].theta[k] = th[k * Nf + e];
     out[i].vtheta[k] = vth[k * Nf + e];
@@ -272,22 +279,88 @@ int ensure_device(md_simulation_t_x *sim) {
   return 0;
 }
 
+// The bead and chain records of a download.  The host mirrors are pageable,
+// and a runtime copy to pageable memory runs at the rate of the one thread
+// that moves the staged bytes (17 GB/s at 20 MB, and 0.1 ms to set up at any
+// size).  Up to kDirectBytes the packing kernels write the records straight
+// into pinned memory, from which the caller's thread moves them; larger ones
+// are packed on the device and copied in 1 MB pieces by four threads, each
+// through its own pinned slot and stream, so that device copies and host
+// moves overlap (N=1024 P=32, 22 MB: 2.0 -> 0.6 ms).  One caller at a time.
+constexpr int kCopyThreads = 4;
+constexpr size_t kPieceBytes = 1u << 20, kDirectBytes = 3u << 20;
+static std::mutex g_copy_busy;
+static char *g_copy_slots = nullptr;  // kCopyThreads pieces, pinned, kept
+
+// Device memory to host in pieces, after everything queued on s0.
+struct HostCopy {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+
+static int copy_pieces(const HostCopy *list, int count) {
+  static hipStream_t lane[kCopyThreads];
+  for (int t = 0; t < kCopyThreads; ++t)
+    if (!lane[t]) XMD_CHECK(hipStreamCreateWithFlags(&lane[t], hipStreamNonBlocking));
+  XMD_CHECK(hipStreamSynchronize(rt().s0));
+  std::vector<HostCopy> piece;
+  for (int i = 0; i < count; ++i)
+    for (size_t o = 0; o < list[i].bytes; o += kPieceBytes)
+      piece.push_back({(char *)list[i].dst + o, (const char *)list[i].src + o, std::min(kPieceBytes, list[i].bytes - o)});
+  std::atomic<size_t> next{0};
+  std::atomic<int> failed{0};
+  const int device = rt().device;
+  auto work = [&](int t) {
+    char *slot = g_copy_slots + t * kPieceBytes;
+    if (hipSetDevice(device) != hipSuccess) failed = 1;
+    for (size_t k; !failed && (k = next++) < piece.size();) {
+      const HostCopy &c = piece[k];
+      if (hipMemcpyAsync(slot, c.src, c.bytes, hipMemcpyDeviceToHost, lane[t]) != hipSuccess ||
+          hipStreamSynchronize(lane[t]) != hipSuccess)
+        failed = 1;
+      else
+        memcpy(c.dst, slot, c.bytes);
+    }
+  };
+  std::thread helper[kCopyThreads - 1];
+  int started = 0;
+  try {
+    for (; started < kCopyThreads - 1; ++started) helper[started] = std::thread(work, started + 1);
+  } catch (...) {  // no thread to be had: the caller's own does the rest
+  }
+  work(0);
+  for (int t = 0; t < started; ++t) helper[t].join();
+  if (failed) {
+    fprintf(stderr, "xmd: copy to the host failed\n");
+    return -1;
+  }
+  return 0;
+}
+
 int download_sim(DevSim *d) {
   md_simulation_t_x *sim = d->host;
   hipStream_t st = rt().s0;
   int nb = d->nb, Nf = d->Nf;
-  hipLaunchKernelGGL(k_beads_to_host, dim3((nb + 255) / 256), dim3(256), 0, st, (md_particle_t_x *)d->stage,
-                     d->X, d->V, d->F, d->M, nb, d->N, d->P);
+  const size_t bbytes = nb * sizeof(md_particle_t_x), cbytes = Nf * sizeof(md_nhc_t_x);
+  std::lock_guard<std::mutex> hold(g_copy_busy);
+  if (!g_copy_slots) XMD_CHECK(hipHostMalloc((void **)&g_copy_slots, kCopyThreads * kPieceBytes, hipHostMallocDefault));
+  const bool direct = bbytes + cbytes <= kDirectBytes;
+  md_particle_t_x *beads = (md_particle_t_x *)(direct ? g_copy_slots : d->stage);
+  md_nhc_t_x *chains = (md_nhc_t_x *)(direct ? g_copy_slots + bbytes : d->nstage);
+  hipLaunchKernelGGL(k_beads_to_host, dim3((nb + 255) / 256), dim3(256), 0, st, beads, d->X, d->V, d->F, d->M, nb,
+                     d->N, d->P);
+  hipLaunchKernelGGL(k_chains_to_host, dim3((Nf + 255) / 256), dim3(256), 0, st, chains, (const md_nhc_t_x *)d->nstage,
+                     d->th, d->vth, d->Q, Nf, nb, d->N, d->P, d->massive ? 1 : 0, MD_NHC_LENGTH_X);
   XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipMemcpyAsync(sim->particles, d->stage, nb * sizeof(md_particle_t_x), hipMemcpyDeviceToHost, st));
-  // chain slots beyond the integrated length keep their host values
-  XMD_CHECK(hipMemcpyAsync(d->nstage, sim->nhcs, Nf * sizeof(md_nhc_t_x), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_chains_to_host, dim3((Nf + 255) / 256), dim3(256), 0, st, (md_nhc_t_x *)d->nstage, d->th,
-                     d->vth, d->Q, Nf, nb, d->N, d->P, d->massive ? 1 : 0, MD_NHC_LENGTH_X);
-  XMD_CHECK(hipGetLastError());
-  XMD_CHECK(hipMemcpyAsync(sim->nhcs, d->nstage, Nf * sizeof(md_nhc_t_x), hipMemcpyDeviceToHost, st));
-  XMD_CHECK(hipStreamSynchronize(st));
-  return 0;
+  if (direct) {
+    XMD_CHECK(hipStreamSynchronize(st));
+    memcpy(sim->particles, beads, bbytes);
+    memcpy(sim->nhcs, chains, cbytes);
+    return 0;
+  }
+  const HostCopy out[2] = {{sim->particles, beads, bbytes}, {sim->nhcs, chains, cbytes}};
+  return copy_pieces(out, 2);
 }
 
 static int alloc_pimd(DevPimd *p) {
