@@ -96,73 +96,121 @@ __device__ __forceinline__ double e2(const double *X, const double *M, int nb, i
 
 // ------------------------------------------------------------ E_n^(k)
 
-// Particle l (0-based): Eint_l, E_l^(1), link C_l.  A block holds 64
-// particles (lanes); its four waves split the P - 1 interior springs and
-// the partial sums are added in a fixed order.
-__device__ __forceinline__ void chain_body(int bx, const double *__restrict__ X, const double *__restrict__ M, int N,
-                                           int P, double om, Geo g, double *__restrict__ Eint,
-                                           double *__restrict__ Clink, double *__restrict__ ENk,
-                                           double *__restrict__ ET) {
-  __shared__ double part[4][64];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int l = bx * 64 + lane;
-  const int nb = N * P;
-  double e = 0;
-  if (l < N) {
-    const int j0 = ((P - 1) * wv) / 4, j1 = ((P - 1) * (wv + 1)) / 4;
-    for (int j = j0; j < j1; ++j) e += spring_e(X, nb, j * N + l, (j + 1) * N + l, M[j * N + l], om, g);
-  }
-  part[wv][lane] = e;
-  __syncthreads();
-  if (wv == 0 && l < N) {
-    e = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
-    Eint[l] = e;
-    const int sP = (P - 1) * N + l;
-    const double e1 = e + spring_e(X, nb, sP, l, M[sP], om, g);
-    ENk[tri_row(l + 1)] = e1;
-    ET[col_off(l, N)] = e1;
-    Clink[l] = (l < N - 1) ? e + spring_e(X, nb, sP, l + 1, M[sP], om, g) : 0.0;
-  }
+// The two factors of spring_e, t d = 1/2 m w^2 d^2: a sum of springs is a
+// sequence of fma(t, d, sum) whose operands are ready beforehand.
+struct SpringTD {
+  double t, d;
+};
+__device__ __forceinline__ SpringTD spring_td(const double *X, int nb, int sa, int sb, double m, double om,
+                                              const Geo &g) {
+  const double dx = comp_sq(X[sa] - X[sb], g.L0, g.iL0, g.image);
+  const double dy = comp_sq(X[nb + sa] - X[nb + sb], g.L1, g.iL1, g.image);
+  const double dz = comp_sq(X[2 * nb + sa] - X[2 * nb + sb], g.L2, g.iL2, g.image);
+  const double d = sqrt(dx * dx + dy * dy + dz * dz);
+  return SpringTD{0.5 * m * om * om * d, d};
 }
 
-__global__ __launch_bounds__(256) void k_chain(const double *__restrict__ X, const double *__restrict__ M, int N,
-                                               int P, double om, Geo g, double *__restrict__ Eint,
-                                               double *__restrict__ Clink, double *__restrict__ ENk,
-                                               double *__restrict__ ET) {
-  chain_body(blockIdx.x, X, M, N, P, om, g, Eint, Clink, ENk, ET);
+// Particle l (0-based): Eint_l, E_l^(1), link C_l.  A block holds CHAIN_PW
+// particles.  Its 256 threads compute their springs (the P - 1 interior ones,
+// then bead P-1 to bead 0 of the particle and of the next one) into LDS, 16
+// springs of every particle at a time; four threads per particle then add the
+// interior springs of a quarter of the beads each, one by one, and the four
+// sums are added in a fixed order.  (64 particles per block with the springs
+// of a quarter computed and added by one thread: the fused kernel took 13.8
+// us at N = 256, P = 64 and 5.9 at N = P = 8 against 9.0 and 2.4 here; unrolling that loop by 8 to have more
+// loads in flight made it slower, its code comes from a cold cache.)
+// Returns C_l in threads below CHAIN_PW (0 past the last particle).
+constexpr int CHAIN_PW = 16, CHAIN_CH = 80;
+
+__device__ __forceinline__ double chain_body(int bx, const double *__restrict__ X, const double *__restrict__ M, int N,
+                                             int P, double om, Geo g, double *__restrict__ Eint,
+                                             double *__restrict__ ENk, double *__restrict__ ET) {
+  __shared__ SpringTD sp[CHAIN_CH][CHAIN_PW];
+  __shared__ double part[4][CHAIN_PW];
+  const int t = threadIdx.x, i = t % CHAIN_PW, wq = t / CHAIN_PW;
+  const int l = bx * CHAIN_PW + i, lc = min(l, N - 1), ln = min(l + 1, N - 1);
+  const int nb = N * P, sP = (P - 1) * N;
+  const int j0 = ((P - 1) * wq) / 4, j1 = wq < 4 ? ((P - 1) * (wq + 1)) / 4 : 0;
+  double e = 0;
+  for (int c0 = 0; c0 <= P; c0 += CHAIN_CH) {
+    const int c1 = min(c0 + CHAIN_CH, P + 1);
+    if (c0 > 0) __syncthreads();
+#pragma unroll 1
+    for (int j = c0 + wq; j < c1; j += 256 / CHAIN_PW) {
+      const int a = min(j, P - 1) * N + lc;
+      const int b = j < P - 1 ? a + N : j == P - 1 ? lc : ln;
+      sp[j - c0][i] = spring_td(X, nb, a, b, M[a], om, g);
+    }
+    __syncthreads();
+    for (int j = max(j0, c0); j < min(j1, c1); ++j) e = fma(sp[j - c0][i].t, sp[j - c0][i].d, e);
+  }
+  if (wq < 4) part[wq][i] = e;
+  const int last = (P / CHAIN_CH) * CHAIN_CH;  // first spring of the last chunk
+  SpringTD close = sp[max(0, P - 1 - last)][i], link = sp[P - last][i];
+  if (P - 1 < last) close = spring_td(X, nb, sP + lc, lc, M[sP + lc], om, g);
+  __syncthreads();
+  if (wq != 0 || l >= N) return 0.0;
+  e = ((part[0][i] + part[1][i]) + part[2][i]) + part[3][i];
+  Eint[l] = e;
+  const double e1 = fma(close.t, close.d, e);
+  ENk[tri_row(l + 1)] = e1;
+  ET[col_off(l, N)] = e1;
+  return l < N - 1 ? fma(link.t, link.d, e) : 0.0;
 }
 
 // Exclusive double-double prefix sum of in[0..n-1] into pre[2*i] (hi, lo)
-// by one workgroup of NT threads.
-template <int NT = 256>
+// by one workgroup of NT threads.  DEV: in[] was written by other workgroups
+// of the same launch (device-scope loads).  The segment values are loaded in
+// groups before they are added one by one, the tree has only the levels that
+// segments in use can reach, and its levels alternate between two buffers
+// (one barrier each).
+template <bool DEV, int NT = 256>
 __device__ __forceinline__ void scan_dd_body(const double *__restrict__ in, int n, double *__restrict__ pre) {
-  __shared__ double sh[NT], sl[NT];
+  constexpr int G = 8;
+  __shared__ dd sh[2][NT];
   const int t = threadIdx.x;
   const int seg = (n + NT - 1) / NT;
   const int a = min(n, t * seg), b = min(n, a + seg);
+  auto load = [&](int i) {
+    const double *q = in + min(i, n - 1);
+    return DEV ? __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *q;
+  };
   dd tot{0, 0};
-  for (int i = a; i < b; ++i) tot = dd_add(tot, dd{in[i], 0});
-  sh[t] = tot.hi;
-  sl[t] = tot.lo;
+  double x[G];
+  for (int i = a; i < b; i += G) {
+#pragma unroll
+    for (int k = 0; k < G; ++k) x[k] = k < seg ? load(i + k) : 0.0;
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+      if (i + k < b) tot = dd_add(tot, dd{x[k], 0});
+  }
+  int cur = 0;
+  sh[0][t] = tot;
   __syncthreads();
-  for (int w = 1; w < NT; w <<= 1) {
-    dd v{sh[t], sl[t]};
-    if (t >= w) v = dd_add(v, dd{sh[t - w], sl[t - w]});
-    __syncthreads();
-    sh[t] = v.hi;
-    sl[t] = v.lo;
+  for (int w = 1; w < NT && w * seg < n; w <<= 1) {
+    dd v = sh[cur][t];
+    if (t >= w) v = dd_add(v, sh[cur][t - w]);
+    cur ^= 1;
+    sh[cur][t] = v;
     __syncthreads();
   }
-  dd run = t > 0 ? dd{sh[t - 1], sl[t - 1]} : dd{0, 0};
-  for (int i = a; i < b; ++i) {
-    pre[2 * i] = run.hi;
-    pre[2 * i + 1] = run.lo;
-    run = dd_add(run, dd{in[i], 0});
+  dd run = t > 0 ? sh[cur][t - 1] : dd{0, 0};
+  for (int i = a; i < b; i += G) {
+    if (seg > G)
+#pragma unroll
+      for (int k = 0; k < G; ++k) x[k] = load(i + k);
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+      if (i + k < b) {
+        pre[2 * (i + k)] = run.hi;
+        pre[2 * (i + k) + 1] = run.lo;
+        run = dd_add(run, dd{x[k], 0});
+      }
   }
 }
 
 __global__ __launch_bounds__(256) void k_scan_dd(const double *__restrict__ in, int n, double *__restrict__ pre) {
-  scan_dd_body(in, n, pre);
+  scan_dd_body<false>(in, n, pre);
 }
 
 // In the concurrent step the cycle energies, the recursion set-up, the
@@ -174,43 +222,84 @@ __global__ __launch_bounds__(256) void k_scan_dd(const double *__restrict__ in, 
 // put it on the longest chain).
 __device__ __forceinline__ void chain_priority() { __builtin_amdgcn_s_setprio(3); }
 
-// k_chain and k_scan_dd in one launch: the last workgroup to finish its
-// particles (counted in *done, which it resets) scans the links.
+// Springs, links and their prefix sums in one launch: the last workgroup to finish its
+// particles (counted in *done, which it resets) scans the links.  They are
+// stored through to memory and read from there, and the count follows once
+// the stores have completed, so no cache is flushed or emptied for the rest
+// of what the kernels beside this one hold in it.
 __global__ __launch_bounds__(256) void k_chain_scan(const double *__restrict__ X, const double *__restrict__ M, int N,
                                                     int P, double om, Geo g, double *__restrict__ Eint,
                                                     double *__restrict__ Clink, double *__restrict__ ENk,
                                                     double *__restrict__ ET, double *__restrict__ pre,
                                                     int *__restrict__ done) {
   __shared__ int last;
+  __shared__ double link[CHAIN_PW];
   chain_priority();
-  chain_body(blockIdx.x, X, M, N, P, om, g, Eint, Clink, ENk, ET);
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  const double c = chain_body(blockIdx.x, X, M, N, P, om, g, Eint, ENk, ET);
+  const int l = blockIdx.x * CHAIN_PW + threadIdx.x;
+  if (gridDim.x == 1) {
+    if (threadIdx.x < CHAIN_PW) link[threadIdx.x] = c;
+    __syncthreads();
+    scan_dd_body<false>(link, N, pre);
+    return;
+  }
+  if (threadIdx.x < 64) {
+    if (threadIdx.x < CHAIN_PW && l < N) __hip_atomic_store(Clink + l, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    if (threadIdx.x == 0)
+      last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  }
   __syncthreads();
   if (!last) return;
-  __threadfence();
-  scan_dd_body(Clink, N, pre);
+  scan_dd_body<true>(Clink, N, pre);
   if (threadIdx.x == 0) __hip_atomic_store(done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Row n' (0-based) of the cycle-energy triangle, k >= 2, both layouts.
-__device__ __forceinline__ void enk_fill_body(int r, const double *__restrict__ X, const double *__restrict__ M,
+// Cycle energies with k >= 2, both layouts, one EKT x EKT tile per workgroup:
+// particles r (last of the cycle) by m0 (first).  The rows of ENk are written
+// as they are computed, lanes along m0; the columns of ET from a copy in LDS,
+// lanes along r.  (A workgroup per row r wrote ET one double per column, N
+// doubles apart, every line in parts from several XCDs: the step with
+// nothing beside the set-up took 9026 us per 16 steps at N = 2001, P = 24 and
+// 6033 per 20 at N = 1024, P = 32, with the tiles 8773 and 5953.)
+constexpr int EKT = 32;
+
+__host__ __device__ inline int enk_tiles(int N) {
+  const int n = (N + EKT - 1) / EKT;
+  return n * (n + 1) / 2;
+}
+
+__device__ __forceinline__ void enk_fill_body(int tile, const double *__restrict__ X, const double *__restrict__ M,
                                               int N, int P, double om, Geo g, const double *__restrict__ Eint,
                                               const double *__restrict__ pre, double *__restrict__ ENk,
                                               double *__restrict__ ET) {
-  // r: 0-based last particle of the cycle
+  __shared__ double T[EKT][EKT + 1];
+  int tr = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
+  while (tr * (tr + 1) / 2 > tile) --tr;
+  while ((tr + 1) * (tr + 2) / 2 <= tile) ++tr;
+  const int r0 = tr * EKT, c0 = (tile - tr * (tr + 1) / 2) * EKT;
+  const int lane = threadIdx.x % EKT, sub = threadIdx.x / EKT;
   const int nb = N * P;
-  const int sP = (P - 1) * N + r;
-  const double mP = M[sP], ein = Eint[r];
-  const dd ar{pre[2 * r], pre[2 * r + 1]};
-  for (int k = 2 + threadIdx.x; k <= r + 1; k += blockDim.x) {
-    const int m0 = r - k + 1;  // 0-based first particle
+  const int m0 = c0 + lane;
+#pragma unroll
+  for (int i = 0; i < EKT; i += 256 / EKT) {
+    const int r = r0 + i + sub;
+    if (r >= N || m0 >= r) continue;
+    const int sP = (P - 1) * N + r;
+    const double mP = M[sP], ein = Eint[r];
+    const dd ar{pre[2 * r], pre[2 * r + 1]};
     double chain = dd_sub_to_double(ar, dd{pre[2 * m0], pre[2 * m0 + 1]});
     double E = chain + ein + spring_e(X, nb, sP, m0, mP, om, g);
-    ENk[tri_row(r + 1) + k - 1] = E;
-    ET[col_off(m0, N) + k - 1] = E;
+    ENk[tri_row(r + 1) + r - m0] = E;
+    T[i + sub][lane] = E;
+  }
+  __syncthreads();
+  const int r = r0 + lane;
+#pragma unroll
+  for (int i = 0; i < EKT; i += 256 / EKT) {
+    const int m = c0 + i + sub;
+    if (r < N && m < r) ET[col_off(m, N) + r - m] = T[lane][i + sub];
   }
 }
 
@@ -222,7 +311,7 @@ __global__ __launch_bounds__(256) void k_enk_fill(const double *__restrict__ X, 
 }
 
 // Positions, masses and prefix sums from which a cycle energy is computed
-// directly, with the arithmetic of k_chain (k = 1) and k_enk_fill (k >= 2).
+// directly, with the arithmetic of k_chain_scan (k = 1) and k_enk_fill (k >= 2).
 struct EnkArgs {
   const double *X, *M, *Eint, *pre;
   double om;
@@ -529,19 +618,19 @@ __global__ __launch_bounds__(256) void k_rec_prep(RecArgs a, int dir0) {
   rec_prep_wg<false>(a, dir0 + blockIdx.y, blockIdx.x, EnkArgs{}, E);
 }
 
-// k_enk_fill (workgroups 0 .. N-1) and the recursion set-up of both
-// directions (the next 2 nprepb workgroups, coefficients computed directly)
-// in one launch.
+// The recursion set-up of both directions (workgroups 0 .. 2 nprepb - 1,
+// coefficients computed directly) and k_enk_fill (the next enk_tiles(N)) in
+// one launch.
 __global__ __launch_bounds__(256) void k_enk_prep(EnkArgs e, double *__restrict__ ENk, double *__restrict__ ET,
                                                   RecArgs a, int nprepb) {
   __shared__ double E[2][RB + 1];
   chain_priority();
-  const int bx = blockIdx.x;
-  if (bx < e.N) {
-    enk_fill_body(bx, e.X, e.M, e.N, e.P, e.om, e.g, e.Eint, e.pre, ENk, ET);
+  const int w = blockIdx.x;
+  if (w >= 2 * nprepb) {
+    enk_fill_body(w - 2 * nprepb, e.X, e.M, e.N, e.P, e.om, e.g, e.Eint, e.pre, ENk, ET);
     return;
   }
-  const int w = bx - e.N, dir = w / nprepb;
+  const int dir = w / nprepb;
   rec_prep_wg<true>(a, dir, w - dir * nprepb, e, E);
 }
 
@@ -1529,13 +1618,15 @@ __global__ __launch_bounds__(256) void kb_chain(const ExRep *__restrict__ reps, 
                                                 int nrep) {
   const int r = batch_rep(start, nrep, blockIdx.x);
   const ExRep &R = reps[r];
-  chain_body(blockIdx.x - start[r], R.X, R.M, R.N, R.P, R.om, R.g, R.Eint, R.clink, R.ENk, R.ET);
+  const int l = (blockIdx.x - start[r]) * CHAIN_PW + threadIdx.x;
+  const double c = chain_body(blockIdx.x - start[r], R.X, R.M, R.N, R.P, R.om, R.g, R.Eint, R.ENk, R.ET);
+  if (threadIdx.x < CHAIN_PW && l < R.N) R.clink[l] = c;
 }
 
-// one 1024-thread block per replica
+// one workgroup per replica
 __global__ __launch_bounds__(256) void kb_scan_dd(const ExRep *__restrict__ reps) {
   const ExRep &R = reps[blockIdx.x];
-  scan_dd_body(R.clink, R.N, R.Cpre);
+  scan_dd_body<false>(R.clink, R.N, R.Cpre);
 }
 
 __global__ __launch_bounds__(256) void kb_enk_fill(const ExRep *__restrict__ reps, const int *__restrict__ start,
@@ -1631,12 +1722,10 @@ int launch_enk(DevPimd *p, int image, hipStream_t st) {
   Geo g = geo_of(p, image);
   double om = p->host->omegaP;
   double *clink = p->work + (N + 1);
-  hipLaunchKernelGGL(k_chain, dim3((N + 63) / 64), dim3(256), 0, st, d->X, d->M, N, P, om, g, p->Eint, clink,
-                     p->ENk, p->ET);
+  hipLaunchKernelGGL(k_chain_scan, dim3((N + CHAIN_PW - 1) / CHAIN_PW), dim3(256), 0, st, d->X, d->M, N, P, om, g,
+                     p->Eint, clink, p->ENk, p->ET, p->Cpre, p->done);
   XMD_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_scan_dd, dim3(1), dim3(256), 0, st, clink, N, p->Cpre);
-  XMD_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_enk_fill, dim3(N), dim3(256), 0, st, d->X, d->M, N, P, om, g, p->Eint, p->Cpre, p->ENk, p->ET);
+  hipLaunchKernelGGL(k_enk_fill, dim3(enk_tiles(N)), dim3(256), 0, st, d->X, d->M, N, P, om, g, p->Eint, p->Cpre, p->ENk, p->ET);
   XMD_CHECK(hipGetLastError());
   p->enk_dev = true;
   p->last_image = image;
@@ -1707,12 +1796,12 @@ int launch_enk_prep(DevPimd *p, int image, hipStream_t st) {
   e.N = N;
   e.P = P;
   double *clink = p->work + (N + 1);
-  hipLaunchKernelGGL(k_chain_scan, dim3((N + 63) / 64), dim3(256), 0, st, d->X, d->M, N, P, e.om, e.g, p->Eint, clink,
-                     p->ENk, p->ET, p->Cpre, p->done);
+  hipLaunchKernelGGL(k_chain_scan, dim3((N + CHAIN_PW - 1) / CHAIN_PW), dim3(256), 0, st, d->X, d->M, N, P, e.om, e.g,
+                     p->Eint, clink, p->ENk, p->ET, p->Cpre, p->done);
   XMD_CHECK(hipGetLastError());
   RecArgs a = rec_args(p);
   const int nprepb = rec_prep_wgs(N, a.nblk);
-  hipLaunchKernelGGL(k_enk_prep, dim3(N + 2 * nprepb), dim3(256), 0, st, e, p->ENk, p->ET, a, nprepb);
+  hipLaunchKernelGGL(k_enk_prep, dim3(2 * nprepb + enk_tiles(N)), dim3(256), 0, st, e, p->ENk, p->ET, a, nprepb);
   XMD_CHECK(hipGetLastError());
   p->enk_dev = true;
   p->last_image = image;
@@ -1916,8 +2005,8 @@ ExchBatch *exch_batch_create(const std::vector<BatchItem> &items) {
     R.a = rec_args(p);
     R.prep_blocks = rec_prep_wgs(p->N, R.a.nblk);
     reps.push_back(R);
-    bc.push_back((p->N + 63) / 64);
-    be.push_back(p->N);
+    bc.push_back((p->N + CHAIN_PW - 1) / CHAIN_PW);
+    be.push_back(enk_tiles(p->N));
     bp.push_back(2 * R.prep_blocks);
     bf.push_back(p->N);
     b->ps.push_back(p);
@@ -1944,7 +2033,7 @@ void exch_batch_free(ExchBatch *b) {
   delete b;
 }
 
-// cycle energies (k_chain, k_scan_dd, k_enk_fill of every replica)
+// cycle energies (k_chain_scan and k_enk_fill of every replica)
 int exch_batch_enk(ExchBatch *b, hipStream_t st) {
   hipLaunchKernelGGL(kb_chain, dim3(b->chain.total), dim3(256), 0, st, (const ExRep *)b->chain.reps, b->chain.start,
                      b->nrep);
