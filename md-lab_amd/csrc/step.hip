@@ -1,30 +1,15 @@
 // The fused MD step and its hipGraph capture, plus run-time knobs.
 //
-// Stream layout of one step (the reference driver's order of stages):
-//   s0: NHC half 1 (+ wrap) --fork2--> cycle energies --fork--> reset F,
-//       trap, ring springs (pair forces here unless they are Ewald), Ewald
-//       phase tables, structure factors and reciprocal forces (into a side
-//       buffer) --wait join, join2--> add the pair and exchange end-bead
-//       forces, NHC half 2 (one kernel with massive thermostats)
-// With massive thermostats NHC half 1 and the wrap are one kernel, and so are
-// the force reset, trap and interior springs.
-//   s1: (after fork) forward + backward recursions, end-bead exchange forces
-//       into a side buffer --join--> (added into F on s0)
-//   s2: (Ewald) real-space tile sums, forked from s0 right after NHC half 1
-//       (positions only) --join2--> s0 then adds the real-space,
-//       reciprocal and exchange forces
-// The recursions only read cycle energies, so they overlap the pair forces;
-// the end-bead exchange forces are added into F after both branches are done
-// (the serial profiling order computes and adds them there in one kernel).
-// The real-space grid goes first on s2: it fills the device while the short
-// cycle-energy kernels (highest wave priority) run beside it, and the
-// recursions then overlap the matrix-core k-space kernels, which leave them
-// more of the compute units than the real-space waves do (UEG N=1024 P=32:
-// 0.219 -> 0.199 ms per step against the real-space grid on s0 after the
-// recursion fork).  The k-space kernels run on s0 after the bead-local
-// forces, beside the end of the real-space grid, rather than after it on s2
-// (0.1975 -> 0.192 ms with the phase tables moved, 0.185 -> 0.1815 ms with
-// the structure factors and forces following them).
+// Stages of one step (the reference driver's): NHC half 1 (+ wrap), cycle
+// energies and recursion set-up, recursions, end-bead exchange forces (into a
+// side buffer), bead-local forces (reset, trap, springs), pair forces (for
+// Ewald: real space; phase tables, structure factors, reciprocal forces, all
+// into side buffers), sum of the parts, NHC half 2 (one kernel with massive
+// thermostats, as are NHC half 1 with the wrap and the bead-local forces).
+// Everything between the NHC halves reads positions only, so the exchange
+// chain and the pair branch may run side by side; which parts go beside which
+// depends on how much of the device the pair kernels fill (Order below).
+// The serial profiling order runs every stage on s0.
 //
 // Batches of independent replicas (md_pimd_run_batch_x) run the same stages
 // with one launch per stage over a packed table of all replicas, captured
@@ -103,6 +88,37 @@ static Lane main_lane() {
   return L;
 }
 
+// What runs beside the exchange chain (set-up, recursions, exchange forces).
+// The chain is latency: short kernels, then two dependent solves on few
+// workgroups that each want an empty compute unit.  Beside a pair grid that
+// fills the device the short kernels wait for workgroup slots and the solves
+// for room, and a fork costs its parent 5 us; so, with w = N^2 P pair terms
+// (us per step, the order before -> the order chosen, on thermal states with
+// exchange cycles t and uniform ones u):
+//   Pairs   the pair branch on s2 and the chain on s0, both from NHC on:
+//           no pair kernel fills the device (trap N=8 P=8 45 -> 34,
+//           N=256 P=64 t 92 -> 88, u 84 -> 65; Ewald N=256 P=32 t 109 -> 100,
+//           u 99 -> 97, N=512 P=32 t 160 -> 147, u 120 -> 122)
+//   KSpace  Ewald, smaller still: bead-local and reciprocal forces on s2 from
+//           NHC on, the real space on s0 after the set-up, beside the solves
+//           on s1 (N=16 P=32 78 -> 62, N=128 P=64 t 98 -> 91, u 98 -> 90)
+//   Beside  Ewald, the real space on s2 from NHC on, bead-local and reciprocal
+//           forces on s0 after the set-up, the solves on s1 (N=1024 P=32
+//           t 273, u 188; 266 and 201 with Late)
+//   Late    as Beside, the real space after the set-up and behind the solves:
+//           they are placed first (N=1500 P=32 t 442 -> 374, u 311 -> 325;
+//           N=2001 P=24 t 600 -> 491, u 405 -> 384)
+//   After   no Ewald: pair branch on s0 after the set-up, solves on s1 (trap
+//           N=600 P=64 t 164, u 146; 214 and 161 with Pairs)
+enum class Order { Serial, Pairs, KSpace, Beside, Late, After };
+
+static Order force_order(const StepPlan &sp, bool ewald) {
+  const double w = (double)sp.p->N * sp.p->N * sp.p->P;
+  if (ewald && sp.p->sur_mode) return Order::Beside;
+  if (ewald) return w < 1.5e6 ? Order::KSpace : w < 1.2e7 ? Order::Pairs : w < 5e7 ? Order::Beside : Order::Late;
+  return w < 8e6 ? Order::Pairs : Order::After;
+}
+
 // ev: optional per-stage events (2 per stage: start, stop), may be null.
 // serial: run every stage on s0 (true per-stage device times for profiling).
 // fused (may be null: F complete on return): set (Fpart non-null) when the
@@ -111,73 +127,72 @@ static Lane main_lane() {
 static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane &R, ForceSums *fused) {
   DevPimd *p = sp.p;
   DevSim *d = p->ds;
-  hipStream_t sx = serial ? R.s0 : R.s1;
+  const int kind = sp.pair_kind;
+  const bool ewald = !serial && kind >= 0 && pair_ewald_tab(p, kind);
+  const Order o = serial ? Order::Serial : force_order(sp, ewald);
+  const bool pairs_s2 = o == Order::Pairs || o == Order::KSpace;  // bead-local and pair forces on s2
+  const bool fork_solve = o != Order::Serial && o != Order::Pairs;
+  const hipStream_t sx = fork_solve ? R.s1 : R.s0, sb = pairs_s2 ? R.s2 : R.s0;
   auto rec = [&](int k, hipStream_t st) -> int {
     if (ev) XMD_CHECK(hipEventRecord(ev[k], st));
     return 0;
   };
-  // Reciprocal space (positions only) forks onto s2 first: the phase tables
-  // and structure factors overlap the cycle energies.
-  const int kfork =
-      (!serial && sp.pair_kind >= 0) ? launch_pair_ewald_fork(p, sp.pair_kind, R.s0, R.s2, R.fork2, R.join2) : 0;
-  if (kfork < 0) return -1;
-  // Cycle energies (short, position-only); then the two recursions are
-  // forked onto s1 before the real-space grid is queued, so their
-  // workgroups are resident before it fills the device.
+  auto fork = [&](hipEvent_t e, hipStream_t st) -> int {
+    XMD_CHECK(hipEventRecord(e, R.s0));
+    XMD_CHECK(hipStreamWaitEvent(st, e, 0));
+    return 0;
+  };
+  auto real = [&](hipStream_t st) -> int {
+    return rec(8, st) || launch_pair_ewald_real(p, st) || rec(9, st) ? -1 : 0;
+  };
+  auto bead = [&](hipStream_t st) -> int {
+    if (rec(6, st)) return -1;
+    if (d->massive) {
+      if (launch_step_bead_forces(item_of(sp), st)) return -1;
+    } else {
+      if (launch_reset_force(d, st)) return -1;
+      if (sp.trap && launch_trap_force(d, md_trap_frequency_x, md_trap_center_x, (double)p->P, st)) return -1;
+      if (launch_ring_springs(p, sp.image, sp.L, st)) return -1;
+    }
+    return rec(7, st);
+  };
+  auto kspace = [&](hipStream_t st) -> int {
+    return rec(10, st) || launch_pair_kspace(p, st) || rec(11, st) ? -1 : 0;
+  };
+  const bool s2 = pairs_s2 || o == Order::Beside || o == Order::Late;
+  if (s2 && o != Order::Late && fork(R.fork2, R.s2)) return -1;
+  if (o == Order::Beside && real(R.s2)) return -1;
+  if (o == Order::KSpace && (bead(R.s2) || kspace(R.s2))) return -1;
   if (rec(2, R.s0) || (serial ? launch_enk(p, sp.image, R.s0) : launch_enk_prep(p, sp.image, R.s0)) ||
       rec(3, R.s0))
     return -1;
-  if (!serial) {
-    XMD_CHECK(hipEventRecord(R.fork, R.s0));
-    XMD_CHECK(hipStreamWaitEvent(R.s1, R.fork, 0));
-  }
+  if (fork_solve && fork(R.fork, R.s1)) return -1;
   if (rec(4, sx) || (serial ? launch_recursion(p, true, true, sx, ev ? ev[16] : nullptr) : launch_recursion_solve(p, sx)) ||
       rec(5, sx))
     return -1;
-  // overlapped: the end-bead exchange forces follow the recursions on s1
-  // into a side buffer, added into F after the join
-  if (!serial && launch_exchange_force(p, sp.image, R.s1, true)) return -1;
-  if (!serial) XMD_CHECK(hipEventRecord(R.join, R.s1));
+  if (!serial && (rec(12, sx) || launch_exchange_force(p, sp.image, sx, true) || rec(13, sx))) return -1;
+  if (fork_solve) XMD_CHECK(hipEventRecord(R.join, R.s1));
+  if (o == Order::Late && (fork(R.fork2, R.s2) || real(R.s2))) return -1;
   // bead-local and pair forces
-  if (rec(6, R.s0)) return -1;
-  if (d->massive) {
-    if (launch_step_bead_forces(item_of(sp), R.s0)) return -1;
+  if (o == Order::KSpace) {
+    if (real(R.s0)) return -1;
+  } else if (bead(sb)) {
+    return -1;
+  } else if (ewald) {
+    if ((o == Order::Pairs && real(sb)) || kspace(sb)) return -1;
   } else {
-    if (launch_reset_force(d, R.s0)) return -1;
-    if (sp.trap && launch_trap_force(d, md_trap_frequency_x, md_trap_center_x, (double)p->P, R.s0)) return -1;
-    if (launch_ring_springs(p, sp.image, sp.L, R.s0)) return -1;
+    if (rec(8, sb) || (kind >= 0 && launch_pair_real(p, kind, sb)) || rec(9, sb)) return -1;
+    if (rec(10, sb) || (kind >= 0 && pair_has_recip(kind) && launch_pair_recip(p, kind, sb)) || rec(11, sb)) return -1;
   }
-  if (rec(7, R.s0)) return -1;
-  if (kfork && launch_pair_kspace(p, R.s0)) return -1;
-  if (kfork) {
-    if (rec(8, R.s0) || rec(9, R.s0) || rec(10, R.s0) || rec(11, R.s0)) return -1;
-  } else if (sp.pair_kind >= 0) {
-    if (rec(8, R.s0) || launch_pair_real(p, sp.pair_kind, R.s0) || rec(9, R.s0)) return -1;
-    if (pair_has_recip(sp.pair_kind)) {
-      if (rec(10, R.s0) || launch_pair_recip(p, sp.pair_kind, R.s0) || rec(11, R.s0)) return -1;
-    } else if (rec(10, R.s0) || rec(11, R.s0)) {
-      return -1;
-    }
-  } else if (rec(8, R.s0) || rec(9, R.s0) || rec(10, R.s0) || rec(11, R.s0)) {
-    return -1;
+  if (serial) return rec(12, R.s0) || launch_exchange_force(p, sp.image, R.s0, false) || rec(13, R.s0) ? -1 : 0;
+  if (fork_solve) XMD_CHECK(hipStreamWaitEvent(R.s0, R.join, 0));
+  if (s2) {
+    XMD_CHECK(hipEventRecord(R.join2, R.s2));
+    XMD_CHECK(hipStreamWaitEvent(R.s0, R.join2, 0));
   }
-  if (!serial) {
-    XMD_CHECK(hipStreamWaitEvent(R.s0, R.join, 0));
-    if (kfork) {
-      // one kernel adds the real-space, reciprocal and exchange forces
-      XMD_CHECK(hipStreamWaitEvent(R.s0, R.join2, 0));
-      if (fused && d->massive) {
-        if (rec(12, R.s0) || force_sums(p, p->Fx, fused) || rec(13, R.s0)) return -1;
-      } else if (rec(12, R.s0) || launch_combine_forces(p, p->Fx, R.s0) || rec(13, R.s0)) {
-        return -1;
-      }
-    } else if (rec(12, R.s0) || launch_add_exchange_force(p, R.s0) || rec(13, R.s0)) {
-      return -1;
-    }
-  } else if (rec(12, R.s0) || launch_exchange_force(p, sp.image, R.s0, false) || rec(13, R.s0)) {
-    return -1;
-  }
-  return 0;
+  if (!ewald) return launch_add_exchange_force(p, R.s0);
+  // one kernel adds the real-space, reciprocal and exchange forces
+  return fused && d->massive ? force_sums(p, p->Fx, fused) : launch_combine_forces(p, p->Fx, R.s0);
 }
 
 // head: NHC half 1 starts the step (false: the previous step's chained tail

@@ -194,17 +194,16 @@ unsigned pair_alloc_epoch();
 // Real-space Ewald launch choice autotuning (pair_forces.hip): with it on,
 // tune the object's (N, P) bucket before first use (never during capture).
 int autotune_if_needed(DevPimd *p, int kind);
-// Ewald forces in parts: launch_pair_ewald_fork forks s2 from st (through
-// `fork`), queues there the real-space tile kernel (per-tile partial forces;
-// with the learned stand-in in use, then its kernels) and records `join`;
-// launch_pair_kspace, called later in st's order, queues the phase tables,
-// structure factors and reciprocal forces (into a side buffer) on st.  All of
-// these read positions only.  After `join` (and the exchange branch)
+// Ewald forces in parts, where pair_ewald_tab says so (Ewald with the table
+// kernels): launch_pair_ewald_real queues the real-space tile kernel (per-tile
+// partial forces; with the learned stand-in in use, then its kernels),
+// launch_pair_kspace the phase tables, structure factors and reciprocal forces
+// (into a side buffer; nothing with the stand-in).  Both read positions only
+// and may run beside each other and the exchange branch.  After all of them
 // launch_combine_forces adds the real-space, reciprocal and, when Fx is
-// given, exchange end-bead forces into F in the order of the unsplit
-// kernels.  The fork returns 1 when it applies (Ewald with the table
-// kernels), 0 when nothing was launched (use launch_pair_force), -1 on error.
-int launch_pair_ewald_fork(DevPimd *p, int kind, hipStream_t st, hipStream_t s2, hipEvent_t fork, hipEvent_t join);
+// given, exchange end-bead forces into F in the order of the unsplit kernels.
+bool pair_ewald_tab(DevPimd *p, int kind);
+int launch_pair_ewald_real(DevPimd *p, hipStream_t st);
 int launch_pair_kspace(DevPimd *p, hipStream_t st);
 int launch_combine_forces(DevPimd *p, const double *Fx, hipStream_t st);
 // The parts launch_combine_forces adds, for a fused consumer of F.
