@@ -1515,7 +1515,7 @@ static int near_ok(const PairParams &pp) {
 }
 
 template <int MODE, bool ENERGY>
-static int launch_pair_mode(DevPimd *p, const PairParams &pp, hipStream_t st, double *esum) {
+static int launch_pair_mode(DevPimd *p, const PairParams &pp, hipStream_t st, double *esum, bool reduce = true) {
   DevSim *d = p->ds;
   if (ensure_tiles(p)) return -1;
   TileBufs &B = pair_bufs(p)->tb;
@@ -1529,6 +1529,7 @@ static int launch_pair_mode(DevPimd *p, const PairParams &pp, hipStream_t st, do
                        B.Epart, B.tiles, p->N, d->nb, B.T, B.ntp, pp);
   XMD_CHECK(hipGetLastError());
   if (ENERGY) return device_sum(B.Epart, items, esum);
+  if (!reduce) return 0;
   const int n3 = 3 * d->nb;
   hipLaunchKernelGGL(k_reduce_tiles, dim3((n3 + 255) / 256), dim3(256), 0, st, B.Fpart, d->F, n3, B.T, pp.P);
   XMD_CHECK(hipGetLastError());
@@ -1820,17 +1821,17 @@ static int launch_recip(DevPimd *p, const PairParams &pp, int cube_n, double gma
   return force ? launch_recip_force(p, pp, K, st) : 0;
 }
 
-int launch_pair_real(DevPimd *p, int kind, hipStream_t st) {
+int launch_pair_real(DevPimd *p, int kind, hipStream_t st, bool reduce) {
   PairParams pp = make_params(p);
   switch (kind) {
     case PK_GAUSS:
-      return launch_pair_mode<PK_GAUSS, false>(p, pp, st, nullptr);
+      return launch_pair_mode<PK_GAUSS, false>(p, pp, st, nullptr, reduce);
     case PK_PGAUSS:
-      return launch_pair_mode<PK_PGAUSS, false>(p, pp, st, nullptr);
+      return launch_pair_mode<PK_PGAUSS, false>(p, pp, st, nullptr, reduce);
     case PK_LJ:
-      return launch_pair_mode<PK_LJ, false>(p, pp, st, nullptr);
+      return launch_pair_mode<PK_LJ, false>(p, pp, st, nullptr, reduce);
     case PK_HE:
-      return launch_pair_mode<PK_HE, false>(p, pp, st, nullptr);
+      return launch_pair_mode<PK_HE, false>(p, pp, st, nullptr, reduce);
     case PK_EWALD:
     case PK_EWALD_R:
     case PK_EWALD_NI:
@@ -1841,11 +1842,11 @@ int launch_pair_real(DevPimd *p, int kind, hipStream_t st) {
       if (kind == PK_EWALD) {
         EwaldPlan pl;
         pp = ewald_params(p, pl);
-        if (near_ok(pp)) return launch_ewald_real_tab(p, pp, st);
-        return launch_pair_mode<PK_EWALD, false>(p, pp, st, nullptr);
+        if (near_ok(pp)) return launch_ewald_real_tab(p, pp, st, reduce);
+        return launch_pair_mode<PK_EWALD, false>(p, pp, st, nullptr, reduce);
       }
-      if (kind == PK_EWALD_R) return launch_pair_mode<PK_EWALD_R, false>(p, pp, st, nullptr);
-      return launch_pair_mode<PK_EWALD_NI, false>(p, pp, st, nullptr);
+      if (kind == PK_EWALD_R) return launch_pair_mode<PK_EWALD_R, false>(p, pp, st, nullptr, reduce);
+      return launch_pair_mode<PK_EWALD_NI, false>(p, pp, st, nullptr, reduce);
     default:
       return -1;
   }
@@ -2003,11 +2004,11 @@ __global__ __launch_bounds__(256) void k_combine_forces(double *__restrict__ F, 
   F[k] = combined_force(F, c, n3, k);
 }
 
-int force_sums(DevPimd *p, const double *Fx, ForceSums *out) {
+int force_sums(DevPimd *p, const double *Fx, bool recip, ForceSums *out) {
   TileBufs &B = pair_bufs(p)->tb;
   ForceSums c;
   c.Fpart = B.Fpart;
-  c.Frec = B.Frec;
+  c.Frec = recip ? B.Frec : nullptr;
   c.Fx = Fx;
   c.T = B.T;
   c.N = p->N;
@@ -2018,7 +2019,7 @@ int force_sums(DevPimd *p, const double *Fx, ForceSums *out) {
 
 int launch_combine_forces(DevPimd *p, const double *Fx, hipStream_t st) {
   ForceSums c;
-  if (force_sums(p, Fx, &c)) return -1;
+  if (force_sums(p, Fx, true, &c)) return -1;
   const int n3 = 3 * p->ds->nb;
   hipLaunchKernelGGL(k_combine_forces, dim3((n3 + 255) / 256), dim3(256), 0, st, p->ds->F, c, n3);
   XMD_CHECK(hipGetLastError());

@@ -130,6 +130,10 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   const int kind = sp.pair_kind;
   const bool ewald = !serial && kind >= 0 && pair_ewald_tab(p, kind);
   const Order o = serial ? Order::Serial : force_order(sp, ewald);
+  // pair forces without a reciprocal part: with massive thermostats their tile
+  // sums and the exchange forces are left for NHC half 2 as well, two launches
+  // and a pass over F fewer
+  const bool parts = !serial && fused && d->massive && kind >= 0 && (ewald || !pair_has_recip(kind));
   const bool pairs_s2 = o == Order::Pairs || o == Order::KSpace;  // bead-local and pair forces on s2
   const bool fork_solve = o != Order::Serial && o != Order::Pairs;
   const hipStream_t sx = fork_solve ? R.s1 : R.s0, sb = pairs_s2 ? R.s2 : R.s0;
@@ -181,7 +185,7 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   } else if (ewald) {
     if ((o == Order::Pairs && real(sb)) || kspace(sb)) return -1;
   } else {
-    if (rec(8, sb) || (kind >= 0 && launch_pair_real(p, kind, sb)) || rec(9, sb)) return -1;
+    if (rec(8, sb) || (kind >= 0 && launch_pair_real(p, kind, sb, !parts)) || rec(9, sb)) return -1;
     if (rec(10, sb) || (kind >= 0 && pair_has_recip(kind) && launch_pair_recip(p, kind, sb)) || rec(11, sb)) return -1;
   }
   if (serial) return rec(12, R.s0) || launch_exchange_force(p, sp.image, R.s0, false) || rec(13, R.s0) ? -1 : 0;
@@ -190,9 +194,9 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
     XMD_CHECK(hipEventRecord(R.join2, R.s2));
     XMD_CHECK(hipStreamWaitEvent(R.s0, R.join2, 0));
   }
-  if (!ewald) return launch_add_exchange_force(p, R.s0);
+  if (parts) return force_sums(p, p->Fx, ewald, fused);
   // one kernel adds the real-space, reciprocal and exchange forces
-  return fused && d->massive ? force_sums(p, p->Fx, fused) : launch_combine_forces(p, p->Fx, R.s0);
+  return ewald ? launch_combine_forces(p, p->Fx, R.s0) : launch_add_exchange_force(p, R.s0);
 }
 
 // head: NHC half 1 starts the step (false: the previous step's chained tail

@@ -161,7 +161,7 @@ int pair_kind_of(md_pair_force_t_x pf);
 int pair_energy_kind_of(md_pair_energy_t_x pe);
 int launch_pair_force(DevPimd *p, int kind, hipStream_t st);
 // Pair and exchange forces computed in parts, summed into F: the real-space
-// tile sums over P, then the reciprocal forces, then (Fx given) the stored
+// tile sums over P, then (Frec given) the reciprocal forces, then (Fx given) the stored
 // exchange forces of the end beads (slices P-1 and 0).  Fpart == nullptr:
 // nothing to add.
 struct ForceSums {
@@ -175,7 +175,7 @@ __device__ __forceinline__ double combined_force(const double *__restrict__ F, c
   double s = 0;
   for (int q = 0; q < c.T; ++q) s += c.Fpart[(size_t)q * n3 + k];
   double f = F[k] + s / (double)c.P;
-  f += c.Frec[k];
+  if (c.Frec) f += c.Frec[k];
   if (c.Fx) {
     const int nb = c.N * c.P, d = k / nb, i = k - d * nb;
     if (i >= (c.P - 1) * c.N) f += c.Fx[d * c.N + (i - (c.P - 1) * c.N)];
@@ -207,8 +207,10 @@ int launch_pair_ewald_real(DevPimd *p, hipStream_t st);
 int launch_pair_kspace(DevPimd *p, hipStream_t st);
 int launch_combine_forces(DevPimd *p, const double *Fx, hipStream_t st);
 // The parts launch_combine_forces adds, for a fused consumer of F.
-int force_sums(DevPimd *p, const double *Fx, ForceSums *out);
-int launch_pair_real(DevPimd *p, int kind, hipStream_t st);
+// recip: the reciprocal forces are among them.
+int force_sums(DevPimd *p, const double *Fx, bool recip, ForceSums *out);
+// reduce false: the tile sums stay in their buffer (force_sums).
+int launch_pair_real(DevPimd *p, int kind, hipStream_t st, bool reduce = true);
 // Exact reciprocal-space Ewald terms of the step's plan (alpha, k set of
 // md_coulomb_3d_ewald_force_x): forces (accelerations / P, [3][nb]) into Frec
 // and each bead's share of its slice's reciprocal energy into Erec [nb];
