@@ -997,6 +997,155 @@ __device__ __forceinline__ void recip_force_tile(FrcLds<NZT> &sh, int slice, int
 // Workgroups per slice of the reciprocal force kernels (64 beads each).
 __host__ __device__ inline int frc_tiles(int N) { return (N + 63) / 64; }
 
+// Forces on the 16 beads [b0, b0 + 16) of one slice, the column tiles dealt
+// to the four waves (tile 4 i + w to wave w): for grids too small to fill the
+// device with 64 beads per workgroup, whose waves each walk every tile, and
+// for slices of few beads, where most of those waves hold none.  A P, Q tile
+// is used by one wave here, each entry by one lane, so it goes from memory
+// straight to registers, a round ahead.  The products of a round's four tiles
+// are exchanged through LDS and wave w adds them, tile after tile, for the
+// beads 4 w .. 4 w + 3: every sum has the order, and the bits, of
+// recip_force_tile.
+template <int NZT>
+struct FrcSplitLds {
+  static constexpr int ZP = 16 * NZT, RX = 8 * NZT;
+  double2 rx[16 * RX], ry[16 * RX];  // phase rows, as in FrcLds
+  double u[4][5][4][64];             // [tile of the round][g, ar, ai, vr, vi][D register][lane]
+  int2 cl[4][16];                    // (m_x, m_y) of the round's columns
+};
+
+template <int NZT>
+__device__ __forceinline__ void recip_force_split(FrcSplitLds<NZT> &sh, int slice, int b0,
+                                                  const double2 *__restrict__ tx, const double2 *__restrict__ ty,
+                                                  const double2 *__restrict__ tz, const int2 *__restrict__ cols,
+                                                  int ncolp, const double2 *__restrict__ PQ,
+                                                  const double *__restrict__ Mass, double *__restrict__ F, int N,
+                                                  int nb, double L0, double L1, double L2, double Pd,
+                                                  double *__restrict__ Frec) {
+  using S = FrcSplitLds<NZT>;
+  constexpr int ZP = S::ZP, RX = S::RX, MH = RX, KS = MH / 4;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int nloc = min(16, N - b0);
+  {
+    const double2 *gx = tx + (size_t)(slice * N + b0) * RX;
+    const double2 *gy = ty + (size_t)(slice * N + b0) * RX;
+    for (int e = tid; e < 16 * RX; e += 256) {
+      const bool ok = e < nloc * RX;
+      sh.rx[e] = ok ? gx[e] : make_double2(0.0, 0.0);
+      sh.ry[e] = ok ? gy[e] : make_double2(0.0, 0.0);
+    }
+  }
+  const int zl = lane >> 4, cq = lane & 15;
+  const bool aok = cq < nloc;
+  const double2 *pza = tz + (size_t)(slice * N + b0 + (aok ? cq : 0)) * MH + zl;
+  double zc[KS], zn[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    const double2 z = aok ? pza[4 * k] : make_double2(0.0, 0.0);
+    zc[k] = z.x;
+    zn[k] = z.y;
+  }
+  const int nct = ncolp / 16;
+  // operands P_m, Q_m of column cq of tile ct, m = 4 k + zl
+  const double2 *Ws = PQ + (size_t)slice * ncolp * ZP + cq * ZP + 2 * zl;
+  double2 pq[2 * KS];
+  int2 kr, cl;
+  auto fetch = [&](int ct) {
+    const int c = min(ct, nct - 1);  // past the last tile: unused
+    const double2 *w = Ws + (size_t)c * 16 * ZP;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      pq[2 * k] = w[8 * k];
+      pq[2 * k + 1] = w[8 * k + 1];
+    }
+    kr = cols[ncolp + c];
+    cl = cols[c * 16 + cq];
+  };
+  fetch(wv);
+  double fx = 0, fy = 0, fz = 0;
+  for (int ct0 = 0; ct0 < nct; ct0 += 4) {
+    __syncthreads();
+    if (ct0 + wv < nct) {
+      v4d ur4 = {0, 0, 0, 0}, ui4 = ur4, vr4 = ur4, vi4 = ur4;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        if (k < kr.x || k > kr.y) continue;
+        const double2 Pm = pq[2 * k], Qm = pq[2 * k + 1];
+        const double m = (double)(4 * k + zl);
+        ur4 = mfma4(zc[k], Pm.x, ur4);
+        ui4 = mfma4(zc[k], Pm.y, ui4);
+        vr4 = mfma4(zc[k], m * Qm.x, vr4);
+        vi4 = mfma4(zc[k], m * Qm.y, vi4);
+        ur4 = mfma4(zn[k], -Qm.y, ur4);
+        ui4 = mfma4(zn[k], Qm.x, ui4);
+        vr4 = mfma4(zn[k], -m * Pm.y, vr4);
+        vi4 = mfma4(zn[k], m * Pm.x, vi4);
+      }
+      const int2 c = cl;
+      fetch(ct0 + 4 + wv);
+      if (zl == 0) sh.cl[wv][cq] = c;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int bl = 4 * r + zl;
+        const double2 ex = sh.rx[bl * RX + c.x];
+        double2 ey = sh.ry[bl * RX + (c.y < 0 ? -c.y : c.y)];
+        if (c.y < 0) ey.y = -ey.y;
+        const double ur = ur4[r], ui = ui4[r];
+        const double ar = ex.x * ey.x - ex.y * ey.y, ai = ex.x * ey.y + ex.y * ey.x;
+        sh.u[wv][0][r][lane] = fma(ar, ui, ai * ur);
+        sh.u[wv][1][r][lane] = ar;
+        sh.u[wv][2][r][lane] = ai;
+        sh.u[wv][3][r][lane] = vr4[r];
+        sh.u[wv][4][r][lane] = vi4[r];
+      }
+    }
+    __syncthreads();
+    for (int t = 0; t < min(4, nct - ct0); ++t) {
+      const int2 c = sh.cl[t][cq];
+      const double g = sh.u[t][0][wv][lane], ar = sh.u[t][1][wv][lane], ai = sh.u[t][2][wv][lane];
+      const double vr = sh.u[t][3][wv][lane], vi = sh.u[t][4][wv][lane];
+      fx = fma((double)c.x, g, fx);
+      fy = fma((double)c.y, g, fy);
+      fz = fma(ar, vi, fma(ai, vr, fz));
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    fx += __shfl_xor(fx, o, 64);
+    fy += __shfl_xor(fy, o, 64);
+    fz += __shfl_xor(fz, o, 64);
+  }
+  const int bl = 4 * wv + zl;
+  if (cq == 0 && bl < nloc) {
+    const int s = slice * N + b0 + bl;
+    const double m = Mass[s];
+    if (Frec) {
+      Frec[s] = fx / L0 / m / Pd;
+      Frec[nb + s] = fy / L1 / m / Pd;
+      Frec[2 * nb + s] = fz / L2 / m / Pd;
+    } else {
+      F[s] += fx / L0 / m / Pd;
+      F[nb + s] += fy / L1 / m / Pd;
+      F[2 * nb + s] += fz / L2 / m / Pd;
+    }
+  }
+}
+
+// Workgroups per slice with 16 beads each.
+__host__ __device__ inline int frc_split_tiles(int N) { return (N + 15) / 16; }
+
+template <int NZT>
+__global__ __launch_bounds__(256) void k_recip_force_split(
+    const double2 *__restrict__ tx, const double2 *__restrict__ ty, const double2 *__restrict__ tz,
+    const int2 *__restrict__ cols, int ncolp, int MZ, const double2 *__restrict__ W,
+    const double *__restrict__ Mass, double *__restrict__ F, int N, int nb, int P, double L0, double L1, double L2,
+    double Pd, double *__restrict__ Frec) {
+  __shared__ FrcSplitLds<NZT> sh;
+  int slice, bt;
+  xcd_tile(blockIdx.x, frc_split_tiles(N), P, slice, bt);
+  recip_force_split<NZT>(sh, slice, bt * 16, tx, ty, tz, cols, ncolp, W, Mass, F, N, nb, L0, L1, L2, Pd, Frec);
+}
+
 template <int NZT, bool EN = false>
 __device__ __forceinline__ void k_recip_force_mfma_body(int bx,
     const double2 *__restrict__ tx, const double2 *__restrict__ ty, const double2 *__restrict__ tz,
@@ -1772,6 +1921,10 @@ static void (*const k_frc_of[4])(const double2 *, const double2 *, const double2
                                  const double2 *, const double *, double *, int, int, int, double, double, double,
                                  double, double *) = {k_recip_force_mfma<1>, k_recip_force_mfma<2>, k_recip_force_mfma<3>,
                                             k_recip_force_mfma<4>};
+static void (*const k_frs_of[4])(const double2 *, const double2 *, const double2 *, const int2 *, int, int,
+                                 const double2 *, const double *, double *, int, int, int, double, double, double,
+                                 double, double *) = {k_recip_force_split<1>, k_recip_force_split<2>, k_recip_force_split<3>,
+                                            k_recip_force_split<4>};
 
 // Phase tables of every slice (reads X only) for the k set of pp.
 static int launch_recip_phase(DevPimd *p, const PairParams &pp, int cube_n, double gmax2, hipStream_t st,
@@ -1806,8 +1959,14 @@ static int launch_recip_sk(DevPimd *p, const PairParams &pp, int cube_n, double 
 static int launch_recip_force(DevPimd *p, const PairParams &pp, const KSpace *K, hipStream_t st,
                               double *Frec = nullptr) {
   DevSim *d = p->ds;
-  hipLaunchKernelGGL(k_frc_of[K->ZP / 16 - 1], dim3(frc_tiles(p->N) * p->P), dim3(256), 0, st, K->tx, K->ty, K->tz,
-                     K->cols, K->ncolp, K->MZ, K->W, d->M, d->F, p->N, d->nb, p->P, pp.L[0], pp.L[1], pp.L[2], pp.P,
+  // fewer workgroups of 64 beads than compute units: 16 beads each, column
+  // tiles dealt to the waves (stage of phases, structure factors and forces,
+  // us, without -> with: N=16 P=32 34 -> 25, N=128 P=64 45 -> 36, N=333 P=27
+  // 48 -> 45.5; N=512 P=32, one workgroup a unit, 51.5 -> 61.5)
+  const bool split = frc_tiles(p->N) * p->P < 256;
+  hipLaunchKernelGGL((split ? k_frs_of : k_frc_of)[K->ZP / 16 - 1],
+                     dim3((split ? frc_split_tiles(p->N) : frc_tiles(p->N)) * p->P), dim3(256), 0, st, K->tx,
+                     K->ty, K->tz, K->cols, K->ncolp, K->MZ, K->W, d->M, d->F, p->N, d->nb, p->P, pp.L[0], pp.L[1], pp.L[2], pp.P,
                      Frec);
   XMD_CHECK(hipGetLastError());
   return 0;

@@ -97,11 +97,12 @@ static Lane main_lane() {
 // exchange cycles t and uniform ones u):
 //   Pairs   the pair branch on s2 and the chain on s0, both from NHC on:
 //           no pair kernel fills the device (trap N=8 P=8 45 -> 34,
-//           N=256 P=64 t 92 -> 88, u 84 -> 65; Ewald N=256 P=32 t 109 -> 100,
-//           u 99 -> 97, N=512 P=32 t 160 -> 147, u 120 -> 122)
-//   KSpace  Ewald, smaller still: bead-local and reciprocal forces on s2 from
-//           NHC on, the real space on s0 after the set-up, beside the solves
-//           on s1 (N=16 P=32 78 -> 62, N=128 P=64 t 98 -> 91, u 98 -> 90)
+//           N=256 P=64 t 92 -> 88, u 84 -> 65; Ewald N=333 P=27 t 130 -> 118,
+//           N=512 P=32 t 160 -> 147, u 120 -> 122)
+//   Wide    Ewald, smaller still: likewise, the real space apart on s1, in
+//           front of the kernels that follow one another (N=16 P=32 67 -> 51
+//           against Pairs, N=128 P=64 t 89 -> 87, u 88 -> 76, N=256 P=32
+//           t 98 -> 102, u 90 -> 80, N=333 P=27 t 118 -> 122)
 //   Beside  Ewald, the real space on s2 from NHC on, bead-local and reciprocal
 //           forces on s0 after the set-up, the solves on s1 (N=1024 P=32
 //           t 273, u 188; 266 and 201 with Late)
@@ -110,12 +111,12 @@ static Lane main_lane() {
 //           N=2001 P=24 t 600 -> 491, u 405 -> 384)
 //   After   no Ewald: pair branch on s0 after the set-up, solves on s1 (trap
 //           N=600 P=64 t 164, u 146; 214 and 161 with Pairs)
-enum class Order { Serial, Pairs, KSpace, Beside, Late, After };
+enum class Order { Serial, Pairs, Wide, Beside, Late, After };
 
 static Order force_order(const StepPlan &sp, bool ewald) {
   const double w = (double)sp.p->N * sp.p->N * sp.p->P;
   if (ewald && sp.p->sur_mode) return Order::Beside;
-  if (ewald) return w < 1.5e6 ? Order::KSpace : w < 1.2e7 ? Order::Pairs : w < 5e7 ? Order::Beside : Order::Late;
+  if (ewald) return w < 2.5e6 ? Order::Wide : w < 1.2e7 ? Order::Pairs : w < 5e7 ? Order::Beside : Order::Late;
   return w < 8e6 ? Order::Pairs : Order::After;
 }
 
@@ -134,8 +135,8 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   // sums and the exchange forces are left for NHC half 2 as well, two launches
   // and a pass over F fewer
   const bool parts = !serial && fused && d->massive && kind >= 0 && (ewald || !pair_has_recip(kind));
-  const bool pairs_s2 = o == Order::Pairs || o == Order::KSpace;  // bead-local and pair forces on s2
-  const bool fork_solve = o != Order::Serial && o != Order::Pairs;
+  const bool pairs_s2 = o == Order::Pairs || o == Order::Wide;  // bead-local and pair forces on s2
+  const bool fork_solve = o == Order::Beside || o == Order::Late || o == Order::After;
   const hipStream_t sx = fork_solve ? R.s1 : R.s0, sb = pairs_s2 ? R.s2 : R.s0;
   auto rec = [&](int k, hipStream_t st) -> int {
     if (ev) XMD_CHECK(hipEventRecord(ev[k], st));
@@ -165,8 +166,8 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   };
   const bool s2 = pairs_s2 || o == Order::Beside || o == Order::Late;
   if (s2 && o != Order::Late && fork(R.fork2, R.s2)) return -1;
+  if (o == Order::Wide) XMD_CHECK(hipStreamWaitEvent(R.s1, R.fork2, 0));
   if (o == Order::Beside && real(R.s2)) return -1;
-  if (o == Order::KSpace && (bead(R.s2) || kspace(R.s2))) return -1;
   if (rec(2, R.s0) || (serial ? launch_enk(p, sp.image, R.s0) : launch_enk_prep(p, sp.image, R.s0)) ||
       rec(3, R.s0))
     return -1;
@@ -178,22 +179,23 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   if (fork_solve) XMD_CHECK(hipEventRecord(R.join, R.s1));
   if (o == Order::Late && (fork(R.fork2, R.s2) || real(R.s2))) return -1;
   // bead-local and pair forces
-  if (o == Order::KSpace) {
-    if (real(R.s0)) return -1;
-  } else if (bead(sb)) {
-    return -1;
-  } else if (ewald) {
+  if (bead(sb)) return -1;
+  if (ewald) {
     if ((o == Order::Pairs && real(sb)) || kspace(sb)) return -1;
+    if (o == Order::Wide) {
+      if (real(R.s1)) return -1;
+      XMD_CHECK(hipEventRecord(R.join, R.s1));
+    }
   } else {
     if (rec(8, sb) || (kind >= 0 && launch_pair_real(p, kind, sb, !parts)) || rec(9, sb)) return -1;
     if (rec(10, sb) || (kind >= 0 && pair_has_recip(kind) && launch_pair_recip(p, kind, sb)) || rec(11, sb)) return -1;
   }
   if (serial) return rec(12, R.s0) || launch_exchange_force(p, sp.image, R.s0, false) || rec(13, R.s0) ? -1 : 0;
-  if (fork_solve) XMD_CHECK(hipStreamWaitEvent(R.s0, R.join, 0));
   if (s2) {
     XMD_CHECK(hipEventRecord(R.join2, R.s2));
     XMD_CHECK(hipStreamWaitEvent(R.s0, R.join2, 0));
   }
+  if (fork_solve || o == Order::Wide) XMD_CHECK(hipStreamWaitEvent(R.s0, R.join, 0));
   if (parts) return force_sums(p, p->Fx, ewald, fused);
   // one kernel adds the real-space, reciprocal and exchange forces
   return ewald ? launch_combine_forces(p, p->Fx, R.s0) : launch_add_exchange_force(p, R.s0);
