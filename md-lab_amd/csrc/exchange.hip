@@ -1605,7 +1605,7 @@ __global__ __launch_bounds__(SIGN_WG) void k_vi_sign(RecArgs a, const double *__
 // decomposition (virtual block index = global block - start[replica]).
 struct ExRep {
   const double *X, *M;
-  double *F;
+  double *F, *Fx;
   int N, P;
   double om;
   Geo g;
@@ -1662,7 +1662,15 @@ __global__ __launch_bounds__(256) void kb_exch_force(const ExRep *__restrict__ r
                                                      int nrep) {
   const int r = batch_rep(start, nrep, blockIdx.x);
   const ExRep &R = reps[r];
-  exch_force_body(blockIdx.x - start[r], R.X, R.M, R.F, R.N, R.P, R.om, R.g, R.a);
+  exch_force_body(blockIdx.x - start[r], R.X, R.M, R.F, R.N, R.P, R.om, R.g, R.a, R.Fx);
+}
+
+// *err = 1 when any replica's recursion has an error to report, else 0.
+__global__ __launch_bounds__(256) void kb_rec_error(const ExRep *__restrict__ reps, int nrep, int *__restrict__ err) {
+  int e = 0;
+  for (int r = threadIdx.x; r < nrep; r += 256) e |= reps[r].a.sync[4 * reps[r].a.nblk] != 0;
+  e = __syncthreads_or(e);
+  if (threadIdx.x == 0) *err = e != 0;
 }
 
 // ------------------------------------------------------------ launchers
@@ -1993,6 +2001,7 @@ ExchBatch *exch_batch_create(const std::vector<BatchItem> &items) {
     R.X = d->X;
     R.M = d->M;
     R.F = d->F;
+    R.Fx = p->Fx;
     R.N = p->N;
     R.P = p->P;
     R.om = p->host->omegaP;
@@ -2071,10 +2080,19 @@ int exch_batch_force(ExchBatch *b, hipStream_t st) {
   return 0;
 }
 
+// Waits for s0 and reports the replicas' recursion errors: their error words
+// are gathered into one pinned word by a kernel behind the last step (a copy
+// per replica took 8 us each), and read one by one only when one is set.
 int exch_batch_status(ExchBatch *b) {
+  int *err = (int *)host_scratch(1);
+  if (!err) return -1;
+  hipLaunchKernelGGL(kb_rec_error, dim3(1), dim3(256), 0, rt().s0, (const ExRep *)b->chain.reps, b->nrep, err);
+  XMD_CHECK(hipGetLastError());
+  XMD_CHECK(hipStreamSynchronize(rt().s0));
   int rc = 0;
-  for (DevPimd *p : b->ps)
-    if (recursion_status(p)) rc = -1;
+  if (*err)
+    for (DevPimd *p : b->ps)
+      if (recursion_status(p)) rc = -1;
   return rc;
 }
 

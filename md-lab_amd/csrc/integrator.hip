@@ -322,7 +322,7 @@ struct BeadRep {
   double T, h;
   int pbc, image, trap;
   double L[3], w, c[3], om;
-  ForceSums cs;  // half 2: parts added into F first (cs.Fpart set)
+  ForceSums cs;  // half 2: parts added into F first (Fpart or Fx set)
 };
 
 // NHC half-kick (+ drift for HALF 1), then the box wrap after HALF 1, for
@@ -332,7 +332,7 @@ struct BeadRep {
 template <int HALF>
 __device__ __forceinline__ void nhc_wrap_body(const BeadRep &R, int e) {
   double f;
-  if (HALF != 1 && R.cs.Fpart) {
+  if (HALF != 1 && (R.cs.Fpart || R.cs.Fx)) {
     f = combined_force(R.F, R.cs, 3 * R.nb, e);
     R.F[e] = f;
   } else {
@@ -469,15 +469,17 @@ struct BeadBatch {
   BatchTable t;
 };
 
-BeadBatch *bead_batch_create(const std::vector<BatchItem> &items) {
+BeadBatch *bead_batch_create(const std::vector<BatchItem> &items, const std::vector<ForceSums> &sums) {
   std::vector<BeadRep> reps;
   std::vector<int> blocks;
-  for (const BatchItem &it : items) {
+  for (size_t i = 0; i < items.size(); ++i) {
+    const BatchItem &it = items[i];
     if (!it.p->ds->massive) {
       fprintf(stderr, "xmd: batched steps need massive thermostats (one chain per degree of freedom)\n");
       return nullptr;
     }
     reps.push_back(bead_rep(it));
+    reps.back().cs = sums[i];
     blocks.push_back((3 * it.p->ds->nb + 255) / 256);
   }
   BeadBatch *b = new BeadBatch();

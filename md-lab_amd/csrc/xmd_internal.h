@@ -162,8 +162,7 @@ int pair_energy_kind_of(md_pair_energy_t_x pe);
 int launch_pair_force(DevPimd *p, int kind, hipStream_t st);
 // Pair and exchange forces computed in parts, summed into F: the real-space
 // tile sums over P, then (Frec given) the reciprocal forces, then (Fx given) the stored
-// exchange forces of the end beads (slices P-1 and 0).  Fpart == nullptr:
-// nothing to add.
+// exchange forces of the end beads (slices P-1 and 0).
 struct ForceSums {
   const double *Fpart = nullptr, *Frec = nullptr, *Fx = nullptr;
   int T = 0, N = 0, P = 0;
@@ -172,9 +171,12 @@ struct ForceSums {
 // F[k] plus the parts, in the order above (so the rounding is that of the
 // unsplit kernels: k_reduce_tiles, k_recip_force_mfma, k_add_exch in turn).
 __device__ __forceinline__ double combined_force(const double *__restrict__ F, const ForceSums &c, int n3, int k) {
-  double s = 0;
-  for (int q = 0; q < c.T; ++q) s += c.Fpart[(size_t)q * n3 + k];
-  double f = F[k] + s / (double)c.P;
+  double f = F[k];
+  if (c.Fpart) {
+    double s = 0;
+    for (int q = 0; q < c.T; ++q) s += c.Fpart[(size_t)q * n3 + k];
+    f += s / (double)c.P;
+  }
   if (c.Frec) f += c.Frec[k];
   if (c.Fx) {
     const int nb = c.N * c.P, d = k / nb, i = k - d * nb;
@@ -285,14 +287,15 @@ int batch_table_make(BatchTable &t, const void *reps, size_t rep_bytes, const st
 void batch_table_free(BatchTable &t);
 
 // Fused bead-local stages of one system's step (massive thermostats only).
-// half 2 with cs (cs->Fpart set): F += the parts first (combined_force),
+// half 2 with cs (Fpart or Fx set): F += the parts first (combined_force),
 // stored, and used by the half-kick.  half 3: half 2 (with cs as for half 2)
 // and then the next step's half 1 (+ wrap) in one kernel.
 int launch_step_nhc(const BatchItem &it, int half, hipStream_t st, const ForceSums *cs = nullptr);
 int launch_step_bead_forces(const BatchItem &it, hipStream_t st);
 
 struct BeadBatch;  // integrator stages
-BeadBatch *bead_batch_create(const std::vector<BatchItem> &items);
+// sums: per item, the parts NHC half 2 adds into F first
+BeadBatch *bead_batch_create(const std::vector<BatchItem> &items, const std::vector<ForceSums> &sums);
 void bead_batch_free(BeadBatch *b);
 int bead_batch_nhc(BeadBatch *b, int half, hipStream_t st);     // NHC half (+ wrap after half 1)
 int bead_batch_forces(BeadBatch *b, hipStream_t st);            // reset, trap, interior springs
@@ -302,12 +305,15 @@ ExchBatch *exch_batch_create(const std::vector<BatchItem> &items);
 void exch_batch_free(ExchBatch *b);
 int exch_batch_enk(ExchBatch *b, hipStream_t st);
 int exch_batch_recursion(ExchBatch *b, hipStream_t st);
-int exch_batch_force(ExchBatch *b, hipStream_t st);
-int exch_batch_status(ExchBatch *b);
+int exch_batch_force(ExchBatch *b, hipStream_t st);  // stored apart (Fx)
+int exch_batch_status(ExchBatch *b);                 // waits for s0
 
 struct PairBatch;  // pair forces
 PairBatch *pair_batch_create(const std::vector<BatchItem> &items);
 void pair_batch_free(PairBatch *b);
-int pair_batch_forces(PairBatch *b, hipStream_t st);
+const std::vector<ForceSums> &pair_batch_sums(PairBatch *b);  // per item, what NHC half 2 adds into F
+int pair_batch_real(PairBatch *b, hipStream_t st);    // Gaussian tiles, Ewald real space (tile sums)
+int pair_batch_kspace(PairBatch *b, hipStream_t st);  // Ewald reciprocal forces (side buffers)
+int pair_batch_solo(PairBatch *b, hipStream_t st);    // the other replicas' pair forces, into F
 
 }  // namespace xmd
