@@ -307,6 +307,68 @@ __device__ __forceinline__ void pair_term(double dx, double dy, double dz, const
   }
 }
 
+// a / b for many a by one divisor: y = RN(1/b), two residual corrections.
+// After the first the quotient is within one ulp, and with a correctly rounded
+// y the second then gives RN(a/b) (Markstein's theorem), provided no residual
+// underflows: const_div_ok holds for 2^-900 <= |a| <= 2^900 and a divisor
+// within 2^+-60 of one.
+__device__ __forceinline__ double const_div(double a, double b, double y) {
+  double q = a * y;
+  q = fma(fma(-q, b, a), y, q);
+  return fma(fma(-q, b, a), y, q);
+}
+
+// Force on a bead from GAUSS_U others: (dx, dy, dz)[u] -> the terms of
+// pair_term<MODE, false>, to the last bit.  The chains (sqrt, exp, divisions)
+// are free of branches so that they interleave; the divisions by s^2 are
+// const_div's, and a wave with a dividend outside its range (a coordinate in
+// common, a far pair) repeats them plainly.  Issue bound: a rotation was 160
+// FP64 instructions, 65 of them five divisions, and is 130 (tiles and their
+// reduction at N=600 P=64 89 -> 74 us, N=512 P=32 52 -> 46.5; 2, 3 and 4 others
+// at a time measure the same, 2 has the smallest code).
+constexpr int GAUSS_U = 2;
+
+template <int MODE>
+__device__ __forceinline__ void gauss_terms(double *dx, double *dy, double *dz, const PairParams &pp, double pre,
+                                            double y, bool y_ok) {
+  constexpr double LO = 0x1p-900, HI = 0x1p900;
+  double a[GAUSS_U], qx[GAUSS_U], qy[GAUSS_U], qz[GAUSS_U];
+  bool in = y_ok;
+#pragma unroll
+  for (int u = 0; u < GAUSS_U; ++u) {
+    if (MODE == PK_PGAUSS) {
+      dx[u] = pf_min_image(dx[u], pp.L[0]);
+      dy[u] = pf_min_image(dy[u], pp.L[1]);
+      dz[u] = pf_min_image(dz[u], pp.L[2]);
+    }
+    const double d = sqrt(dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u]);
+    a[u] = -d * d;
+    const double w = pre * exp(const_div(a[u], pp.s2, y));
+    const double ax = w * (2 * dx[u]), ay = w * (2 * dy[u]), az = w * (2 * dz[u]);
+    const double mn = fmin(fmin(fabs(ax), -a[u]), fmin(fabs(ay), fabs(az)));
+    const double mx = fmax(fmax(fabs(ax), -a[u]), fmax(fabs(ay), fabs(az)));
+    in = in && mn >= LO && mx <= HI;
+    qx[u] = const_div(ax, pp.s2, y);
+    qy[u] = const_div(ay, pp.s2, y);
+    qz[u] = const_div(az, pp.s2, y);
+  }
+  if (!__all(in)) {
+#pragma unroll 1
+    for (int u = 0; u < GAUSS_U; ++u) {
+      const double w = pre * exp(a[u] / pp.s2);
+      qx[u] = w * (2 * dx[u]) / pp.s2;
+      qy[u] = w * (2 * dy[u]) / pp.s2;
+      qz[u] = w * (2 * dz[u]) / pp.s2;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < GAUSS_U; ++u) {
+    dx[u] = qx[u];
+    dy[u] = qy[u];
+    dz[u] = qz[u];
+  }
+}
+
 // Symmetric tile-pair kernel.  One 64-lane workgroup per (slice, I, J),
 // I <= J (64-bead tiles of one slice).  Lane t owns bead i = 64 I + t; the
 // J tile sits in LDS together with its reaction accumulators.  At rotation
@@ -344,7 +406,9 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
   jx[t] = jact ? X[base + jl] : 0.0;
   jy[t] = jact ? X[nb + base + jl] : 0.0;
   jz[t] = jact ? X[2 * nb + base + jl] : 0.0;
+  constexpr bool GAUSS = !ENERGY && (MODE == PK_GAUSS || MODE == PK_PGAUSS);
   jm[t] = jact ? M[base + jl] : 1.0;
+  if (GAUSS) jm[t] = 1.0 / jm[t];
   rx[t] = 0;
   ry[t] = 0;
   rz[t] = 0;
@@ -352,21 +416,57 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
   const bool diag = I == J;
   const int s_lo = diag ? 1 : 0, s_hi = diag ? 32 : 63;
   double fx = 0, fy = 0, fz = 0, e = 0;
-  for (int s = s_lo; s <= s_hi; ++s) {
-    const int j = (t + s) & 63;
-    const int jg = J * 64 + j;
-    const bool ok = act && jg < N && !(diag && s == 32 && t >= 32);
-    if (ok) {
-      double gx = 0, gy = 0, gz = 0;
-      pair_term<MODE, ENERGY, NEAR>(xi - jx[j], yi - jy[j], zi - jz[j], pp, gx, gy, gz, e);
-      if (!ENERGY) {
-        const double invm = 1.0 / (jg > i ? jm[j] : mi);
-        fx += gx * invm;
-        fy += gy * invm;
-        fz += gz * invm;
-        rx[j] -= gx * invm;
-        ry[j] -= gy * invm;
-        rz[j] -= gz * invm;
+  if (GAUSS) {
+    // GAUSS_U rotations at a time: their terms are independent chains (sqrt,
+    // exp, divisions), added one rotation after the other
+    const double pre = pp.g / (M_PI * pp.s2), y = 1.0 / pp.s2;
+    const bool y_ok = pp.s2 >= 0x1p-60 && pp.s2 <= 0x1p60;
+    const double im = 1.0 / mi;
+    // a diagonal tile of n <= 32 beads has no pair past rotation n - 1
+    const int nj = N - J * 64, s_end = diag && nj <= 32 ? nj - 1 : s_hi;
+    for (int s = s_lo; s <= s_end; s += GAUSS_U) {
+      double gx[GAUSS_U], gy[GAUSS_U], gz[GAUSS_U];
+      bool ok[GAUSS_U];
+#pragma unroll
+      for (int u = 0; u < GAUSS_U; ++u) {
+        const int j = (t + s + u) & 63;
+        ok[u] = act && s + u <= s_end && J * 64 + j < N && !(diag && s + u == 32 && t >= 32);
+        gx[u] = ok[u] ? xi - jx[j] : 1.0;
+        gy[u] = ok[u] ? yi - jy[j] : 1.0;
+        gz[u] = ok[u] ? zi - jz[j] : 1.0;
+      }
+      gauss_terms<MODE>(gx, gy, gz, pp, pre, y, y_ok);
+#pragma unroll
+      for (int u = 0; u < GAUSS_U; ++u) {
+        // a lane without a pair adds zeros (at a rotation no two lanes share j)
+        const int j = (t + s + u) & 63;
+        const double hx = ok[u] ? gx[u] : 0.0, hy = ok[u] ? gy[u] : 0.0, hz = ok[u] ? gz[u] : 0.0;
+        const double invm = J * 64 + j > i ? jm[j] : im;
+        fx += hx * invm;
+        fy += hy * invm;
+        fz += hz * invm;
+        rx[j] -= hx * invm;
+        ry[j] -= hy * invm;
+        rz[j] -= hz * invm;
+      }
+    }
+  } else {
+    for (int s = s_lo; s <= s_hi; ++s) {
+      const int j = (t + s) & 63;
+      const int jg = J * 64 + j;
+      const bool ok = act && jg < N && !(diag && s == 32 && t >= 32);
+      if (ok) {
+        double gx = 0, gy = 0, gz = 0;
+        pair_term<MODE, ENERGY, NEAR>(xi - jx[j], yi - jy[j], zi - jz[j], pp, gx, gy, gz, e);
+        if (!ENERGY) {
+          const double invm = 1.0 / (jg > i ? jm[j] : mi);
+          fx += gx * invm;
+          fy += gy * invm;
+          fz += gz * invm;
+          rx[j] -= gx * invm;
+          ry[j] -= gy * invm;
+          rz[j] -= gz * invm;
+        }
       }
     }
   }
