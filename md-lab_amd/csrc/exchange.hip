@@ -649,9 +649,15 @@ __device__ __forceinline__ void lse_pair(double &M, double &S, double m, double 
 // branch a conditional exp becomes.
 __device__ __forceinline__ double exp_if(bool ok, double x) { return exp(ok ? x : -2000.0); }
 
-// Log-sum-exp of 16 terms t_j of this lane, kept at buf[64 j] (LDS): the
-// exponentials run in a rolled loop, whose constants stay in registers (26
-// instead of 46 instructions each when unrolled).
+// Log-sum-exp of 16 terms t_j of this lane, kept at buf[64 j] (LDS), added in
+// order of j; only terms within LSE_SKIP of the largest count.  On states with
+// permutation cycles those are one or two of the 16 (a cycle ends where it
+// must), and an exponential, 46 instructions, is what a term costs: each lane
+// then picks its own out one by one.  Where a lane has many, the exponentials
+// run in a rolled loop over all, whose constants stay in registers (26 instead
+// of 46 instructions each when unrolled).
+constexpr int SPARSE_MAX = 6;
+
 __device__ __forceinline__ void lse16(const double *t, double *buf, double &M, double &S) {
   M = NEG;
 #pragma unroll
@@ -660,14 +666,26 @@ __device__ __forceinline__ void lse16(const double *t, double *buf, double &M, d
     buf[RB * j] = t[j];
   }
   S = 0.0;
-  const bool any = M > NEG;
+  const double lim = M > NEG ? M - LSE_SKIP : HUGE_VAL;
+  unsigned mask = 0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) mask |= t[j] > lim ? 1u << j : 0u;
+  if (!__any(__popc(mask) > SPARSE_MAX)) {
+#pragma unroll 1
+    while (__any(mask != 0)) {
+      const double e = exp_if(mask != 0, buf[RB * (mask ? __builtin_ctz(mask) : 0)] - M);
+      S += mask ? e : 0.0;
+      mask &= mask - 1;
+    }
+    return;
+  }
 #pragma unroll 1
   for (int j = 0; j < 16; j += 4) {
     double e[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) e[i] = buf[RB * (j + i)];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) e[i] = exp_if(any && e[i] > M - LSE_SKIP, e[i] - M);
+    for (int i = 0; i < 4; ++i) e[i] = exp_if(e[i] > lim, e[i] - M);
 #pragma unroll
     for (int i = 0; i < 4; ++i) S += e[i];
   }
@@ -792,6 +810,7 @@ struct alignas(16) RecLds {
   double lv[RB];                // its values L
   double tacc[4][RB], sacc[4][RB];  // look-ahead partials of the four waves (an exact fold: M and S)
   int fast;                     // the block's chain-frame solve stayed in range
+  int past;                     // the next block's will not (exact solve at once)
   double nm[RB], ns[RB];        // next block's accumulators, loaded by wave 1
   double pm[2][4][RB], ps[2][4][RB];  // fold partials (updater, or a self-fold in SOLO)
 };
@@ -897,12 +916,15 @@ __device__ __forceinline__ void rec_copy_wait() { __asm__ volatile("s_waitcnt vm
 // left the range also is.  Thermal states take this path in nearly every
 // block (each particle inside a longer cycle lies its ring-closing energy
 // above the chain, 48 at P = 32), so its coefficients are prefetched like the
-// frame's and the four waves share the exps of the solve (16 columns each)
-// and of the fold (its four 16-term log-sum-exps).  What bounds it is the
-// instruction issue of single waves (FP64 at about 6 cycles an instruction,
-// an exp 30 of them) and the serial scan and substitution.  Both directions
-// at UEG N=1024 P=32 with cycles: 755 -> 200 us, 42 -> 11.6 us per block,
-// against one wave loading and exponentiating all of a block.
+// frame's, the four waves share the exps of the solve (the triangle packed,
+// 8 per lane) and of the fold (its four 16-term log-sum-exps), and wave 2 finds
+// out beside the exact substitution whether the next block's frame solve would
+// fail as well, which then is not tried.  What bounds it is the instruction
+// issue of single waves (FP64 at about 6 cycles an instruction, an exp 30 of
+// them) and the serial scan and substitution.  Both directions at UEG N=1024
+// P=32 with cycles: 755 -> 175 us, 42 -> 10.3 us per block, against one wave
+// loading and exponentiating all of a block (11.6 with the frame tried in
+// every block, 16 exps per lane in the triangle and 16 in the fold).
 // SOLO: no updater workgroups; the solver folds blocks 0 .. b-1 into block
 // b+1 itself (same order and arithmetic as an updater), so it waits on no
 // other workgroup.
@@ -940,6 +962,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
     Sm = lane < nr0 ? AS[1 + lane] : 0.0;
     E = ECd[lane];
     Dl = ECd[RB];
+    if (lane == 0) S.past = 0;
   }
   for (int b = 0; b < a.nblk; ++b) {
     const int cur = b & 1;
@@ -962,6 +985,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       }
     };
     __syncthreads();
+    const bool past = S.past != 0;
     // block b+1's frame coefficients into LDS (copied there without passing
     // registers, by waves 1-3: wave 0's own LDS reads would wait for copies
     // it had issued), in flight during this block's attempt
@@ -1002,7 +1026,8 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       S.nm[lane] = lane < nrows1 ? m : NEG;
       S.ns[lane] = lane < nrows1 ? sv : 0.0;
     };
-    if (wv == 0) {
+    if (past) {
+    } else if (wv == 0) {
       sigma = readlane_d(M, 0) + log(readlane_d(Sm, 0));
       double W = lane < nrows ? Sm * exp(M - sigma - E) : 0.0;
       // column r of dg holds A(q, r) at row q = lane (0 unless r < q); NaN
@@ -1015,8 +1040,8 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       next_acc(false);
       rec_copy_wait();
     }
-    __syncthreads();
-    const bool fast = S.fast != 0;
+    if (!past) __syncthreads();
+    const bool fast = !past && S.fast != 0;
     RecRaw xl;  // block b+1's rows on this block
     if (fast) {
       next_acc(true);
@@ -1026,6 +1051,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
 #pragma unroll
       for (int j = 0; j < 16; ++j) dg[(16 * wv + j) * RB + lane] = c[j];
       rec_load16<FWD>(a, p1 + lane, p0 + 16 * wv, xl);
+      if (past && wv != 0) rec_copy_wait();
       __syncthreads();
       double sig = lane < nrows ? M : NEG;
       if (wv == 0) {
@@ -1033,16 +1059,31 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
         S.sg[lane] = lane < nrows ? sig : NEG;
       }
       __syncthreads();
-      const double sq = S.sg[lane];
+      // the triangle r < q, two columns to a pass: column r in the lanes above
+      // r, column 63 - r (turned about: row 63 - lane) in those below; the
+      // mirror position of each is outside it and set to 0
+      const double sq = S.sg[lane], sm = S.sg[RB - 1 - lane];
 #pragma unroll 1
-      for (int r = 16 * wv; r < 16 * wv + 16; r += 4) {  // rolled: see lse16
+      for (int r = 8 * wv; r < 8 * wv + 8; r += 4) {  // rolled: see lse16
         double e[4];
+        int at[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) e[i] = dg[(r + i) * RB + lane];
+        for (int i = 0; i < 4; ++i) {
+          const int w = (r + i) * RB + lane;
+          at[i] = lane > r + i ? w : RSQ - 1 - w;
+          e[i] = dg[at[i]];
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) e[i] = exp_if(e[i] > NEG, e[i] + S.sg[r + i] - sq);
+        for (int i = 0; i < 4; ++i) {
+          const bool up = lane > r + i;
+          const double d = S.sg[up ? r + i : RB - 1 - r - i];
+          e[i] = exp_if(lane != r + i && e[i] > NEG, e[i] + d - (up ? sq : sm));
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dg[(r + i) * RB + lane] = e[i];
+        for (int i = 0; i < 4; ++i) {
+          dg[at[i]] = e[i];
+          dg[RSQ - 1 - at[i]] = 0.0;
+        }
       }
       __syncthreads();
       if (wv == 0) {
@@ -1052,6 +1093,14 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
         publish(sig + log(W));
       } else {
         next_acc(true);
+        // Will block b+1 leave the range?  Its W is at least that of a row 0
+        // alone, W_0 = 1 (every W_q >= 1 and no term is negative), with a
+        // factor of 2 for the rounding of either.
+        if (wv == 2 && more) {
+          double W = lane == 0 ? 1.0 : 0.0;
+          const bool in = rec_subst(S.dg[cur ^ 1], nrows1, 2.0 * a.big, W);
+          if (lane == 0) S.past = in ? 0 : 1;
+        }
       }
       __syncthreads();
     }
