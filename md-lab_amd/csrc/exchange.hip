@@ -919,19 +919,23 @@ __device__ __forceinline__ void rec_copy_wait() { __asm__ volatile("s_waitcnt vm
 // frame's, the four waves share the exps of the solve (the triangle packed,
 // 8 per lane) and of the fold (its four 16-term log-sum-exps), and wave 2 finds
 // out beside the exact substitution whether the next block's frame solve would
-// fail as well, which then is not tried.  What bounds it is the instruction
-// issue of single waves (FP64 at about 6 cycles an instruction, an exp 30 of
-// them) and the serial scan and substitution.  Both directions at UEG N=1024
-// P=32 with cycles: 755 -> 175 us, 42 -> 10.3 us per block, against one wave
-// loading and exponentiating all of a block (11.6 with the frame tried in
-// every block, 16 exps per lane in the triangle and 16 in the fold).
+// fail as well, which then is not tried: waves 1-3 make its coefficients
+// beside wave 0's merge.  What bounds it is the instruction issue of single
+// waves (FP64 at about 6 cycles an instruction, an exp 30 of them) and the
+// serial scan and substitution.  Both directions at UEG N=1024 P=32 with
+// cycles: 755 -> 160 us, 42 -> 9.4 us per block, against one wave loading and
+// exponentiating all of a block (11.6 with the frame tried in every block, 16
+// exps per lane in the triangle and 16 in the fold; a fifth wave, so that wave
+// 0 is left the serial parts alone, took 8.7 us per block, but such a workgroup
+// waits longer for room beside the pair kernels: N=256 trap 4.6 -> 5.4 ms).
 // SOLO: no updater workgroups; the solver folds blocks 0 .. b-1 into block
 // b+1 itself (same order and arithmetic as an updater), so it waits on no
 // other workgroup.
 template <bool FWD, bool SOLO = false>
 __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S) {
   const int N = a.N;
-  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int lane = threadIdx.x & 63;
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   int *err = a.sync + 4 * a.nblk;
   // Test hook: while sync[4 nblk + 1] (set by the host, never by a normal
   // run) is positive, a forward solve takes one from it and its first poll
@@ -956,6 +960,13 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
   for (int w = tid; w < (nr0 + 15) / 16 * 16 * RB; w += 256) S.dg[0][w] = DGd[w];
   RecRaw xd;  // this wave's 16 columns of the block on itself, for an exact solve
   rec_load16<FWD>(a, 1 + lane, 1 + 16 * wv, xd);
+  // this wave's columns of the block of rows p .. p + n - 1 on itself, from xd
+  auto own_coefs = [&](int p, int n, double *tile) {
+    double c[16];
+    rec_conv16<FWD>(a, p + lane, p + 16 * wv, lane - 16 * wv, lane < n, xd, c);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) tile[(16 * wv + j) * RB + lane] = c[j];
+  };
   double M = NEG, Sm = 0.0, E = 0.0, Dl = 0.0;
   if (wv == 0) {
     M = lane < nr0 ? AM[1 + lane] : NEG;
@@ -965,6 +976,9 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
     if (lane == 0) S.past = 0;
   }
   for (int b = 0; b < a.nblk; ++b) {
+    // what depends on the lane alone is computed where it is used: hoisted out
+    // of the loop it took 60 registers
+    __asm__ volatile("" : "+v"(lane));
     const int cur = b & 1;
     const int p0 = 1 + b * RB, nrows = min(RB, N - p0 + 1);
     const bool more = b + 1 < a.nblk;
@@ -993,7 +1007,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
     if (more) {
       if (wv != 0) {
         rec_copy_tile(DGd + (size_t)(b + 1) * RSQ, S.dg[cur ^ 1], wv - 1);
-        rec_copy_tile(LAd + (size_t)(b + 1) * RSQ, S.la, wv - 1);
+        if (!past) rec_copy_tile(LAd + (size_t)(b + 1) * RSQ, S.la, wv - 1);
       } else {
         En = ECd[(size_t)(b + 1) * (RB + 1) + lane];
         Dn = ECd[(size_t)(b + 1) * (RB + 1) + RB];
@@ -1046,12 +1060,8 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
     if (fast) {
       next_acc(true);
     } else {
-      double c[16];
-      rec_conv16<FWD>(a, p0 + lane, p0 + 16 * wv, lane - 16 * wv, lane < nrows, xd, c);
-#pragma unroll
-      for (int j = 0; j < 16; ++j) dg[(16 * wv + j) * RB + lane] = c[j];
+      if (!past || wv == 0) own_coefs(p0, nrows, dg);
       rec_load16<FWD>(a, p1 + lane, p0 + 16 * wv, xl);
-      if (past && wv != 0) rec_copy_wait();
       __syncthreads();
       double sig = lane < nrows ? M : NEG;
       if (wv == 0) {
@@ -1085,6 +1095,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
           dg[RSQ - 1 - at[i]] = 0.0;
         }
       }
+      if (past && wv != 0) rec_copy_wait();
       __syncthreads();
       if (wv == 0) {
         double W = 0.0;
@@ -1105,6 +1116,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       __syncthreads();
     }
     if (!more) break;
+    if (!SOLO) rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
     if (fast) {
       double acc = 0.0;
 #pragma unroll
@@ -1123,9 +1135,11 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
     // SOLO: block b+1's accumulators over blocks 0 .. b-1, folded here
     double Mf = NEG, Sf = 0.0;
     if (SOLO && b + 1 >= 2) rec_fold_rows<FWD, false>(a, dir, b + 1, S.pm, S.ps, dg, Mf, Sf);
-    rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
+    if (SOLO) rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
     __syncthreads();
-    if (wv == 0) {
+    if (wv != 0) {
+      if (S.past) own_coefs(p1, nrows1, S.dg[cur ^ 1]);  // beside the merge
+    } else {
       double Mn, Sn;
       if (SOLO) {
         Mn = b + 1 >= 2 ? Mf : (lane < nrows1 ? AM[p1 + lane] : NEG);
