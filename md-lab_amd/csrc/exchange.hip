@@ -1209,10 +1209,18 @@ __global__ void k_vbn_to_L(const double *VBN, double *Lf, int N, double beta) {
 
 // --------------------------------------------------------- exchange force
 
+// Whether an element exp(x) of the connection matrix can be other than 0 (its
+// exponential underflows below -745.2; infinities and NaN keep their way).
+__device__ __forceinline__ bool connected(double x) { return !(x < -746.0 && x > -HUGE_VAL); }
+
 // Block per particle l (1-based l = blockIdx.x + 1): bead P against every
 // bead 1 (row l of G) and bead 1 against every bead P (column l of G).
 // Fx null: the forces are added into F.  Otherwise they are stored in Fx
 // ([slice P-1, slice 0][dimension][particle]) for k_add_exch to add later.
+// With permutation cycles a particle is connected to few others, and a wave of
+// partners it is not connected to is passed over after its exponents
+// (k_exch_force on such states, before -> now: N=2001 35.5 -> 23.0 us, N=1024
+// 15.6 -> 11.8).
 __device__ __forceinline__ void exch_force_body(int bx, const double *__restrict__ X, const double *__restrict__ M,
                                                 double *__restrict__ F, int N, int P, double om, Geo g,
                                                 const RecArgs &a, double *__restrict__ Fx = nullptr) {
@@ -1233,7 +1241,9 @@ __device__ __forceinline__ void exch_force_body(int bx, const double *__restrict
       const int k = l - j + 1;
       if (a.xi0 && k != 1) continue;
       const double c = (k - 1) * a.lnxi - a.beta * a.ENk[tri_row(l) + k - 1] - a.lnn[l];
-      G = exp(c + a.Lf[j - 1] + Rl - LN);
+      const double x = c + a.Lf[j - 1] + Rl - LN;
+      if (!__any(connected(x))) continue;
+      G = exp(x);
     } else {
       if (l == N) continue;
       G = 1 - exp(a.Lf[l] + Rl - LN);
@@ -1250,7 +1260,9 @@ __device__ __forceinline__ void exch_force_body(int bx, const double *__restrict
       const int k = jp - l + 1;
       if (a.xi0 && k != 1) continue;
       const double c = (k - 1) * a.lnxi - a.beta * a.ET[col_off(l - 1, N) + k - 1] - a.lnn[jp];
-      G = exp(c + Llm1 + a.Rb[jp] - LN);
+      const double x = c + Llm1 + a.Rb[jp] - LN;
+      if (!__any(connected(x))) continue;
+      G = exp(x);
     } else {
       G = 1 - exp(a.Lf[l - 1] + a.Rb[l - 1] - LN);
     }
