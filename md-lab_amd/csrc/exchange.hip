@@ -1233,6 +1233,15 @@ __device__ __forceinline__ void exch_force_body(int bx, const double *__restrict
   const double xP[3] = {X[sP], X[nb + sP], X[2 * nb + sP]};
   const double x1[3] = {X[s1], X[nb + s1], X[2 * nb + s1]};
   const double Ls[3] = {g.L0, g.L1, g.L2};
+  // threads 0 .. 2 finish one dimension each; what they need is loaded now
+  const int ed = threadIdx.x;
+  double eP = 0, e1 = 0, mP = 1, m1 = 1;
+  if (ed < 3) {
+    eP = X[ed * nb + (P - 2) * N + (l - 1)];
+    e1 = X[ed * nb + N + (l - 1)];
+    mP = M[sP];
+    m1 = M[s1];
+  }
   double gs = 0, gc[3] = {0, 0, 0}, hs = 0, hc[3] = {0, 0, 0};
   // row l: partners j = 1..l+1 (bead 1 of particle j)
   for (int j = 1 + threadIdx.x; j <= l + 1; j += blockDim.x) {
@@ -1283,23 +1292,21 @@ __device__ __forceinline__ void exch_force_body(int bx, const double *__restrict
 #pragma unroll
     for (int q = 0; q < 8; ++q) red[q][wv] = v[q];
   __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) red[q][0] = ((red[q][0] + red[q][1]) + red[q][2]) + red[q][3];
-    const int sPm = (P - 2) * N + (l - 1), s2 = N + (l - 1);
-    const double mP = M[sP], m1 = M[s1];
-    for (int d = 0; d < 3; ++d) {
-      double aP = comp(xP[d] - X[d * nb + sPm], Ls[d], g.image);
-      double gradP = (mP * om * om) * (red[0][0] * aP) + (mP * om * om) * red[1 + d][0];
-      double a1 = comp(x1[d] - X[d * nb + s2], Ls[d], g.image);
-      double grad1 = (m1 * om * om) * (red[4][0] * a1) + (m1 * om * om) * red[5 + d][0];
-      if (Fx) {
-        Fx[d * N + (l - 1)] = -gradP / mP;
-        Fx[(3 + d) * N + (l - 1)] = -grad1 / m1;
-      } else {
-        F[d * nb + sP] += -gradP / mP;
-        F[d * nb + s1] += -grad1 / m1;
-      }
+  if (ed < 3) {
+    auto sum = [&](int q) { return ((red[q][0] + red[q][1]) + red[q][2]) + red[q][3]; };
+    const double L = ed == 0 ? Ls[0] : ed == 1 ? Ls[1] : Ls[2];
+    const double xPd = ed == 0 ? xP[0] : ed == 1 ? xP[1] : xP[2], x1d = ed == 0 ? x1[0] : ed == 1 ? x1[1] : x1[2];
+    const double rP = sum(0), cP = sum(1 + ed), r1 = sum(4), c1 = sum(5 + ed);
+    double aP = comp(xPd - eP, L, g.image);
+    double gradP = (mP * om * om) * (rP * aP) + (mP * om * om) * cP;
+    double a1 = comp(x1d - e1, L, g.image);
+    double grad1 = (m1 * om * om) * (r1 * a1) + (m1 * om * om) * c1;
+    if (Fx) {
+      Fx[ed * N + (l - 1)] = -gradP / mP;
+      Fx[(3 + ed) * N + (l - 1)] = -grad1 / m1;
+    } else {
+      F[ed * nb + sP] += -gradP / mP;
+      F[ed * nb + s1] += -grad1 / m1;
     }
   }
 }
