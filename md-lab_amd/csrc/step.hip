@@ -95,6 +95,10 @@ static Lane main_lane() {
 // for room, and a fork costs its parent 5 us; so, with w = N^2 P pair terms
 // (us per step, the order before -> the order chosen, on thermal states with
 // exchange cycles t and uniform ones u):
+//   Line    no Ewald, the smallest: everything on s0.  Such a graph costs the
+//           host 10 us a step, one with branches 32, which at N=5 P=6 (36 ->
+//           32) and N=8 P=8 (34 .. 38 -> 35) is what the device takes, so that
+//           a busy host sets the pace; N=24 P=16 38 -> 45
 //   Pairs   the pair branch on s2 and the chain on s0, both from NHC on:
 //           no pair kernel fills the device (trap N=8 P=8 45 -> 34,
 //           N=256 P=64 t 92 -> 88, u 84 -> 65; Ewald N=333 P=27 t 130 -> 118,
@@ -111,13 +115,13 @@ static Lane main_lane() {
 //           N=2001 P=24 t 600 -> 491, u 405 -> 384)
 //   After   no Ewald: pair branch on s0 after the set-up, solves on s1 (trap
 //           N=600 P=64 t 164, u 146; 214 and 161 with Pairs)
-enum class Order { Serial, Pairs, Wide, Beside, Late, After };
+enum class Order { Serial, Line, Pairs, Wide, Beside, Late, After };
 
 static Order force_order(const StepPlan &sp, bool ewald) {
   const double w = (double)sp.p->N * sp.p->N * sp.p->P;
   if (ewald && sp.p->sur_mode) return Order::Beside;
   if (ewald) return w < 2.5e6 ? Order::Wide : w < 1.2e7 ? Order::Pairs : w < 5e7 ? Order::Beside : Order::Late;
-  return w < 8e6 ? Order::Pairs : Order::After;
+  return w < 1.5e3 ? Order::Line : w < 8e6 ? Order::Pairs : Order::After;
 }
 
 // ev: optional per-stage events (2 per stage: start, stop), may be null.

@@ -11,9 +11,10 @@ from test_gpu_graph_reuse import make, state, ueg_box
 
 pytestmark = pytest.mark.gpu
 
-# Ewald lines at 2.5e6, 1.2e7 and 5e7, other pair forces at 8e6
+# Ewald lines at 2.5e6, 1.2e7 and 5e7, other pair forces at 1.5e3 and 8e6
 CASES = [("ueg", 16, 32), ("ueg", 176, 48), ("ueg", 177, 48), ("ueg", 611, 32), ("ueg", 613, 32), ("ueg", 1249, 32),
-         ("ueg", 1251, 32), ("trap", 24, 16), ("trap", 353, 64), ("trap", 354, 64), ("ueg", 228, 48), ("ueg", 229, 48)]
+         ("ueg", 1251, 32), ("trap", 24, 16), ("trap", 353, 64), ("trap", 354, 64), ("ueg", 228, 48), ("ueg", 229, 48),
+         ("trap", 8, 8), ("trap", 5, 59), ("trap", 5, 61)]
 
 
 @pytest.mark.parametrize("kind,N,P", CASES)
