@@ -24,6 +24,8 @@ def test_cycle_energies(N, P):
     lib = pyxmd.Lib()
     x = bridges(N, P, 1.0, 12, np.random.default_rng([7, N, P]))
     s = pyxmd.System(lib, "trap", N, P, 1.0, 1.0, seed=1, positions=x.reshape(N * P, 3))
+    if N * P % 2:  # an odd number of draws leaves a spare, which the next seed does not clear
+        lib.md_random_gaussian_x()
     hb = s.host_beads()
     o = Oracle()
     b = beads_from(hb["x"].reshape(-1), m=hb["m"])

@@ -21,6 +21,8 @@ def test_energy_routes(N, P):
     lib = pyxmd.Lib()
     L = pyxmd.ueg_box(N, 2.0)
     s = pyxmd.System(lib, "ueg", N, P, pyxmd.ueg_temperature(N, L, 0.5), 1.0, seed=5 + N, L=L, nsum=8)
+    if N * P % 2:  # an odd number of draws leaves a spare, which the next seed does not clear
+        lib.md_random_gaussian_x()
     try:
         lib.md_set_ewald_real_cutoff_x(6.6)
         want = energy(lib, s)
