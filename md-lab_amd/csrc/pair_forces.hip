@@ -369,6 +369,15 @@ __device__ __forceinline__ void gauss_terms(double *dx, double *dy, double *dz, 
   }
 }
 
+// A tile's partial sum into its slot, or (add = P > 0: one tile, whose slots
+// lie as F does) into F as k_reduce_tiles would add it.
+__device__ __forceinline__ void put_tile(double *slot, double v, double add) {
+  if (add > 0.0)
+    *slot += (0.0 + v) / add;
+  else
+    *slot = v;
+}
+
 // Symmetric tile-pair kernel.  One 64-lane workgroup per (slice, I, J),
 // I <= J (64-bead tiles of one slice).  Lane t owns bead i = 64 I + t; the
 // J tile sits in LDS together with its reaction accumulators.  At rotation
@@ -385,7 +394,7 @@ template <int MODE, bool ENERGY, bool NEAR>
 __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restrict__ X, const double *__restrict__ M,
                                                    double *__restrict__ Fpart, double *__restrict__ Epart,
                                                    const int2 *__restrict__ tiles, int N, int nb, int T, int ntp,
-                                                   PairParams pp) {
+                                                   PairParams pp, double add = 0.0) {
   __shared__ double jx[64], jy[64], jz[64], jm[64], rx[64], ry[64], rz[64];
   const int item = bx;
   const int slice = item / ntp;
@@ -478,9 +487,9 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
   }
   auto put = [&](int bead, int slot, double vx, double vy, double vz) {
     const size_t s0 = (size_t)slot * 3 * nb + base + bead;
-    Fpart[s0] = vx;
-    Fpart[s0 + nb] = vy;
-    Fpart[s0 + 2 * (size_t)nb] = vz;
+    put_tile(Fpart + s0, vx, add);
+    put_tile(Fpart + s0 + nb, vy, add);
+    put_tile(Fpart + s0 + 2 * (size_t)nb, vz, add);
   };
   if (diag) {
     if (act) put(i, I, fx + rx[t], fy + ry[t], fz + rz[t]);
@@ -494,8 +503,8 @@ template <int MODE, bool ENERGY, bool NEAR>
 __global__ __launch_bounds__(64) void k_pair_tiles(const double *__restrict__ X, const double *__restrict__ M,
                                                    double *__restrict__ Fpart, double *__restrict__ Epart,
                                                    const int2 *__restrict__ tiles, int N, int nb, int T, int ntp,
-                                                   PairParams pp) {
-  k_pair_tiles_body<MODE, ENERGY, NEAR>(blockIdx.x, X, M, Fpart, Epart, tiles, N, nb, T, ntp, pp);
+                                                   PairParams pp, double add) {
+  k_pair_tiles_body<MODE, ENERGY, NEAR>(blockIdx.x, X, M, Fpart, Epart, tiles, N, nb, T, ntp, pp, add);
 }
 
 // F[d*nb + s] += sum_slot Fpart / P, slots in a fixed order.
@@ -1504,7 +1513,7 @@ __device__ __forceinline__ double wave_rol1(double v) {
 template <int IMG, int WPB = 4>
 __device__ __forceinline__ void k_ewald_real_body(int bx, const double *__restrict__ X, const double *__restrict__ M,
                                                     double *__restrict__ Fpart, const int2 *__restrict__ tiles, int N,
-                                                    int nb, int T, int ntp, int nitems, EwReal ep) {
+                                                    int nb, int T, int ntp, int nitems, EwReal ep, double add = 0.0) {
   __shared__ double2 tab[kEwTabIntervals * kEwTabStride / 2];
   // the wave index and everything derived from it are wave-uniform: read
   // them as such, so the step loop below runs on scalar registers
@@ -1575,9 +1584,9 @@ __device__ __forceinline__ void k_ewald_real_body(int bx, const double *__restri
   }
   auto put = [&](int bead, int slot, double vx, double vy, double vz) {
     const size_t s0 = (size_t)slot * 3 * nb + base + bead;
-    Fpart[s0] = vx;
-    Fpart[s0 + nb] = vy;
-    Fpart[s0 + 2 * (size_t)nb] = vz;
+    put_tile(Fpart + s0, vx, add);
+    put_tile(Fpart + s0 + nb, vy, add);
+    put_tile(Fpart + s0 + 2 * (size_t)nb, vz, add);
   };
   if (diag) {
     if (act) put(i, I, fx + rx, fy + ry, fz + rz);
@@ -1593,8 +1602,8 @@ __device__ __forceinline__ void k_ewald_real_body(int bx, const double *__restri
 template <int IMG, int WPB>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_ewald_real(const double *__restrict__ X, const double *__restrict__ M,
                                                          double *__restrict__ Fpart, const int2 *__restrict__ tiles,
-                                                         int N, int nb, int T, int ntp, int nitems, EwReal ep) {
-  k_ewald_real_body<IMG, WPB>(blockIdx.x, X, M, Fpart, tiles, N, nb, T, ntp, nitems, ep);
+                                                         int N, int nb, int T, int ntp, int nitems, EwReal ep, double add) {
+  k_ewald_real_body<IMG, WPB>(blockIdx.x, X, M, Fpart, tiles, N, nb, T, ntp, nitems, ep, add);
 }
 
 // Real-space energy of every tile pair, items and rotation as in
@@ -1770,15 +1779,18 @@ static int launch_pair_mode(DevPimd *p, const PairParams &pp, hipStream_t st, do
   TileBufs &B = pair_bufs(p)->tb;
   const bool near = (MODE == PK_EWALD_NI) || (MODE == PK_EWALD_R2) || near_ok(pp);
   const int items = p->P * B.ntp;
+  const bool direct = !ENERGY && reduce && B.T == 1;  // one tile: straight into F
+  double *out = direct ? d->F : B.Fpart;
+  const double add = direct ? pp.P : 0.0;
   if (near)
-    hipLaunchKernelGGL((k_pair_tiles<MODE, ENERGY, true>), dim3(items), dim3(64), 0, st, d->X, d->M, B.Fpart,
-                       B.Epart, B.tiles, p->N, d->nb, B.T, B.ntp, pp);
+    hipLaunchKernelGGL((k_pair_tiles<MODE, ENERGY, true>), dim3(items), dim3(64), 0, st, d->X, d->M, out,
+                       B.Epart, B.tiles, p->N, d->nb, B.T, B.ntp, pp, add);
   else
-    hipLaunchKernelGGL((k_pair_tiles<MODE, ENERGY, false>), dim3(items), dim3(64), 0, st, d->X, d->M, B.Fpart,
-                       B.Epart, B.tiles, p->N, d->nb, B.T, B.ntp, pp);
+    hipLaunchKernelGGL((k_pair_tiles<MODE, ENERGY, false>), dim3(items), dim3(64), 0, st, d->X, d->M, out,
+                       B.Epart, B.tiles, p->N, d->nb, B.T, B.ntp, pp, add);
   XMD_CHECK(hipGetLastError());
   if (ENERGY) return device_sum(B.Epart, items, esum);
-  if (!reduce) return 0;
+  if (!reduce || direct) return 0;
   const int n3 = 3 * d->nb;
   hipLaunchKernelGGL(k_reduce_tiles, dim3((n3 + 255) / 256), dim3(256), 0, st, B.Fpart, d->F, n3, B.T, pp.P);
   XMD_CHECK(hipGetLastError());
@@ -1921,7 +1933,7 @@ static int image_mode(const PairParams &pp) {
 // autotuner times every valid choice on an object's current positions and
 // keeps the fastest per bucket (N rounded up to a power of two, P, and the
 // most specific valid enumeration).
-using RealKern = void (*)(const double *, const double *, double *, const int2 *, int, int, int, int, int, EwReal);
+using RealKern = void (*)(const double *, const double *, double *, const int2 *, int, int, int, int, int, EwReal, double);
 static const RealKern k_ewald_real_of[3][4] = {
     {k_ewald_real<IMG_FACE, 1>, k_ewald_real<IMG_FACE, 2>, k_ewald_real<IMG_FACE, 4>, k_ewald_real<IMG_FACE, 8>},
     {k_ewald_real<IMG_NEAR, 1>, k_ewald_real<IMG_NEAR, 2>, k_ewald_real<IMG_NEAR, 4>, k_ewald_real<IMG_NEAR, 8>},
@@ -1985,14 +1997,15 @@ static int launch_ewald_real_tab(DevPimd *p, const PairParams &pp, hipStream_t s
   const int items = p->P * B.ntp;
   const RealChoice ch = real_choice(p->N, p->P, pp);
   const int wpb = 1 << ch.wlog;
+  const bool direct = reduce && B.T == 1;  // one tile: straight into F
   hipLaunchKernelGGL(k_ewald_real_of[ch.img][ch.wlog], dim3((items + wpb - 1) / wpb), dim3(64 * wpb), 0, st, d->X, d->M,
-                     B.Fpart, B.tiles_r, p->N, d->nb, B.T, B.ntp, items, ep);
+                     direct ? d->F : B.Fpart, B.tiles_r, p->N, d->nb, B.T, B.ntp, items, ep, direct ? pp.P : 0.0);
   XMD_CHECK(hipGetLastError());
   if (g_real_probe) {
     XMD_CHECK(hipEventRecord(g_real_probe, st));
     g_real_probe_hit = true;
   }
-  if (!reduce) return 0;
+  if (!reduce || direct) return 0;
   const int n3 = 3 * d->nb;
   hipLaunchKernelGGL(k_reduce_tiles, dim3((n3 + 255) / 256), dim3(256), 0, st, B.Fpart, d->F, n3, B.T, pp.P);
   XMD_CHECK(hipGetLastError());
@@ -2139,7 +2152,7 @@ int autotune_real(DevPimd *p, int reps, double *ms, int *choice) {
       const int wpb = 1 << wl;
       auto launch = [&]() {
         hipLaunchKernelGGL(k_ewald_real_of[img][wl], dim3((items + wpb - 1) / wpb), dim3(64 * wpb), 0, st, d->X,
-                           d->M, B.Fpart, B.tiles_r, p->N, d->nb, B.T, B.ntp, items, ep);
+                           d->M, B.Fpart, B.tiles_r, p->N, d->nb, B.T, B.ntp, items, ep, 0.0);
       };
       launch();
       XMD_CHECK(hipEventRecord(e0, st));
