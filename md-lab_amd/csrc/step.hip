@@ -108,11 +108,12 @@ static Lane main_lane() {
 //           against Pairs, N=128 P=64 t 89 -> 87, u 88 -> 76, N=256 P=32
 //           t 98 -> 102, u 90 -> 80, N=333 P=27 t 118 -> 122)
 //   Beside  Ewald, the real space on s2 from NHC on, bead-local and reciprocal
-//           forces on s0 after the set-up, the solves on s1 (N=1024 P=32
-//           t 273, u 188; 266 and 201 with Late)
+//           forces on s0 after the set-up, the solves on s1 (N=700 P=32 t 177,
+//           u 137, and 161 and 155 with Pairs; N=1024 P=32 t 237, u 184, and
+//           228 and 198 with Late)
 //   Late    as Beside, the real space after the set-up and behind the solves:
-//           they are placed first (N=1500 P=32 t 442 -> 374, u 311 -> 325;
-//           N=2001 P=24 t 600 -> 491, u 405 -> 384)
+//           they are placed first (N=1500 P=32 t 394 -> 328, u 308 -> 318;
+//           N=2001 P=24 t 525 -> 407, u 398 -> 370)
 //   After   no Ewald: pair branch on s0 after the set-up, solves on s1 (trap
 //           N=600 P=64 t 164, u 146; 214 and 161 with Pairs)
 enum class Order { Serial, Line, Pairs, Wide, Beside, Late, After };
