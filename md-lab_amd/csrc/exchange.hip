@@ -227,17 +227,16 @@ __device__ __forceinline__ void chain_priority() { __builtin_amdgcn_s_setprio(3)
 // stored through to memory and read from there, and the count follows once
 // the stores have completed, so no cache is flushed or emptied for the rest
 // of what the kernels beside this one hold in it.
-__global__ __launch_bounds__(256) void k_chain_scan(const double *__restrict__ X, const double *__restrict__ M, int N,
-                                                    int P, double om, Geo g, double *__restrict__ Eint,
-                                                    double *__restrict__ Clink, double *__restrict__ ENk,
-                                                    double *__restrict__ ET, double *__restrict__ pre,
-                                                    int *__restrict__ done) {
+__device__ __forceinline__ void chain_scan_body(int bx, int nwg, const double *__restrict__ X,
+                                                const double *__restrict__ M, int N, int P, double om, const Geo &g,
+                                                double *__restrict__ Eint, double *__restrict__ Clink,
+                                                double *__restrict__ ENk, double *__restrict__ ET,
+                                                double *__restrict__ pre, int *__restrict__ done) {
   __shared__ int last;
   __shared__ double link[CHAIN_PW];
-  chain_priority();
-  const double c = chain_body(blockIdx.x, X, M, N, P, om, g, Eint, ENk, ET);
-  const int l = blockIdx.x * CHAIN_PW + threadIdx.x;
-  if (gridDim.x == 1) {
+  const double c = chain_body(bx, X, M, N, P, om, g, Eint, ENk, ET);
+  const int l = bx * CHAIN_PW + threadIdx.x;
+  if (nwg == 1) {
     if (threadIdx.x < CHAIN_PW) link[threadIdx.x] = c;
     __syncthreads();
     scan_dd_body<false>(link, N, pre);
@@ -248,12 +247,39 @@ __global__ __launch_bounds__(256) void k_chain_scan(const double *__restrict__ X
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
     if (threadIdx.x == 0)
-      last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+      last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nwg - 1;
   }
   __syncthreads();
   if (!last) return;
   scan_dd_body<true>(Clink, N, pre);
   if (threadIdx.x == 0) __hip_atomic_store(done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(256) void k_chain_scan(const double *__restrict__ X, const double *__restrict__ M, int N,
+                                                    int P, double om, Geo g, double *__restrict__ Eint,
+                                                    double *__restrict__ Clink, double *__restrict__ ENk,
+                                                    double *__restrict__ ET, double *__restrict__ pre,
+                                                    int *__restrict__ done) {
+  chain_priority();
+  chain_scan_body(blockIdx.x, gridDim.x, X, M, N, P, om, g, Eint, Clink, ENk, ET, pre, done);
+}
+
+// The same (workgroups 0 .. nwg - 1) with the bead-local forces in the
+// workgroups behind them: a launch fewer where launches are what a step costs
+// (100 steps of N = P = 8 3.48 -> 3.32 ms, of N=16 P=32 UEG 5.1 -> 5.0; N=128
+// P=64 and N=256 P=64 as before).
+__global__ __launch_bounds__(256) void k_chain_bead(const double *__restrict__ X, const double *__restrict__ M, int N,
+                                                    int P, double om, Geo g, double *__restrict__ Eint,
+                                                    double *__restrict__ Clink, double *__restrict__ ENk,
+                                                    double *__restrict__ ET, double *__restrict__ pre,
+                                                    int *__restrict__ done, int nwg, BeadRep R) {
+  if ((int)blockIdx.x < nwg) {
+    chain_priority();
+    chain_scan_body(blockIdx.x, nwg, X, M, N, P, om, g, Eint, Clink, ENk, ET, pre, done);
+    return;
+  }
+  const int i = ((int)blockIdx.x - nwg) * 256 + threadIdx.x;
+  if (i < 3 * R.nb) bead_forces_body(R, i);
 }
 
 // Cycle energies with k >= 2, both layouts, one EKT x EKT tile per workgroup:
@@ -1873,7 +1899,7 @@ int inject_recursion_timeouts(DevPimd *p, int count) {
   return 0;
 }
 
-int launch_enk_prep(DevPimd *p, int image, hipStream_t st) {
+int launch_enk_prep(DevPimd *p, int image, hipStream_t st, const BeadRep *bead) {
   DevSim *d = p->ds;
   const int N = p->N, P = p->P;
   EnkArgs e;
@@ -1886,8 +1912,13 @@ int launch_enk_prep(DevPimd *p, int image, hipStream_t st) {
   e.N = N;
   e.P = P;
   double *clink = p->work + (N + 1);
-  hipLaunchKernelGGL(k_chain_scan, dim3((N + CHAIN_PW - 1) / CHAIN_PW), dim3(256), 0, st, d->X, d->M, N, P, e.om, e.g,
-                     p->Eint, clink, p->ENk, p->ET, p->Cpre, p->done);
+  const int nwg = (N + CHAIN_PW - 1) / CHAIN_PW;
+  if (bead)
+    hipLaunchKernelGGL(k_chain_bead, dim3(nwg + (3 * d->nb + 255) / 256), dim3(256), 0, st, d->X, d->M, N, P, e.om, e.g,
+                       p->Eint, clink, p->ENk, p->ET, p->Cpre, p->done, nwg, *bead);
+  else
+    hipLaunchKernelGGL(k_chain_scan, dim3(nwg), dim3(256), 0, st, d->X, d->M, N, P, e.om, e.g, p->Eint, clink, p->ENk,
+                       p->ET, p->Cpre, p->done);
   XMD_CHECK(hipGetLastError());
   RecArgs a = rec_args(p);
   const int nprepb = rec_prep_wgs(N, a.nblk);

@@ -312,19 +312,6 @@ __global__ __launch_bounds__(256) void k_bead_sums(const double *__restrict__ X,
 
 // ------------------------------------------------- batched replicas
 //
-// Per-replica arguments of the bead-local stages; every thread owns one
-// degree of freedom e = d * nb + s of one replica, with the same arithmetic
-// as the single-system kernels above.
-struct BeadRep {
-  double *X, *V, *F, *th, *vth;
-  const double *M, *Q;
-  int nb, N, P, Mlen;
-  double T, h;
-  int pbc, image, trap;
-  double L[3], w, c[3], om;
-  ForceSums cs;  // half 2: parts added into F first (Fpart or Fx set)
-};
-
 // NHC half-kick (+ drift for HALF 1), then the box wrap after HALF 1, for
 // degree of freedom e < 3 nb.  HALF 3: half 2 of one step and half 1 of the
 // next in one pass (the force does not change between them; every chain is
@@ -369,35 +356,6 @@ __global__ __launch_bounds__(256) void k_nhc_wrap(BeadRep R) {
   nhc_wrap_body<HALF>(R, e);
 }
 
-// Force reset, trap (md_pimd_x.c:1370-1389) and interior ring springs of
-// degree of freedom i < 3 nb: the arithmetic of k_fill, k_trap and
-// k_ring_springs in one pass.
-__device__ __forceinline__ void bead_forces_body(const BeadRep &R, int i) {
-  const int nb = R.nb;
-  const int d = i / nb, s = i - d * nb;
-  double Fv = 0.0;
-  if (R.trap) {
-    double f = 0;
-    f += -R.w * R.w * (R.X[i] - R.c[d]);
-    Fv += f / R.P;
-  }
-  if (s >= R.N && s < nb - R.N) {
-    const double m = R.M[s], om = R.om;
-    const double x = R.X[i];
-    double a = x - R.X[i + R.N];
-    double c = x - R.X[i - R.N];
-    if (R.image) {
-      a = min_image(a, R.L[d]);
-      c = min_image(c, R.L[d]);
-    }
-    double g = 0;
-    g += m * om * om * a;
-    g += m * om * om * c;
-    Fv += -g / m;
-  }
-  R.F[i] = Fv;
-}
-
 __global__ __launch_bounds__(256) void kb_bead_forces(const BeadRep *__restrict__ reps, const int *__restrict__ start,
                                                       int nrep) {
   const int r = batch_rep(start, nrep, blockIdx.x);
@@ -413,7 +371,7 @@ __global__ __launch_bounds__(256) void k_bead_forces(BeadRep R) {
   bead_forces_body(R, i);
 }
 
-static BeadRep bead_rep(const BatchItem &it) {
+BeadRep bead_rep(const BatchItem &it) {
   DevPimd *p = it.p;
   DevSim *d = p->ds;
   BeadRep R;

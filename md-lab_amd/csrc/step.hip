@@ -140,6 +140,10 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   // sums and the exchange forces are left for NHC half 2 as well, two launches
   // and a pass over F fewer
   const bool parts = !serial && fused && d->massive && kind >= 0 && (ewald || !pair_has_recip(kind));
+  // (then nothing but NHC half 2 reads F, and in the orders of small systems
+  // the bead-local forces ride with the springs of the cycle energies)
+  const bool ride = parts && (o == Order::Line || o == Order::Pairs || o == Order::Wide);
+  const BeadRep ride_rep = bead_rep(item_of(sp));
   const bool pairs_s2 = o == Order::Pairs || o == Order::Wide;  // bead-local and pair forces on s2
   const bool fork_solve = o == Order::Beside || o == Order::Late || o == Order::After;
   const hipStream_t sx = fork_solve ? R.s1 : R.s0, sb = pairs_s2 ? R.s2 : R.s0;
@@ -173,7 +177,8 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   if (s2 && o != Order::Late && fork(R.fork2, R.s2)) return -1;
   if (o == Order::Wide) XMD_CHECK(hipStreamWaitEvent(R.s1, R.fork2, 0));
   if (o == Order::Beside && real(R.s2)) return -1;
-  if (rec(2, R.s0) || (serial ? launch_enk(p, sp.image, R.s0) : launch_enk_prep(p, sp.image, R.s0)) ||
+  if (rec(2, R.s0) || (serial ? launch_enk(p, sp.image, R.s0)
+                             : launch_enk_prep(p, sp.image, R.s0, ride ? &ride_rep : nullptr)) ||
       rec(3, R.s0))
     return -1;
   if (fork_solve && fork(R.fork, R.s1)) return -1;
@@ -184,7 +189,7 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   if (fork_solve) XMD_CHECK(hipEventRecord(R.join, R.s1));
   if (o == Order::Late && (fork(R.fork2, R.s2) || real(R.s2))) return -1;
   // bead-local and pair forces
-  if (bead(sb)) return -1;
+  if (ride ? rec(6, R.s0) || rec(7, R.s0) : bead(sb)) return -1;
   if (ewald) {
     if ((o == Order::Pairs && real(sb)) || kspace(sb)) return -1;
     if (o == Order::Wide) {

@@ -28,6 +28,8 @@ extern "C" {
 #include "md_pimd_x.h"
 }
 
+#include "xmd_device.h"
+
 #define XMD_CHECK(call)                                                                    \
   do {                                                                                     \
     hipError_t e_ = (call);                                                                \
@@ -231,10 +233,12 @@ bool pair_has_recip(int kind);
 int pair_energy(DevPimd *p, int kind, double *out);
 
 int launch_enk(DevPimd *p, int image, hipStream_t st);
+struct BeadRep;
 // launch_enk plus the recursion set-up of both directions in two kernels;
 // launch_recursion_solve then runs both recursions (together: launch_enk
 // followed by launch_recursion(p, true, true)).
-int launch_enk_prep(DevPimd *p, int image, hipStream_t st);
+// bead: the bead-local forces ride in the first of them.
+int launch_enk_prep(DevPimd *p, int image, hipStream_t st, const BeadRep *bead = nullptr);
 int launch_recursion_solve(DevPimd *p, hipStream_t st);
 int init_lnn(DevPimd *p);  // ln n table at p->work[0..N], once per object
 // mid (optional): recorded between the set-up and the persistent solve.
@@ -285,6 +289,50 @@ struct BatchTable {
 };
 int batch_table_make(BatchTable &t, const void *reps, size_t rep_bytes, const std::vector<int> &blocks);
 void batch_table_free(BatchTable &t);
+
+// Per-replica arguments of the bead-local stages; every thread owns one
+// degree of freedom e = d * nb + s of one replica, with the same arithmetic
+// as the single-system kernels above.
+struct BeadRep {
+  double *X, *V, *F, *th, *vth;
+  const double *M, *Q;
+  int nb, N, P, Mlen;
+  double T, h;
+  int pbc, image, trap;
+  double L[3], w, c[3], om;
+  ForceSums cs;  // half 2: parts added into F first (Fpart or Fx set)
+};
+
+// Force reset, trap (md_pimd_x.c:1370-1389) and interior ring springs of
+// degree of freedom i < 3 nb: the arithmetic of k_fill, k_trap and
+// k_ring_springs in one pass.
+__device__ __forceinline__ void bead_forces_body(const BeadRep &R, int i) {
+  const int nb = R.nb;
+  const int d = i / nb, s = i - d * nb;
+  double Fv = 0.0;
+  if (R.trap) {
+    double f = 0;
+    f += -R.w * R.w * (R.X[i] - R.c[d]);
+    Fv += f / R.P;
+  }
+  if (s >= R.N && s < nb - R.N) {
+    const double m = R.M[s], om = R.om;
+    const double x = R.X[i];
+    double a = x - R.X[i + R.N];
+    double c = x - R.X[i - R.N];
+    if (R.image) {
+      a = dv_min_image(a, R.L[d]);
+      c = dv_min_image(c, R.L[d]);
+    }
+    double g = 0;
+    g += m * om * om * a;
+    g += m * om * om * c;
+    Fv += -g / m;
+  }
+  R.F[i] = Fv;
+}
+
+BeadRep bead_rep(const BatchItem &it);
 
 // Fused bead-local stages of one system's step (massive thermostats only).
 // half 2 with cs (Fpart or Fx set): F += the parts first (combined_force),
