@@ -140,9 +140,11 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   // sums and the exchange forces are left for NHC half 2 as well, two launches
   // and a pass over F fewer
   const bool parts = !serial && fused && d->massive && kind >= 0 && (ewald || !pair_has_recip(kind));
-  // (then nothing but NHC half 2 reads F, and in the orders of small systems
-  // the bead-local forces ride with the springs of the cycle energies)
-  const bool ride = parts && (o == Order::Line || o == Order::Pairs || o == Order::Wide);
+  // (then nothing but NHC half 2 reads F, and in small systems the bead-local
+  // forces ride with the springs of the cycle energies: N=8 P=8 34.8 -> 33.2 us
+  // per step, N=64 P=32 59.9 -> 59.5, but N=200 P=40 90 -> 93, their workgroups
+  // in the way of the chain's)
+  const bool ride = parts && (double)p->N * p->N * p->P < 2e5;
   const BeadRep ride_rep = bead_rep(item_of(sp));
   const bool pairs_s2 = o == Order::Pairs || o == Order::Wide;  // bead-local and pair forces on s2
   const bool fork_solve = o == Order::Beside || o == Order::Late || o == Order::After;
