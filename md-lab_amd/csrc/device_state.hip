@@ -182,6 +182,11 @@ void batch_table_free(BatchTable &t) {
   t = BatchTable();
 }
 
+int clear_device(void *p, size_t bytes) {
+  XMD_CHECK(hipMemsetAsync(p, 0, bytes, rt().s0));
+  return 0;
+}
+
 double *host_scratch(size_t n) {
   static double *buf = nullptr;
   static size_t cap = 0;
@@ -384,9 +389,9 @@ static int alloc_pimd(DevPimd *p) {
   const size_t nblk = (N + 63) / 64;
   XMD_CHECK(hipMalloc(&p->rec, (10 * (size_t)(N + 1) + 2 * nblk * (64 * 64 + 64 * 64 + 65)) * sizeof(double)));
   XMD_CHECK(hipMalloc(&p->recsync, (4 * nblk + 2) * sizeof(int)));
-  XMD_CHECK(hipMemset(p->recsync, 0, (4 * nblk + 2) * sizeof(int)));
+  if (clear_device(p->recsync, (4 * nblk + 2) * sizeof(int))) return -1;
   XMD_CHECK(hipMalloc(&p->done, sizeof(int)));
-  XMD_CHECK(hipMemset(p->done, 0, sizeof(int)));
+  if (clear_device(p->done, sizeof(int))) return -1;
   // ln n, n = 0..N, in the first N+1 doubles of the scratch (constant)
   return init_lnn(p);
 }

@@ -1875,7 +1875,7 @@ int recursion_status(DevPimd *p) {
   XMD_CHECK(hipMemcpy(&err, p->recsync + 4 * nblk, sizeof(int), hipMemcpyDeviceToHost));
   if (err) {
     fprintf(stderr, "xmd: exchange recursion hand-off timed out\n");
-    XMD_CHECK(hipMemset(p->recsync + 4 * nblk, 0, sizeof(int)));
+    (void)clear_device(p->recsync + 4 * nblk, sizeof(int));
     return -1;
   }
   return 0;

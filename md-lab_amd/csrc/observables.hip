@@ -315,7 +315,7 @@ static unsigned long long *obs_counts(int points) {
   if (points > g_counts_cap) {
     obs_counts_drop();
     if (hipMalloc(&g_counts, points * sizeof(unsigned long long)) != hipSuccess) return nullptr;
-    if (hipMemset(g_counts, 0, points * sizeof(unsigned long long)) != hipSuccess) {
+    if (clear_device(g_counts, points * sizeof(unsigned long long))) {
       obs_counts_drop();
       return nullptr;
     }

@@ -941,7 +941,7 @@ static int sur_ensure(Surrogate *S, DevPimd *p) {
   const int ngb = (nb + GB - 1) / GB;
   if (ngb > S->cap_gb) {
     if (dalloc(S->gpart, (size_t)ngb * NPAR)) return -1;
-    XMD_CHECK(hipMemset(S->gpart, 0, (size_t)ngb * NPAR * sizeof(float)));
+    if (clear_device(S->gpart, (size_t)ngb * NPAR * sizeof(float))) return -1;
     S->cap_gb = ngb;
   }
   if (p->P > S->cap_sl) {

@@ -127,6 +127,11 @@ int ensure_pimd_device(md_pimd_t_x *pimd);
 int download_sim(DevSim *d);                         // device -> host mirror
 int download_pimd(DevPimd *p);
 
+// Clears device memory in s0's order.  (The null stream's hipMemset is not an
+// order: s0 does not wait for it, and it may return before the memory is
+// cleared.)  Not under capture.
+int clear_device(void *p, size_t bytes);
+
 // Pinned host memory of at least n doubles that kernels read and write
 // directly (grown on demand, kept; used by one call at a time, which waits
 // for its kernels before it returns); nullptr on failure.
