@@ -1422,9 +1422,10 @@ __global__ __launch_bounds__(256) void k_enk2_fill(const double *__restrict__ X,
 // like the forward pass.  Normalising each row keeps the rounding of its
 // exponents (differences of numbers of size beta V_B) out of the total; the
 // unnormalised sum over cycle probabilities exp(c + L(m) + R(n) - L(N)) would
-// be one parallel pass, but is 20 times less accurate.  Weights below e^-80
-// of their row are 0 and 64-column chunks without any other are skipped (a
-// bit mask per row).  What bounds it is the serial substitution (1.7 us per
+// be one parallel pass, but is 20 times less accurate.  The potentials may be another xi's or the
+// host's, so a row whose terms lie far from L(n) takes its largest as the
+// scale.  Weights below e^-80 of the row's scale are 0 and 64-column chunks
+// without any other are skipped (a bit mask per row).  What bounds it is the serial substitution (1.7 us per
 // block): N=1024 507 -> 66 us, N=150 41 -> 17 us, against one workgroup doing
 // both.
 constexpr int EST_NMAX = 2015;                       // rows of a workgroup's chunk mask and LDS
@@ -1448,12 +1449,26 @@ __global__ __launch_bounds__(256) void k_est_weights(RecArgs a, const double *__
   if (n <= N) {
     const double *row = a.ENk + tri_row(n), *brow = Bm + tri_row(n);
     const double ln = a.lnn[n], Ln = a.Lf[n];
-    double w[EST_PER], s0 = 0.0, s1 = 0.0;
+    double w[EST_PER], s0 = 0.0, s1 = 0.0, top = NEG;  // w: first the exponents
 #pragma unroll
     for (int i = 0; i < EST_PER; ++i) {
       const int k = 1 + tid + 256 * i;
       const bool ok = k <= n && !(a.xi0 && k != 1);
-      const double x = ok ? ((k - 1) * a.lnxi - a.beta * row[k - 1] - ln) + (a.Lf[n - k] - Ln) : NEG;
+      w[i] = ok ? ((k - 1) * a.lnxi - a.beta * row[k - 1] - ln) + (a.Lf[n - k] - Ln) : NEG;
+      top = fmax(top, w[i]);
+    }
+    top = wave_max_dpp(top);
+    if ((tid & 63) == 0) red[0][tid >> 6] = top;
+    __syncthreads();
+    top = fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3]));
+    // L(n) itself is the row's scale where it belongs to the row (the largest
+    // exponent is then between -ln n and 0), and where the row has no term
+    const double sh = fabs(top) > 20.0 && fabs(top) < 1e200 ? top : 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < EST_PER; ++i) {
+      const int k = 1 + tid + 256 * i;
+      const double x = w[i] - sh;
       w[i] = 0.0;
       if (__any(x > -80.0)) w[i] = exp_if(x > -80.0, x);
       s0 += w[i];
