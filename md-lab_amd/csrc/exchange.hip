@@ -859,7 +859,7 @@ constexpr double REC_BIG = 1e250;
 
 // Forward substitution and (max,+) scan of a block by one wave, lane = row q,
 // coefficients at dg[r * RB + q] (0 or NEG unless r < q), columns r in order:
-//   W_q += A(q, r) W_r          until W leaves `big` (NaN too; false then)
+//   W_q += A(q, r) W_r          (LIMIT: until W leaves `big`, NaN too; false then)
 //   sig_q = max(sig_q, c(q, r) + sig_r)
 // The chain per column is one broadcast (two v_readlane) and one or two FP64
 // operations, about 30 cycles, when its operands wait in registers: each
@@ -874,18 +874,19 @@ __device__ __forceinline__ void rec_cols(const double *dg, int r0, RecCols &x) {
   for (int j = 0; j < 16; ++j) x.d[j] = dg[(r0 + j) * RB + (threadIdx.x & 63)];
 }
 
+template <bool LIMIT>
 __device__ __forceinline__ bool rec_subst(const double *dg, int ncol, double big, double &W) {
   RecCols x, n;
   rec_cols(dg, 0, x);
 #pragma unroll 1
   for (int r0 = 0; r0 < ncol; r0 += 16) {
-    if (!__all(W <= big)) return false;
+    if (LIMIT && !__all(W <= big)) return false;
     rec_cols(dg, min(r0 + 16, RB - 16), n);
 #pragma unroll
     for (int j = 0; j < 16; ++j) W = fma(x.d[j], readlane_d(W, r0 + j), W);
     x = n;
   }
-  return __all(W <= big);
+  return !LIMIT || __all(W <= big);
 }
 
 __device__ __forceinline__ void rec_shift(const double *dg, int ncol, double &sig) {
@@ -1072,7 +1073,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       double W = lane < nrows ? Sm * exp(M - sigma - E) : 0.0;
       // column r of dg holds A(q, r) at row q = lane (0 unless r < q); NaN
       // and overflow fail the vote too
-      const bool in = rec_subst(dg, nrows, a.big, W);
+      const bool in = rec_subst<true>(dg, nrows, a.big, W);
       S.wl[lane] = W;
       if (lane == 0) S.fast = in ? 1 : 0;
       if (in) publish(sigma + E + log(W));
@@ -1126,7 +1127,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       if (wv == 0) {
         double W = 0.0;
         if (lane < nrows && M > NEG && M > sig - 745.0) W = Sm * exp(M - sig);
-        rec_subst(dg, nrows, HUGE_VAL, W);
+        rec_subst<false>(dg, nrows, 0.0, W);
         publish(sig + log(W));
       } else {
         next_acc(true);
@@ -1135,7 +1136,7 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
         // factor of 2 for the rounding of either.
         if (wv == 2 && more) {
           double W = lane == 0 ? 1.0 : 0.0;
-          const bool in = rec_subst(S.dg[cur ^ 1], nrows1, 2.0 * a.big, W);
+          const bool in = rec_subst<true>(S.dg[cur ^ 1], nrows1, 2.0 * a.big, W);
           if (lane == 0) S.past = in ? 0 : 1;
         }
       }
@@ -1470,7 +1471,7 @@ __global__ __launch_bounds__(256) void k_est_weights(RecArgs a, const double *__
       const int k = 1 + tid + 256 * i;
       const double x = w[i] - sh;
       w[i] = 0.0;
-      if (__any(x > -80.0)) w[i] = exp_if(x > -80.0, x);
+      if (__any(!(x <= -80.0))) w[i] = exp_if(!(x <= -80.0), x);  // NaN stays
       s0 += w[i];
       if (w[i] != 0.0) s1 += w[i] * brow[k - 1];
     }
@@ -1535,12 +1536,17 @@ __global__ __launch_bounds__(RT) void k_est_solve(int N, EstArgs o, double *__re
     __syncthreads();
     if (wv == 0) {
       double W = acc[lane];
-      rec_subst(tile[b & 1], nrows, HUGE_VAL, W);
+      rec_subst<false>(tile[b & 1], nrows, 0.0, W);
       res[p0 + lane] = W;
     }
     __syncthreads();
   }
-  if (tid == 0) *out = res[N];
+  // a row without a value (NaN) reaches every later row's sum, with weight 0
+  // too; the chunks passed over above have not added theirs
+  bool bad = false;
+  for (int m = tid; m <= N; m += RT) bad |= res[m] != res[m];
+  bad = __syncthreads_or(bad);
+  if (tid == 0) *out = bad ? __builtin_nan("") : res[N];
 }
 
 // -1/2 sum_{j>=2} (x_{l,j} - x_{l,1}) . f_{l,j} m  partials (md_pimd_x.c:4332-4345)
@@ -1710,7 +1716,7 @@ __global__ __launch_bounds__(SIGN_WG) void k_vi_sign(RecArgs a, const double *__
     if (wv == 0) {
       double W = 0.0;
       if (lane < nrows && rM[lane] > NEG) W = rS[lane] * exp(rM[lane] - sig);
-      rec_subst(tile, nrows, HUGE_VAL, W);
+      rec_subst<false>(tile, nrows, 0.0, W);
       if (lane < nrows) {
         Lp[p0 + lane] = sig + log(fabs(W));
         sgn[p0 + lane] = W >= 0.0 ? 1 : -1;
