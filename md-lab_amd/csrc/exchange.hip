@@ -1671,13 +1671,13 @@ __global__ __launch_bounds__(SIGN_WG) void k_vi_sign(RecArgs a, const double *__
       for (int i = 0; i < NR; ++i) {
         double t = fma(-a.beta, E[i], base + (16 * i) * lv);
         if (x0 && k + 16 * i != 1) t = NEG;
-        if (!__any(t > M[i] - LSE_SKIP)) continue;
+        if (!__any(!(t <= M[i] - LSE_SKIP))) continue;  // NaN counts
         const double mx = wave_max_dpp(t);
         if (mx > M[i]) {
           if (M[i] > NEG) S[i] *= exp(M[i] - mx);
           M[i] = mx;
         }
-        const bool in = on && t > M[i] - LSE_SKIP;
+        const bool in = on && !(t <= M[i] - LSE_SKIP);
         const double e = exp_if(in, t - M[i]);
         S[i] += (neg && ((k - 1) & 1)) != (in && sgn[m] < 0) ? -e : e;
       }
@@ -1707,7 +1707,7 @@ __global__ __launch_bounds__(SIGN_WG) void k_vi_sign(RecArgs a, const double *__
       const int r = lane > j ? j : RB - 1 - j, q = lane > j ? lane : RB - 1 - lane;
       const bool below = q > r;
       const double c = below ? tile[r * RB + q] : NEG;
-      const double e = exp_if(c > NEG, c + sg[r] - sg[q]);
+      const double e = exp_if(!(c <= NEG), c + sg[r] - sg[q]);
       if (below) tile[r * RB + q] = neg && ((q - r - 1) & 1) ? -e : e;
       if (lane <= j) tile[j * RB + lane] = 0.0;
       if (lane <= RB - 1 - j) tile[(RB - 1 - j) * RB + lane] = 0.0;
@@ -1715,7 +1715,7 @@ __global__ __launch_bounds__(SIGN_WG) void k_vi_sign(RecArgs a, const double *__
     __syncthreads();
     if (wv == 0) {
       double W = 0.0;
-      if (lane < nrows && rM[lane] > NEG) W = rS[lane] * exp(rM[lane] - sig);
+      if (lane < nrows && (rM[lane] > NEG || rS[lane] != rS[lane])) W = rS[lane] * exp(rM[lane] - sig);
       rec_subst<false>(tile, nrows, 0.0, W);
       if (lane < nrows) {
         Lp[p0 + lane] = sig + log(fabs(W));
