@@ -187,24 +187,53 @@ int clear_device(void *p, size_t bytes) {
   return 0;
 }
 
-double *host_scratch(size_t n) {
-  static double *buf = nullptr;
-  static size_t cap = 0;
-  if (n > cap) {
-    if (buf) (void)hipHostFree(buf);
-    buf = nullptr;
-    cap = 0;
-    n = n < 1024 ? 1024 : n;
-    if (hipHostMalloc((void **)&buf, n * sizeof(double), hipHostMallocDefault) != hipSuccess) return nullptr;
-    cap = n;
+// Blocks given back: at most kScratchKept of at most kScratchMax doubles (8 MB,
+// a histogram of a million bins), the largest ones; others are freed.
+constexpr int kScratchKept = 4;
+constexpr size_t kScratchMax = 1u << 20;
+struct ScratchBlock {
+  double *p;
+  size_t cap;
+};
+static std::mutex g_scratch_lock;
+static ScratchBlock g_scratch_kept[kScratchKept];  // p nullptr: free place
+
+HostScratch::HostScratch(size_t n) {
+  {
+    std::lock_guard<std::mutex> hold(g_scratch_lock);
+    ScratchBlock *best = nullptr;
+    for (ScratchBlock &b : g_scratch_kept)
+      if (b.p && b.cap >= n && (!best || b.cap < best->cap)) best = &b;
+    if (best) {
+      p = best->p;
+      cap_ = best->cap;
+      best->p = nullptr;
+      return;
+    }
   }
-  return buf;
+  cap_ = std::max<size_t>(n, 1024);
+  if (hipHostMalloc((void **)&p, cap_ * sizeof(double), hipHostMallocDefault) != hipSuccess) p = nullptr;
+}
+
+HostScratch::~HostScratch() {
+  if (p && cap_ <= kScratchMax) {
+    std::lock_guard<std::mutex> hold(g_scratch_lock);
+    ScratchBlock *worst = &g_scratch_kept[0];
+    for (ScratchBlock &b : g_scratch_kept)
+      if (worst->p && (!b.p || b.cap < worst->cap)) worst = &b;
+    if (!worst->p || worst->cap < cap_) {
+      std::swap(worst->p, p);
+      std::swap(worst->cap, cap_);
+    }
+  }
+  if (p) (void)hipHostFree(p);
 }
 
 int device_sums(const double *const *src, const int *n, int count, double *out) {
   // the results go straight to pinned host memory: a copy of them to
   // pageable memory costs as much as the kernels of a small estimator
-  double *h = host_scratch(count);
+  HostScratch scratch(count);
+  double *h = scratch.p;
   if (!h) return -1;
   for (int k = 0; k < count; ++k)
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, rt().s0, src[k], n[k], h + k);

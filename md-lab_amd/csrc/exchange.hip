@@ -2218,7 +2218,8 @@ int exch_batch_force(ExchBatch *b, hipStream_t st) {
 // are gathered into one pinned word by a kernel behind the last step (a copy
 // per replica took 8 us each), and read one by one only when one is set.
 int exch_batch_status(ExchBatch *b) {
-  int *err = (int *)host_scratch(1);
+  HostScratch scratch(1);
+  int *err = (int *)scratch.p;
   if (!err) return -1;
   hipLaunchKernelGGL(kb_rec_error, dim3(1), dim3(256), 0, rt().s0, (const ExRep *)b->chain.reps, b->nrep, err);
   XMD_CHECK(hipGetLastError());
@@ -2269,7 +2270,8 @@ static int run_estimator(DevPimd *p, const double *Bm, double *out) {
   o.P = o.dg + (size_t)nblk * RSQ;
   o.bn = o.P + tri;
   o.mask = (unsigned *)(o.bn + N);
-  double *h = host_scratch(1);
+  HostScratch scratch(1);
+  double *h = scratch.p;
   if (!h) return -1;
   hipLaunchKernelGGL(k_est_weights, dim3(nblk * RB), dim3(256), 0, rt().s0, a, Bm, o);
   hipLaunchKernelGGL(k_est_solve, dim3(1), dim3(RT), 0, rt().s0, N, o, h);
@@ -2630,7 +2632,8 @@ static int vi_sign_grid(DevPimd *p, int n, const double *vi2, double *out) {
     return -1;
   }
   RecArgs a = rec_args(p);
-  double *h = host_scratch(2 * (size_t)n);  // xi', then the factors
+  HostScratch scratch(2 * (size_t)n);
+  double *h = scratch.p;  // xi', then the factors
   if (!h) return -1;
   for (int i = 0; i < n; ++i) h[i] = vi2[i];
   hipStream_t st = rt().s0;

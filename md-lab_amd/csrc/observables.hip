@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 
 #include "xmd_device.h"
 #include "xmd_internal.h"
@@ -302,6 +303,8 @@ static int obs_geo(md_simulation_t_x *sim, ObsGeo &g) {
 
 // Device counts of at least `points` bins, all zero between calls (k_hist_add
 // clears what it has read; a call that failed in between drops the buffer).
+// g_counts_busy is held from obs_counts to the end of add_counts.
+static std::mutex g_counts_busy;
 static unsigned long long *g_counts = nullptr;
 static int g_counts_cap = 0;
 
@@ -326,7 +329,8 @@ static unsigned long long *obs_counts(int points) {
 
 // counts -> stats->fxs[N-1][b] += incr, once per count
 static int add_counts(md_stats_t_x *stats, int points, double incr) {
-  double *fx = stats->fxs[stats->N - 1], *h = host_scratch(points);
+  HostScratch scratch(points);
+  double *fx = stats->fxs[stats->N - 1], *h = scratch.p;
   const hipStream_t st = rt().s0;
   if (h) {
     memcpy(h, fx, points * sizeof(double));
@@ -357,6 +361,7 @@ static DevPimd *obs_pimd(md_pimd_t_x *pimd) {
 }
 
 static int run_pair_hist(PairHist &h, md_stats_t_x *stats, double incr) {
+  std::lock_guard<std::mutex> hold(g_counts_busy);
   unsigned long long *cnt = obs_counts(h.points);
   if (!cnt) return -1;
   const long work = (long)h.a.N * h.b.N;
@@ -391,7 +396,8 @@ static PairHist pair_hist(DevPimd *a, int bead_a, DevPimd *b, int bead_b, md_sim
 static int run_sk(SkArgs &a, md_stats_t_x *stats, int npts, const double *qis_host) {
   if (npts <= 0) return 0;
   hipStream_t st = rt().s0;
-  double *out = host_scratch(4 * (size_t)npts);  // results, then q vectors
+  HostScratch scratch(4 * (size_t)npts);
+  double *out = scratch.p;  // results, then q vectors
   if (!out) return -1;
   a.qis = nullptr;
   if (a.sphere) {
@@ -422,6 +428,7 @@ int md_pimd_calc_density_distribution_x(md_pimd_t_x *pimd, md_stats_t_x *stats, 
   g.incre = rmax / stats->points;
   g.points = stats->points;
   g.image = image;
+  std::lock_guard<std::mutex> hold(g_counts_busy);
   unsigned long long *cnt = obs_counts(g.points);
   if (!cnt) return -1;
   const int nb = p->ds->nb;
@@ -460,6 +467,7 @@ int md_pimd_calc_pair_correlation_2d_x(md_pimd_t_x *pimd, md_stats_t_x *stats, m
   DevPimd *p = obs_pimd(pimd);
   if (!p || !stats || stats->points <= 0 || !box) return -1;
   const int points = stats->points;
+  std::lock_guard<std::mutex> hold(g_counts_busy);
   unsigned long long *cnt = obs_counts(points);
   if (!cnt) return -1;
   const long work = (long)p->P * p->N * p->N;

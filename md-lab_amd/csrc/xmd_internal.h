@@ -133,9 +133,20 @@ int download_pimd(DevPimd *p);
 int clear_device(void *p, size_t bytes);
 
 // Pinned host memory of at least n doubles that kernels read and write
-// directly (grown on demand, kept; used by one call at a time, which waits
-// for its kernels before it returns); nullptr on failure.
-double *host_scratch(size_t n);
+// directly, for the one call that holds it (which waits for its kernels before
+// it returns).  Blocks come from a small pool shared by all threads and go
+// back to it; p is nullptr on failure.
+class HostScratch {
+ public:
+  explicit HostScratch(size_t n);
+  ~HostScratch();
+  HostScratch(const HostScratch &) = delete;
+  HostScratch &operator=(const HostScratch &) = delete;
+  double *p = nullptr;
+
+ private:
+  size_t cap_ = 0;
+};
 
 // reductions: sum of n doubles on device into *out (host), deterministic
 int device_sum(const double *src, int n, double *out);
