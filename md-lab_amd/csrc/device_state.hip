@@ -8,7 +8,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <cstddef>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -136,12 +135,14 @@ __global__ void k_chains_to_device(const md_nhc_t_x *__restrict__ in, double *th
   }
 }
 
-// All but the group size f, which the device does not keep.
-__global__ void k_chains_to_host(md_nhc_t_x *__restrict__ out, const double *th, const double *vth,
+// up: the records of the upload, for the fields the device does not keep
+// (the host's own records are not sent up again).
+__global__ void k_chains_to_host(md_nhc_t_x *out, const md_nhc_t_x *up, const double *th, const double *vth,
                                  const double *Q, int Nf, int nb, int N, int P, int massive, int M) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= Nf) return;
   int e = massive ? (i % 3) * nb + slot_of(i / 3, N, P) : i;
+  out[i].f = up[i].f;
   for (int k = 0; k < M; ++k) {
     out[i].theta[k] = th[k * Nf + e];
     out[i].vtheta[k] = vth[k * Nf + e];
@@ -322,27 +323,15 @@ int ensure_device(md_simulation_t_x *sim) {
 // moves overlap (N=1024 P=32, 22 MB: 2.0 -> 0.6 ms).  One caller at a time.
 constexpr int kCopyThreads = 4;
 constexpr size_t kPieceBytes = 1u << 20, kDirectBytes = 3u << 20;
-constexpr size_t kChainOwn = offsetof(md_nhc_t_x, theta);
 static std::mutex g_copy_busy;
 static char *g_copy_slots = nullptr;  // kCopyThreads pieces, pinned, kept
 
-// Records of `rec` bytes, device memory to host; the first `own` bytes of each
-// are the host's and stay (the chains' group size).
+// Device memory to host in pieces, after everything queued on s0.
 struct HostCopy {
-  char *dst;
-  const char *src;
-  size_t bytes, rec, own;
+  void *dst;
+  const void *src;
+  size_t bytes;
 };
-
-static void take_records(const HostCopy &c, const char *from) {
-  if (!c.own) {
-    memcpy(c.dst, from, c.bytes);
-    return;
-  }
-  for (size_t o = 0; o < c.bytes; o += c.rec) memcpy(c.dst + o + c.own, from + o + c.own, c.rec - c.own);
-}
-
-// The lists' records in pieces, after everything queued on s0.
 
 static int copy_pieces(const HostCopy *list, int count) {
   static hipStream_t lane[kCopyThreads];
@@ -351,8 +340,8 @@ static int copy_pieces(const HostCopy *list, int count) {
   XMD_CHECK(hipStreamSynchronize(rt().s0));
   std::vector<HostCopy> piece;
   for (int i = 0; i < count; ++i)
-    for (size_t o = 0, step = kPieceBytes / list[i].rec * list[i].rec; o < list[i].bytes; o += step)
-      piece.push_back({list[i].dst + o, list[i].src + o, std::min(step, list[i].bytes - o), list[i].rec, list[i].own});
+    for (size_t o = 0; o < list[i].bytes; o += kPieceBytes)
+      piece.push_back({(char *)list[i].dst + o, (const char *)list[i].src + o, std::min(kPieceBytes, list[i].bytes - o)});
   std::atomic<size_t> next{0};
   std::atomic<int> failed{0};
   const int device = rt().device;
@@ -365,7 +354,7 @@ static int copy_pieces(const HostCopy *list, int count) {
           hipStreamSynchronize(lane[t]) != hipSuccess)
         failed = 1;
       else
-        take_records(c, slot);
+        memcpy(c.dst, slot, c.bytes);
     }
   };
   std::thread helper[kCopyThreads - 1];
@@ -395,16 +384,16 @@ int download_sim(DevSim *d) {
   md_nhc_t_x *chains = (md_nhc_t_x *)(direct ? g_copy_slots + bbytes : d->nstage);
   hipLaunchKernelGGL(k_beads_to_host, dim3((nb + 255) / 256), dim3(256), 0, st, beads, d->X, d->V, d->F, d->M, nb,
                      d->N, d->P);
-  hipLaunchKernelGGL(k_chains_to_host, dim3((Nf + 255) / 256), dim3(256), 0, st, chains, d->th, d->vth, d->Q, Nf, nb,
-                     d->N, d->P, d->massive ? 1 : 0, MD_NHC_LENGTH_X);
+  hipLaunchKernelGGL(k_chains_to_host, dim3((Nf + 255) / 256), dim3(256), 0, st, chains, (const md_nhc_t_x *)d->nstage,
+                     d->th, d->vth, d->Q, Nf, nb, d->N, d->P, d->massive ? 1 : 0, MD_NHC_LENGTH_X);
   XMD_CHECK(hipGetLastError());
-  const HostCopy out[2] = {{(char *)sim->particles, (const char *)beads, bbytes, sizeof(md_particle_t_x), 0},
-                           {(char *)sim->nhcs, (const char *)chains, cbytes, sizeof(md_nhc_t_x), kChainOwn}};
   if (direct) {
     XMD_CHECK(hipStreamSynchronize(st));
-    for (const HostCopy &c : out) take_records(c, c.src);
+    memcpy(sim->particles, beads, bbytes);
+    memcpy(sim->nhcs, chains, cbytes);
     return 0;
   }
+  const HostCopy out[2] = {{sim->particles, beads, bbytes}, {sim->nhcs, chains, cbytes}};
   return copy_pieces(out, 2);
 }
 
