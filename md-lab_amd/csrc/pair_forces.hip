@@ -310,8 +310,8 @@ __device__ __forceinline__ void pair_term(double dx, double dy, double dz, const
 // a / b for many a by one divisor: y = RN(1/b), two residual corrections.
 // After the first the quotient is within one ulp, and with a correctly rounded
 // y the second then gives RN(a/b) (Markstein's theorem), provided no residual
-// underflows: const_div_ok holds for 2^-900 <= |a| <= 2^900 and a divisor
-// within 2^+-60 of one.
+// underflows or overflows: for 2^-960 <= |a| <= 2^960 (or a = 0) and a divisor
+// within 2^+-60 of one.  A smaller |a| gives a quotient below 2^-900.
 __device__ __forceinline__ double const_div(double a, double b, double y) {
   double q = a * y;
   q = fma(fma(-q, b, a), y, q);
@@ -319,21 +319,36 @@ __device__ __forceinline__ double const_div(double a, double b, double y) {
 }
 
 // Force on a bead from GAUSS_U others: (dx, dy, dz)[u] -> the terms of
-// pair_term<MODE, false>, to the last bit.  The chains (sqrt, exp, divisions)
-// are free of branches so that they interleave; the divisions by s^2 are
-// const_div's, and a wave with a dividend outside its range (a coordinate in
-// common, a far pair) repeats them plainly.  Issue bound: a rotation was 160
-// FP64 instructions, 65 of them five divisions, and is 130 (tiles and their
-// reduction at N=600 P=64 89 -> 74 us, N=512 P=32 52 -> 46.5; 2, 3 and 4 others
-// at a time measure the same, 2 has the smallest code).
+// pair_term<MODE, false>, to the last bit where they are normal numbers (below
+// 2e-308 within one of their last places).  The chains (sqrt, exp, divisions)
+// are free of branches so that they interleave, and the divisions by s^2 are
+// const_div's for pairs at any distance: the exponent needs no lower bound
+// (below 2^-900 its exp is 1), and the dividends of the force, which run down
+// to the smallest subnormal at 27 ranges, are scaled by 2^120 and the quotients
+// back.  Their upper bound follows from gauss_quick, so that only a wave with
+// an infinite or undefined distance repeats its terms plainly.  Issue bound: a
+// rotation was 160 FP64 instructions, 65 of them five divisions, which are 26
+// now (2, 3 and 4 others at a time measure the same, 2 has the smallest code).
+// Tiles and their reduction, us, plain divisions -> here: N=600 P=64 trap 91 ->
+// 73, periodic 128 -> 108, N=512 P=32 52 -> 46, N=256 P=64 37 -> 34.6, N=24 P=16
+// 18.2 -> 15, the same for ranges from 0.02 to 0.5.  (Unscaled dividends bounded by
+// 2^-900, a wave with a smaller one repeating its terms plainly, took 74, 109, 47,
+// 35 and 15 at a range of 0.5, but 125, 161, 73, 51 and 21 from 0.2 down, where
+// most waves hold a pair 25 .. 27 ranges apart or more.)
 constexpr int GAUSS_U = 2;
+
+// Whether the quotients stay in range for every finite distance: |force| is at
+// most pre 2 d e^(-d^2/s^2) / s^2, d e^(-d^2/s^2) < s.  Others (ranges beyond
+// 2^+-30, strengths beyond 2^800) take the general loop with plain divisions.
+__device__ __forceinline__ bool gauss_quick(double s2, double pre) {
+  return s2 >= 0x1p-60 && s2 <= 0x1p60 && fabs(pre) <= 0x1p800;
+}
 
 template <int MODE>
 __device__ __forceinline__ void gauss_terms(double *dx, double *dy, double *dz, const PairParams &pp, double pre,
-                                            double y, bool y_ok) {
-  constexpr double LO = 0x1p-900, HI = 0x1p900;
-  double a[GAUSS_U], qx[GAUSS_U], qy[GAUSS_U], qz[GAUSS_U];
-  bool in = y_ok;
+                                            double y) {
+  double a[GAUSS_U];
+  bool in = true;
 #pragma unroll
   for (int u = 0; u < GAUSS_U; ++u) {
     if (MODE == PK_PGAUSS) {
@@ -343,17 +358,18 @@ __device__ __forceinline__ void gauss_terms(double *dx, double *dy, double *dz, 
     }
     const double d = sqrt(dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u]);
     a[u] = -d * d;
+    in = in && a[u] >= -0x1p900;
+  }
+  double qx[GAUSS_U], qy[GAUSS_U], qz[GAUSS_U];
+#pragma unroll
+  for (int u = 0; u < GAUSS_U; ++u) {
     const double w = pre * exp(const_div(a[u], pp.s2, y));
-    const double ax = w * (2 * dx[u]), ay = w * (2 * dy[u]), az = w * (2 * dz[u]);
-    const double mn = fmin(fmin(fabs(ax), -a[u]), fmin(fabs(ay), fabs(az)));
-    const double mx = fmax(fmax(fabs(ax), -a[u]), fmax(fabs(ay), fabs(az)));
-    in = in && mn >= LO && mx <= HI;
-    qx[u] = const_div(ax, pp.s2, y);
-    qy[u] = const_div(ay, pp.s2, y);
-    qz[u] = const_div(az, pp.s2, y);
+    qx[u] = const_div(w * (2 * dx[u]) * 0x1p120, pp.s2, y) * 0x1p-120;
+    qy[u] = const_div(w * (2 * dy[u]) * 0x1p120, pp.s2, y) * 0x1p-120;
+    qz[u] = const_div(w * (2 * dz[u]) * 0x1p120, pp.s2, y) * 0x1p-120;
   }
   if (!__all(in)) {
-#pragma unroll 1
+#pragma unroll 1  // (unrolled, more waves fit a SIMD: no faster, and a batch's reciprocal kernels wait 10 us for room)
     for (int u = 0; u < GAUSS_U; ++u) {
       const double w = pre * exp(a[u] / pp.s2);
       qx[u] = w * (2 * dx[u]) / pp.s2;
@@ -417,7 +433,9 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
   jz[t] = jact ? X[2 * nb + base + jl] : 0.0;
   constexpr bool GAUSS = !ENERGY && (MODE == PK_GAUSS || MODE == PK_PGAUSS);
   jm[t] = jact ? M[base + jl] : 1.0;
-  if (GAUSS) jm[t] = 1.0 / jm[t];
+  const double pre = GAUSS ? pp.g / (M_PI * pp.s2) : 0.0;
+  const bool quick = GAUSS && gauss_quick(pp.s2, pre);
+  if (quick) jm[t] = 1.0 / jm[t];
   rx[t] = 0;
   ry[t] = 0;
   rz[t] = 0;
@@ -425,12 +443,10 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
   const bool diag = I == J;
   const int s_lo = diag ? 1 : 0, s_hi = diag ? 32 : 63;
   double fx = 0, fy = 0, fz = 0, e = 0;
-  if (GAUSS) {
+  if (quick) {
     // GAUSS_U rotations at a time: their terms are independent chains (sqrt,
     // exp, divisions), added one rotation after the other
-    const double pre = pp.g / (M_PI * pp.s2), y = 1.0 / pp.s2;
-    const bool y_ok = pp.s2 >= 0x1p-60 && pp.s2 <= 0x1p60;
-    const double im = 1.0 / mi;
+    const double y = 1.0 / pp.s2, im = 1.0 / mi;
     // a diagonal tile of n <= 32 beads has no pair past rotation n - 1
     const int nj = N - J * 64, s_end = diag && nj <= 32 ? nj - 1 : s_hi;
     for (int s = s_lo; s <= s_end; s += GAUSS_U) {
@@ -444,7 +460,7 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
         gy[u] = ok[u] ? yi - jy[j] : 1.0;
         gz[u] = ok[u] ? zi - jz[j] : 1.0;
       }
-      gauss_terms<MODE>(gx, gy, gz, pp, pre, y, y_ok);
+      if constexpr (GAUSS) gauss_terms<MODE>(gx, gy, gz, pp, pre, y);
 #pragma unroll
       for (int u = 0; u < GAUSS_U; ++u) {
         // a lane without a pair adds zeros (at a rotation no two lanes share j)
