@@ -914,6 +914,12 @@ __device__ __forceinline__ void rec_copy_tile(const double *src, double *dst, in
 
 __device__ __forceinline__ void rec_copy_wait() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// The 16 loads of x have been issued together before any is used.
+__device__ __forceinline__ void rec_pin(double *x) {
+#pragma unroll
+  for (int j = 0; j < 16; ++j) __asm__ volatile("" : "+v"(x[j]));
+}
+
 // The solver walks the blocks in order.  Block b is solved in the frame of
 // its k = 1 chain: row q's unknown is W_q = exp(L(q) - sigma - E(q)), with
 // sigma = L(p0) (the block's first row has no in-block predecessor, so its
@@ -950,11 +956,16 @@ __device__ __forceinline__ void rec_copy_wait() { __asm__ volatile("s_waitcnt vm
 // beside wave 0's merge.  What bounds it is the instruction issue of single
 // waves (FP64 at about 6 cycles an instruction, an exp 30 of them) and the
 // serial scan and substitution.  Both directions at UEG N=1024 P=32 with
-// cycles: 755 -> 160 us, 42 -> 9.4 us per block, against one wave loading and
+// cycles: 755 -> 145 us, 42 -> 8.9 us per block, against one wave loading and
 // exponentiating all of a block (11.6 with the frame tried in every block, 16
 // exps per lane in the triangle and 16 in the fold; a fifth wave, so that wave
-// 0 is left the serial parts alone, took 8.7 us per block, but such a workgroup
+// 0 is left the serial parts alone, gained 0.7 us per block, but such a workgroup
 // waits longer for room beside the pair kernels: N=256 trap 4.6 -> 5.4 ms).
+// States without cycles stay in the frame: 70 us, 4.2 per block (frame and exact
+// path in one stretch of code, the exact path's coefficients loaded for every
+// block and one poll for the accumulators: 88).  Each LDS operand list is
+// read into registers as a whole before its use; left to the compiler every
+// read waits for the one before.
 // SOLO: no updater workgroups; the solver folds blocks 0 .. b-1 into block
 // b+1 itself (same order and arithmetic as an updater), so it waits on no
 // other workgroup.
@@ -984,9 +995,12 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
   constexpr int LPW = RB / 4;              // look-ahead columns per lane
   // block 0: coefficients, accumulators (column 0 only), chain offsets
   const int nr0 = min(RB, N);
-  for (int w = tid; w < (nr0 + 15) / 16 * 16 * RB; w += 256) S.dg[0][w] = DGd[w];
-  RecRaw xd;  // this wave's 16 columns of the block on itself, for an exact solve
-  rec_load16<FWD>(a, 1 + lane, 1 + 16 * wv, xd);
+  if (wv != 0) {
+    rec_copy_tile(DGd, S.dg[0], wv - 1);
+    rec_copy_wait();
+  }
+  RecRaw xd;  // this wave's 16 columns of the block on itself, for an exact solve,
+  bool have_xd = false;  // loaded ahead behind an exact block, else when needed
   // this wave's columns of the block of rows p .. p + n - 1 on itself, from xd
   auto own_coefs = [&](int p, int n, double *tile) {
     double c[16];
@@ -1067,115 +1081,51 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
       S.nm[lane] = lane < nrows1 ? m : NEG;
       S.ns[lane] = lane < nrows1 ? sv : 0.0;
     };
-    if (past) {
-    } else if (wv == 0) {
-      sigma = readlane_d(M, 0) + log(readlane_d(Sm, 0));
-      double W = lane < nrows ? Sm * exp(M - sigma - E) : 0.0;
-      // column r of dg holds A(q, r) at row q = lane (0 unless r < q); NaN
-      // and overflow fail the vote too
-      const bool in = rec_subst<true>(dg, nrows, a.big, W);
-      S.wl[lane] = W;
-      if (lane == 0) S.fast = in ? 1 : 0;
-      if (in) publish(sigma + E + log(W));
-    } else {
-      next_acc(false);
-      rec_copy_wait();
-    }
-    if (!past) __syncthreads();
-    const bool fast = !past && S.fast != 0;
-    RecRaw xl;  // block b+1's rows on this block
-    if (fast) {
-      next_acc(true);
-    } else {
-      if (!past || wv == 0) own_coefs(p0, nrows, dg);
-      rec_load16<FWD>(a, p1 + lane, p0 + 16 * wv, xl);
-      __syncthreads();
-      double sig = lane < nrows ? M : NEG;
+    if (!past) {
       if (wv == 0) {
-        rec_shift(dg, nrows, sig);
-        S.sg[lane] = lane < nrows ? sig : NEG;
-      }
-      __syncthreads();
-      // the triangle r < q, two columns to a pass: column r in the lanes above
-      // r, column 63 - r (turned about: row 63 - lane) in those below; the
-      // mirror position of each is outside it and set to 0
-      const double sq = S.sg[lane], sm = S.sg[RB - 1 - lane];
+        sigma = readlane_d(M, 0) + log(readlane_d(Sm, 0));
+        double W = lane < nrows ? Sm * exp(M - sigma - E) : 0.0;
+        // column r of dg holds A(q, r) at row q = lane (0 unless r < q); NaN
+        // and overflow fail the vote too
+        const bool in = rec_subst<true>(dg, nrows, a.big, W);
+        S.wl[lane] = W;
+        if (lane == 0) S.fast = in ? 1 : 0;
+        if (in) publish(sigma + E + log(W));
+      } else {
+        // (as many polls as fit beside the substitution)
 #pragma unroll 1
-      for (int r = 8 * wv; r < 8 * wv + 8; r += 4) {  // rolled: see lse16
-        double e[4];
-        int at[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int w = (r + i) * RB + lane;
-          at[i] = lane > r + i ? w : RSQ - 1 - w;
-          e[i] = dg[at[i]];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const bool up = lane > r + i;
-          const double d = S.sg[up ? r + i : RB - 1 - r - i];
-          e[i] = exp_if(lane != r + i && e[i] > NEG, e[i] + d - (up ? sq : sm));
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          dg[at[i]] = e[i];
-          dg[RSQ - 1 - at[i]] = 0.0;
-        }
+        for (int k = 0; k < 3 && !have; ++k) next_acc(false);
+        rec_copy_wait();
       }
-      if (past && wv != 0) rec_copy_wait();
       __syncthreads();
-      if (wv == 0) {
-        double W = 0.0;
-        if (lane < nrows && M > NEG && M > sig - 745.0) W = Sm * exp(M - sig);
-        rec_subst<false>(dg, nrows, 0.0, W);
-        publish(sig + log(W));
-      } else {
+      if (S.fast != 0) {
+        have_xd = false;
         next_acc(true);
-        // Will block b+1 leave the range?  Its W is at least that of a row 0
-        // alone, W_0 = 1 (every W_q >= 1 and no term is negative), with a
-        // factor of 2 for the rounding of either.
-        if (wv == 2 && more) {
-          double W = lane == 0 ? 1.0 : 0.0;
-          const bool in = rec_subst<true>(S.dg[cur ^ 1], nrows1, 2.0 * a.big, W);
-          if (lane == 0) S.past = in ? 0 : 1;
+        if (!more) break;
+        const double *lp = S.la + wv * RB + lane, *wp = S.wl + wv;
+        double l[LPW], w[LPW], acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < LPW; ++k) {
+          l[k] = lp[4 * k * RB];
+          w[k] = wp[4 * k];
         }
-      }
-      __syncthreads();
-    }
-    if (!more) break;
-    if (!SOLO) rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
-    if (fast) {
-      double acc = 0.0;
+        rec_pin(l);
+        rec_pin(w);
 #pragma unroll
-      for (int k = 0; k < LPW; ++k) acc = fma(S.la[(wv + 4 * k) * RB + lane], S.wl[wv + 4 * k], acc);
-      S.tacc[wv][lane] = acc;
-    } else {
-      // block b folded into row q' = lane from its values (block b is full)
-      double c[16], t[16], m16, s16;
-      rec_conv16<FWD>(a, p1 + lane, p0 + 16 * wv, 16, lane < nrows1, xl, c);
-#pragma unroll
-      for (int j = 0; j < 16; ++j) t[j] = c[j] > NEG ? c[j] + S.lv[16 * wv + j] : NEG;
-      lse16(t, dg + 16 * wv * RB + lane, m16, s16);
-      S.tacc[wv][lane] = m16;
-      S.sacc[wv][lane] = s16;
-    }
-    // SOLO: block b+1's accumulators over blocks 0 .. b-1, folded here
-    double Mf = NEG, Sf = 0.0;
-    if (SOLO && b + 1 >= 2) rec_fold_rows<FWD, false>(a, dir, b + 1, S.pm, S.ps, dg, Mf, Sf);
-    if (SOLO) rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
-    __syncthreads();
-    if (wv != 0) {
-      if (S.past) own_coefs(p1, nrows1, S.dg[cur ^ 1]);  // beside the merge
-    } else {
-      double Mn, Sn;
-      if (SOLO) {
-        Mn = b + 1 >= 2 ? Mf : (lane < nrows1 ? AM[p1 + lane] : NEG);
-        Sn = b + 1 >= 2 ? Sf : (lane < nrows1 ? AS[p1 + lane] : 0.0);
-      } else {
-        Mn = S.nm[lane];
-        Sn = S.ns[lane];
-      }
-      if (fast) {
+        for (int k = 0; k < LPW; ++k) acc = fma(l[k], w[k], acc);
+        S.tacc[wv][lane] = acc;
+        // SOLO: block b+1's accumulators over blocks 0 .. b-1, folded here
+        double Mn = NEG, Sn = 0.0;
+        if (SOLO && b + 1 >= 2) rec_fold_rows<FWD, false>(a, dir, b + 1, S.pm, S.ps, dg, Mn, Sn);
+        __syncthreads();
+        if (wv != 0) continue;
+        if (!SOLO) {
+          Mn = S.nm[lane];
+          Sn = S.ns[lane];
+        } else if (b + 1 < 2) {
+          Mn = lane < nrows1 ? AM[p1 + lane] : NEG;
+          Sn = lane < nrows1 ? AS[p1 + lane] : 0.0;
+        }
         const double Y = (S.tacc[0][lane] + S.tacc[1][lane]) + (S.tacc[2][lane] + S.tacc[3][lane]);
         const bool out = lane < nrows1 && !(Y <= a.big);
         if (lane < nrows1 && !out && Y > 0.0) lse_pair(Mn, Sn, sigma + Dl + En + log(Y), 1.0);
@@ -1192,7 +1142,100 @@ __device__ __forceinline__ void rec_solver(const RecArgs &a, int dir, RecLds &S)
           }
           if (out) lse_pair(Mn, Sn, m, s);
         }
-      } else if (lane < nrows1) {
+        M = Mn;
+        Sm = Sn;
+        E = En;
+        Dl = Dn;
+        continue;
+      }
+    }
+    RecRaw xl;  // block b+1's rows on this block
+    if (!have_xd) rec_load16<FWD>(a, p0 + lane, p0 + 16 * wv, xd);
+    if (!past || wv == 0) own_coefs(p0, nrows, dg);
+    rec_load16<FWD>(a, p1 + lane, p0 + 16 * wv, xl);
+    __syncthreads();
+    double sig = lane < nrows ? M : NEG;
+    if (wv == 0) {
+      rec_shift(dg, nrows, sig);
+      S.sg[lane] = lane < nrows ? sig : NEG;
+    }
+    __syncthreads();
+    // the triangle r < q, two columns to a pass: column r in the lanes above
+    // r, column 63 - r (turned about: row 63 - lane) in those below; the
+    // mirror position of each is outside it and set to 0
+    const double sq = S.sg[lane], sm = S.sg[RB - 1 - lane];
+#pragma unroll 1
+    for (int r = 8 * wv; r < 8 * wv + 8; r += 4) {  // rolled: see lse16
+      double e[4];
+      int at[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int w = (r + i) * RB + lane;
+        at[i] = lane > r + i ? w : RSQ - 1 - w;
+        e[i] = dg[at[i]];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool up = lane > r + i;
+        const double d = S.sg[up ? r + i : RB - 1 - r - i];
+        e[i] = exp_if(lane != r + i && e[i] > NEG, e[i] + d - (up ? sq : sm));
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dg[at[i]] = e[i];
+        dg[RSQ - 1 - at[i]] = 0.0;
+      }
+    }
+    if (past && wv != 0) rec_copy_wait();
+    __syncthreads();
+    if (wv == 0) {
+      double W = 0.0;
+      if (lane < nrows && M > NEG && M > sig - 745.0) W = Sm * exp(M - sig);
+      rec_subst<false>(dg, nrows, 0.0, W);
+      publish(sig + log(W));
+    } else {
+      next_acc(true);
+      // Will block b+1 leave the range?  Its W is at least that of a row 0
+      // alone, W_0 = 1 (every W_q >= 1 and no term is negative), with a
+      // factor of 2 for the rounding of either.
+      if (wv == 2 && more) {
+        double W = lane == 0 ? 1.0 : 0.0;
+        const bool in = rec_subst<true>(S.dg[cur ^ 1], nrows1, 2.0 * a.big, W);
+        if (lane == 0) S.past = in ? 0 : 1;
+      }
+    }
+    __syncthreads();
+    if (!more) break;
+    if (!SOLO) rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
+    have_xd = true;
+    // block b folded into row q' = lane from its values (block b is full)
+    double c[16], t[16], v[16], m16, s16;
+    const double *lv = S.lv + 16 * wv;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = lv[j];
+    rec_pin(v);
+    rec_conv16<FWD>(a, p1 + lane, p0 + 16 * wv, 16, lane < nrows1, xl, c);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) t[j] = c[j] > NEG ? c[j] + v[j] : NEG;
+    lse16(t, dg + 16 * wv * RB + lane, m16, s16);
+    S.tacc[wv][lane] = m16;
+    S.sacc[wv][lane] = s16;
+    // SOLO: block b+1's accumulators over blocks 0 .. b-1, folded here
+    double Mn = NEG, Sn = 0.0;
+    if (SOLO && b + 1 >= 2) rec_fold_rows<FWD, false>(a, dir, b + 1, S.pm, S.ps, dg, Mn, Sn);
+    if (SOLO) rec_load16<FWD>(a, p1 + lane, p1 + 16 * wv, xd);
+    __syncthreads();
+    if (wv != 0) {
+      if (S.past != 0) own_coefs(p1, nrows1, S.dg[cur ^ 1]);  // beside the merge
+    } else {
+      if (!SOLO) {
+        Mn = S.nm[lane];
+        Sn = S.ns[lane];
+      } else if (b + 1 < 2) {
+        Mn = lane < nrows1 ? AM[p1 + lane] : NEG;
+        Sn = lane < nrows1 ? AS[p1 + lane] : 0.0;
+      }
+      if (lane < nrows1) {
         double m = NEG, s = 0.0;
 #pragma unroll
         for (int w = 0; w < 4; ++w) lse_pair(m, s, S.tacc[w][lane], S.sacc[w][lane]);
