@@ -1827,12 +1827,6 @@ static int launch_pair_mode(DevPimd *p, const PairParams &pp, hipStream_t st, do
 // > 0 fixes alpha' L_min, < 0 lets the cost model below choose.
 double g_ewald_split_aL = -1.0;
 
-struct EwaldPlan {
-  double alpha = 0, rc2 = 0, gmax2 = 0;
-  int cube_n = 0;  // >= 0: the reference's k cube; -1: the ball |G|^2 <= gmax2
-  bool own_split = false;
-};
-
 static double lmin3(const double *L) { return fmin(L[0], fmin(L[1], L[2])); }
 static double lmax3(const double *L) { return fmax(L[0], fmax(L[1], L[2])); }
 
@@ -1915,15 +1909,19 @@ static EwaldPlan plan_ewald(const PairParams &pp, int N, int P) {
 }
 
 // Parameters of the full Ewald interaction under its plan.
-static PairParams ewald_params(DevPimd *p, EwaldPlan &pl, double xcut = g_ewald_xcut) {
-  PairParams pp = make_params(p, xcut);
-  pl = plan_ewald(pp, p->N, p->P);
+static PairParams planned(PairParams pp, const EwaldPlan &pl) {
   if (pl.own_split) {
     pp.alpha = pl.alpha;
     pp.rc2 = pl.rc2;
     pp.nsum = 1 << 20;  // coverage comes from r_c alone
   }
   return pp;
+}
+
+static PairParams ewald_params(DevPimd *p, EwaldPlan &pl, double xcut = g_ewald_xcut) {
+  const PairParams pp = make_params(p, xcut);
+  pl = plan_ewald(pp, p->N, p->P);
+  return planned(pp, pl);
 }
 
 // Image enumeration of the real-space kernel for the cutoff of pp (the face
@@ -2258,25 +2256,21 @@ double ewald_split_alpha(DevPimd *p) {
   return ewald_params(p, pl).alpha;
 }
 
-bool pair_ewald_tab(DevPimd *p, int kind) {
-  if (kind != PK_EWALD || !p->ds->uniform_mass) return false;
-  EwaldPlan pl;
-  return near_ok(ewald_params(p, pl));
+bool pair_ewald_tab(DevPimd *p, int kind, EwaldPlan &pl) {
+  return kind == PK_EWALD && p->ds->uniform_mass && near_ok(ewald_params(p, pl));
 }
 
-int launch_pair_ewald_real(DevPimd *p, hipStream_t st) {
-  EwaldPlan pl;
-  PairParams pp = ewald_params(p, pl);
+int launch_pair_ewald_real(DevPimd *p, const EwaldPlan &pl, hipStream_t st) {
+  const PairParams pp = planned(make_params(p), pl);
   if (ensure_tiles(p) || launch_ewald_real_tab(p, pp, st, false)) return -1;
   // the learned stand-in (or the judge step: exact terms plus the
   // surrogate's for comparison) fills the reciprocal-force buffer here
   return p->sur_mode ? surrogate_kspace(p, pair_bufs(p)->tb.Frec, st) : 0;
 }
 
-int launch_pair_kspace(DevPimd *p, hipStream_t st) {
+int launch_pair_kspace(DevPimd *p, const EwaldPlan &pl, hipStream_t st) {
   if (p->sur_mode) return 0;
-  EwaldPlan pl;
-  PairParams pp = ewald_params(p, pl);
+  const PairParams pp = planned(make_params(p), pl);
   KSpace *K = nullptr;
   if (ensure_tiles(p) || launch_recip_phase(p, pp, pl.cube_n, pl.gmax2, st, &K) || launch_sk(p, K, st) ||
       launch_recip_force(p, pp, K, st, pair_bufs(p)->tb.Frec))

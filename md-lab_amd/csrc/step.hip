@@ -134,7 +134,8 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   DevPimd *p = sp.p;
   DevSim *d = p->ds;
   const int kind = sp.pair_kind;
-  const bool ewald = !serial && kind >= 0 && pair_ewald_tab(p, kind);
+  EwaldPlan plan;
+  const bool ewald = !serial && kind >= 0 && pair_ewald_tab(p, kind, plan);
   const Order o = serial ? Order::Serial : force_order(sp, ewald);
   // pair forces without a reciprocal part: with massive thermostats their tile
   // sums and the exchange forces are left for NHC half 2 as well, two launches
@@ -159,7 +160,7 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
     return 0;
   };
   auto real = [&](hipStream_t st) -> int {
-    return rec(8, st) || launch_pair_ewald_real(p, st) || rec(9, st) ? -1 : 0;
+    return rec(8, st) || launch_pair_ewald_real(p, plan, st) || rec(9, st) ? -1 : 0;
   };
   auto bead = [&](hipStream_t st) -> int {
     if (rec(6, st)) return -1;
@@ -173,7 +174,7 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
     return rec(7, st);
   };
   auto kspace = [&](hipStream_t st) -> int {
-    return rec(10, st) || launch_pair_kspace(p, st) || rec(11, st) ? -1 : 0;
+    return rec(10, st) || launch_pair_kspace(p, plan, st) || rec(11, st) ? -1 : 0;
   };
   const bool s2 = pairs_s2 || o == Order::Beside || o == Order::Late;
   if (s2 && o != Order::Late && fork(R.fork2, R.s2)) return -1;

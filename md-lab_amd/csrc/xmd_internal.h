@@ -214,17 +214,25 @@ unsigned pair_alloc_epoch();
 // Real-space Ewald launch choice autotuning (pair_forces.hip): with it on,
 // tune the object's (N, P) bucket before first use (never during capture).
 int autotune_if_needed(DevPimd *p, int kind);
+// Split of the Ewald sum between real and reciprocal space.
+struct EwaldPlan {
+  double alpha = 0, rc2 = 0, gmax2 = 0;
+  int cube_n = 0;  // >= 0: the reference's k cube; -1: the ball |G|^2 <= gmax2
+  bool own_split = false;
+};
+
 // Ewald forces in parts, where pair_ewald_tab says so (Ewald with the table
-// kernels): launch_pair_ewald_real queues the real-space tile kernel (per-tile
+// kernels), under the plan it made (its cost model takes the host 8 us, so a
+// step makes one plan for all parts): launch_pair_ewald_real queues the real-space tile kernel (per-tile
 // partial forces; with the learned stand-in in use, then its kernels),
 // launch_pair_kspace the phase tables, structure factors and reciprocal forces
 // (into a side buffer; nothing with the stand-in).  Both read positions only
 // and may run beside each other and the exchange branch.  After all of them
 // launch_combine_forces adds the real-space, reciprocal and, when Fx is
 // given, exchange end-bead forces into F in the order of the unsplit kernels.
-bool pair_ewald_tab(DevPimd *p, int kind);
-int launch_pair_ewald_real(DevPimd *p, hipStream_t st);
-int launch_pair_kspace(DevPimd *p, hipStream_t st);
+bool pair_ewald_tab(DevPimd *p, int kind, EwaldPlan &pl);
+int launch_pair_ewald_real(DevPimd *p, const EwaldPlan &pl, hipStream_t st);
+int launch_pair_kspace(DevPimd *p, const EwaldPlan &pl, hipStream_t st);
 int launch_combine_forces(DevPimd *p, const double *Fx, hipStream_t st);
 // The parts launch_combine_forces adds, for a fused consumer of F.
 // recip: the reciprocal forces are among them.
