@@ -99,21 +99,22 @@ static Lane main_lane() {
 //           host 10 us a step, one with branches 32, which at N=5 P=6 (36 ->
 //           32) and N=8 P=8 (34 .. 38 -> 35) is what the device takes, so that
 //           a busy host sets the pace; N=24 P=16 38 -> 45
-//   Pairs   the pair branch on s2 and the chain on s0, both from NHC on:
-//           no pair kernel fills the device (trap N=8 P=8 45 -> 34,
-//           N=256 P=64 t 92 -> 88, u 84 -> 65; Ewald N=333 P=27 t 130 -> 118,
-//           N=512 P=32 t 160 -> 147, u 120 -> 122)
-//   Wide    Ewald, smaller still: likewise, the real space apart on s1, in
-//           front of the kernels that follow one another (N=16 P=32 67 -> 51
-//           against Pairs, N=128 P=64 t 89 -> 87, u 88 -> 76, N=256 P=32
-//           t 98 -> 102, u 90 -> 80, N=333 P=27 t 118 -> 122)
+//   Pairs   no Ewald: the pair branch on s2 and the chain on s0, both from NHC
+//           on: no pair kernel fills the device (trap N=8 P=8 45 -> 34, N=256
+//           P=64 t 92 -> 88, u 84 -> 65)
+//   Wide    Ewald, smaller grids: likewise, the real space apart on s1, in
+//           front of the kernels that follow one another (N=16 P=32 t 67 -> 46,
+//           u 46 with a graph of four steps; 20-step calls, Wide and Beside: N=333
+//           P=27 t 109 and 115, u 83 and 102; N=512 P=32 t 134 and 141, u 114 and
+//           121; N=600 t 159 and 158, u 129 and 133; N=700 t 178 and 170, u 139 and
+//           138; with real and reciprocal space on one stream N=333 t 108, u 109,
+//           N=600 t 156, u 152)
 //   Beside  Ewald, the real space on s2 from NHC on, bead-local and reciprocal
-//           forces on s0 after the set-up, the solves on s1 (N=700 P=32 t 177,
-//           u 137, and 161 and 155 with Pairs; N=1024 P=32 t 237, u 184, and
-//           228 and 198 with Late)
+//           forces on s0 after the set-up, the solves on s1 (N=1024 P=32 t 235, u
+//           191, and 226 and 211 with Late)
 //   Late    as Beside, the real space after the set-up and behind the solves:
-//           they are placed first (N=1500 P=32 t 394 -> 328, u 308 -> 318;
-//           N=2001 P=24 t 525 -> 407, u 398 -> 370)
+//           they are placed first (N=1350 P=32 t 348 -> 296, u 267 -> 287; N=1500 t
+//           388 -> 337, u 310 -> 323; N=2001 P=24 t 519 -> 411, u 372 -> 384)
 //   After   no Ewald: pair branch on s0 after the set-up, solves on s1 (trap
 //           N=600 P=64 t 164, u 146; 214 and 161 with Pairs)
 enum class Order { Serial, Line, Pairs, Wide, Beside, Late, After };
@@ -121,7 +122,7 @@ enum class Order { Serial, Line, Pairs, Wide, Beside, Late, After };
 static Order force_order(const StepPlan &sp, bool ewald) {
   const double w = (double)sp.p->N * sp.p->N * sp.p->P;
   if (ewald && sp.p->sur_mode) return Order::Beside;
-  if (ewald) return w < 2.5e6 ? Order::Wide : w < 1.2e7 ? Order::Pairs : w < 5e7 ? Order::Beside : Order::Late;
+  if (ewald) return w < 1.2e7 ? Order::Wide : w < 5e7 ? Order::Beside : Order::Late;
   return w < 1.5e3 ? Order::Line : w < 8e6 ? Order::Pairs : Order::After;
 }
 
@@ -179,7 +180,16 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   const bool s2 = pairs_s2 || o == Order::Beside || o == Order::Late;
   if (s2 && o != Order::Late && fork(R.fork2, R.s2)) return -1;
   if (o == Order::Wide) XMD_CHECK(hipStreamWaitEvent(R.s1, R.fork2, 0));
-  if (o == Order::Beside && real(R.s2)) return -1;
+  // Wide: in a graph the real space is queued last (N=16 P=32 52 -> 46 us per
+  // step); launched one by one it would then wait for the host to queue the
+  // others first (N=600 P=32 u, one step 199 -> 186)
+  bool real_first = o == Order::Beside;
+  if (o == Order::Wide) {
+    hipStreamCaptureStatus capture;
+    XMD_CHECK(hipStreamIsCapturing(R.s0, &capture));
+    real_first = capture == hipStreamCaptureStatusNone;
+  }
+  if (real_first && real(o == Order::Wide ? R.s1 : R.s2)) return -1;
   if (rec(2, R.s0) || (serial ? launch_enk(p, sp.image, R.s0)
                              : launch_enk_prep(p, sp.image, R.s0, ride ? &ride_rep : nullptr)) ||
       rec(3, R.s0))
@@ -194,9 +204,9 @@ static int enqueue_forces(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane 
   // bead-local and pair forces
   if (ride ? rec(6, R.s0) || rec(7, R.s0) : bead(sb)) return -1;
   if (ewald) {
-    if ((o == Order::Pairs && real(sb)) || kspace(sb)) return -1;
+    if (kspace(sb)) return -1;
     if (o == Order::Wide) {
-      if (real(R.s1)) return -1;
+      if (!real_first && real(R.s1)) return -1;
       XMD_CHECK(hipEventRecord(R.join, R.s1));
     }
   } else {
