@@ -249,6 +249,23 @@ static int enqueue_step(StepPlan &sp, hipEvent_t *ev, bool serial, const Lane &R
   return 0;
 }
 
+// Number of nodes and edges of a graph, the edges as pairs of node numbers.
+static int graph_shape(hipGraph_t g, std::vector<int> &shape) {
+  size_t nn = 0, ne = 0;
+  XMD_CHECK(hipGraphGetNodes(g, nullptr, &nn));
+  XMD_CHECK(hipGraphGetEdges(g, nullptr, nullptr, &ne));
+  std::vector<hipGraphNode_t> node(nn), from(ne), to(ne);
+  if (nn) XMD_CHECK(hipGraphGetNodes(g, node.data(), &nn));
+  if (ne) XMD_CHECK(hipGraphGetEdges(g, from.data(), to.data(), &ne));
+  auto number = [&](hipGraphNode_t n) { return (int)(std::find(node.begin(), node.end(), n) - node.begin()); };
+  shape = {(int)nn};
+  for (size_t k = 0; k < ne; ++k) {
+    shape.push_back(number(from[k]));
+    shape.push_back(number(to[k]));
+  }
+  return 0;
+}
+
 // One step of a whole batch, the single-system step's stages with one launch
 // per stage over all replicas.
 struct Batch {
@@ -409,7 +426,9 @@ int md_pimd_run_steps_x(md_pimd_t_x *pimd, const md_pimd_step_config_x *cfg, int
   // step boundary inside the graph).  An
   // executable graph kept from the previous call on the same object is
   // updated in place when the new graph has its topology, which saves the
-  // instantiation.
+  // instantiation.  The edges are compared here: hipGraphExecUpdate has
+  // accepted a graph of as many kernels and edges between others of them, and
+  // then run its kernels under the old edges.
   constexpr int kStepsPerGraph = 4, kLongCall = 32;
   Runtime &R = rt();
   DevPimd *p = sp.p;
@@ -431,10 +450,12 @@ int md_pimd_run_steps_x(md_pimd_t_x *pimd, const md_pimd_step_config_x *cfg, int
   }
   hipGraphExec_t exec = (hipGraphExec_t)p->step_exec;
   bool updated = false;
+  std::vector<int> shape;
+  if (graph_shape(graph, shape)) return -1;
   if (exec) {
     hipGraphNode_t bad = nullptr;
     hipGraphExecUpdateResult res;
-    updated = hipGraphExecUpdate(exec, graph, &bad, &res) == hipSuccess && res == hipGraphExecUpdateSuccess;
+    updated = shape == p->step_shape && hipGraphExecUpdate(exec, graph, &bad, &res) == hipSuccess && res == hipGraphExecUpdateSuccess;
     if (!updated) {
       (void)hipGetLastError();
       XMD_CHECK(hipGraphExecDestroy(exec));
@@ -443,6 +464,7 @@ int md_pimd_run_steps_x(md_pimd_t_x *pimd, const md_pimd_step_config_x *cfg, int
   }
   if (!updated) XMD_CHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
   p->step_exec = exec;
+  p->step_shape = shape;
   XMD_CHECK(hipGraphDestroy(graph));
   for (int s = 0; s < launches; ++s) XMD_CHECK(hipGraphLaunch(exec, R.s0));
   for (int s = eager + launches * per; s < nsteps; ++s)

@@ -110,6 +110,7 @@ struct DevPimd {
   int *done = nullptr;      // finished-workgroup count of k_chain_scan (zero between launches)
   void *pair_bufs = nullptr;  // pair-kernel tile schedule, partial sums and k-space tables (pair_forces.hip)
   void *step_exec = nullptr;  // executable step graph of the last md_pimd_run_steps_x (hipGraphExec_t)
+  std::vector<int> step_shape;  // its edges (step.hip graph_shape)
   void *sur = nullptr;        // Ewald surrogate attached for md_pimd_run_steps_surrogate_x (Surrogate)
   int sur_mode = 0;           // 0 exact reciprocal space, 1 surrogate, 2 judge (exact used, surrogate compared)
   bool enk_dev = false, enk2_dev = false, vbn_dev = false, back_dev = false;
