@@ -114,15 +114,29 @@ static Lane main_lane() {
 //           191, and 226 and 211 with Late)
 //   Late    as Beside, the real space after the set-up and behind the solves:
 //           they are placed first (N=1350 P=32 t 348 -> 296, u 267 -> 287; N=1500 t
-//           388 -> 337, u 310 -> 323; N=2001 P=24 t 519 -> 411, u 372 -> 384)
+//           388 -> 337, u 310 -> 323; N=2001 P=24 t 519 -> 411, u 372 -> 384);
+//           not where no cycles can be (cycles_expected), whose solves stay
+//           short: xi = 0 N=1350 283 -> 263, N=1500 320 -> 305, N=1750 P=27
+//           357 -> 346, N=2001 380 -> 368; Theta = 8 N=1500 323 -> 309
 //   After   no Ewald: pair branch on s0 after the set-up, solves on s1 (trap
 //           N=600 P=64 t 164, u 146; 214 and 161 with Pairs)
 enum class Order { Serial, Line, Pairs, Wide, Beside, Late, After };
 
+// Whether a system in a box may hold permutation cycles to speak of: at xi = 0
+// there are none, and an ideal gas of degeneracy n lambda^3 has about xi n
+// lambda^3 / 5 of its particles in cycles of two (repulsion makes it less), where
+// a row block needs a dozen of its 64 in cycles to leave the solves' short way.
+static bool cycles_expected(const DevPimd *p) {
+  const md_pimd_t_x *h = p->host;
+  const double lambda2 = 2 * M_PI * MD_hBar_X * MD_hBar_X * h->beta / h->sim->particles[0].m;
+  const double n = p->N / (box_L(h->sim, 0) * box_L(h->sim, 1) * box_L(h->sim, 2));
+  return fabs(h->vi) * n * lambda2 * sqrt(lambda2) >= 0.1;
+}
+
 static Order force_order(const StepPlan &sp, bool ewald) {
   const double w = (double)sp.p->N * sp.p->N * sp.p->P;
   if (ewald && sp.p->sur_mode) return Order::Beside;
-  if (ewald) return w < 1.2e7 ? Order::Wide : w < 5e7 ? Order::Beside : Order::Late;
+  if (ewald) return w < 1.2e7 ? Order::Wide : w < 5e7 || !cycles_expected(sp.p) ? Order::Beside : Order::Late;
   return w < 1.5e3 ? Order::Line : w < 8e6 ? Order::Pairs : Order::After;
 }
 
