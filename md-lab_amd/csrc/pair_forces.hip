@@ -463,7 +463,8 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
       if constexpr (GAUSS) gauss_terms<MODE>(gx, gy, gz, pp, pre, y);
 #pragma unroll
       for (int u = 0; u < GAUSS_U; ++u) {
-        // a lane without a pair adds zeros (at a rotation no two lanes share j)
+        // a lane without a pair adds zeros (at a rotation no two lanes share j;
+        // the next rotation's j is another lane's, so the rotations stay in order)
         const int j = (t + s + u) & 63;
         const double hx = ok[u] ? gx[u] : 0.0, hy = ok[u] ? gy[u] : 0.0, hz = ok[u] ? gz[u] : 0.0;
         const double invm = J * 64 + j > i ? jm[j] : im;
@@ -473,6 +474,7 @@ __device__ __forceinline__ void k_pair_tiles_body(int bx, const double *__restri
         rx[j] -= hx * invm;
         ry[j] -= hy * invm;
         rz[j] -= hz * invm;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
     }
   } else {
