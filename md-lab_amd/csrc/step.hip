@@ -469,7 +469,8 @@ int md_pimd_run_steps_x(md_pimd_t_x *pimd, const md_pimd_step_config_x *cfg, int
   if (exec) {
     hipGraphNode_t bad = nullptr;
     hipGraphExecUpdateResult res;
-    updated = shape == p->step_shape && hipGraphExecUpdate(exec, graph, &bad, &res) == hipSuccess && res == hipGraphExecUpdateSuccess;
+    updated = shape == p->step_shape && hipGraphExecUpdate(exec, graph, &bad, &res) == hipSuccess &&
+              res == hipGraphExecUpdateSuccess;
     if (!updated) {
       (void)hipGetLastError();
       XMD_CHECK(hipGraphExecDestroy(exec));
