@@ -721,9 +721,14 @@ __device__ __forceinline__ void lse16(const double *t, double *buf, double &M, d
 //
 // Per direction one solver workgroup (blocks 0, 1, 2, ... in order, with
 // the look-ahead fold) and one updater workgroup per row block G >= 2 (folds
-// blocks 0 .. G-2 into its 64 rows as soon as each is solved).  All of the
-// launch's workgroups are resident from the start, so no block waits for a
-// new dispatch while other kernels fill the device.  The hand-offs carry
+// blocks 0 .. G-2 into its 64 rows as soon as each is solved).  A
+// workgroup holds 113 KB of LDS, so a compute unit takes one, and beside other
+// kernels the launch need not be resident as a whole.  It comes to its end all
+// the same: workgroups are dispatched in the order of their index, a
+// direction's solver first and its updaters by block; an updater waits only
+// for blocks before its own and the solver only for the updater of its next
+// block, the first one not yet done; and the kernels beside it (pair forces)
+// never wait for it, so they drain and leave room.  The hand-offs carry
 // their own readiness: the set-up marks val[] and fin[MS][] with NaN, the
 // solver writes block b's values into val[], an updater its rows' finished
 // accumulators into fin[MS][], both with device-scope relaxed stores (to the
@@ -2219,7 +2224,8 @@ void exch_batch_free(ExchBatch *b) {
   delete b;
 }
 
-// cycle energies (k_chain_scan and k_enk_fill of every replica)
+// cycle energies: springs and links, their prefix sums (a workgroup per
+// replica), the tables
 int exch_batch_enk(ExchBatch *b, hipStream_t st) {
   hipLaunchKernelGGL(kb_chain, dim3(b->chain.total), dim3(256), 0, st, (const ExRep *)b->chain.reps, b->chain.start,
                      b->nrep);

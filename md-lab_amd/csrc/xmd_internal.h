@@ -317,7 +317,7 @@ void batch_table_free(BatchTable &t);
 
 // Per-replica arguments of the bead-local stages; every thread owns one
 // degree of freedom e = d * nb + s of one replica, with the same arithmetic
-// as the single-system kernels above.
+// as integrator.hip's single-system kernels.
 struct BeadRep {
   double *X, *V, *F, *th, *vth;
   const double *M, *Q;
