@@ -23,3 +23,21 @@ def golden():
 def oracle():
     from orc import Oracle
     return Oracle()
+
+
+@pytest.fixture(autouse=True)
+def engine_settings(request):
+    """The engine's settings are process-wide; a GPU test leaves the chain length
+    as it was and the Ewald parameters as a fresh process has them, so that no
+    test measures what another one set."""
+    if request.node.get_closest_marker("gpu") is None:
+        yield
+        return
+    import pyxmd
+    lib = pyxmd.Lib()
+    M = lib.md_get_nhc_length_x()
+    yield
+    lib.md_set_nhc_length_x(M)
+    lib.md_set_coulomb_truc_x(0.0)
+    lib.md_set_coulomb_n_sum_x(0)
+    lib.md_set_ewald_split_x(-1.0)
