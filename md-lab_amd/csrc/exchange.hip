@@ -1560,6 +1560,7 @@ __global__ __launch_bounds__(RT) void k_est_solve(int N, EstArgs o, double *__re
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int NR = RB / (RT / 64);  // rows per wave
   const int nblk = (N + RB - 1) / RB;
+  bool bad = false;
   if (tid == 0) res[0] = 0.0;
   for (int w = tid; w < RSQ; w += RT) tile[0][w] = o.dg[w];
   __syncthreads();
@@ -1586,15 +1587,16 @@ __global__ __launch_bounds__(RT) void k_est_solve(int N, EstArgs o, double *__re
       double W = acc[lane];
       rec_subst<false>(tile[b & 1], nrows, 0.0, W);
       res[p0 + lane] = W;
+      bad |= lane < nrows && W != W;
     }
     __syncthreads();
   }
   // a row without a value (NaN) reaches every later row's sum, with weight 0
   // too; the chunks passed over above have not added theirs
-  bool bad = false;
-  for (int m = tid; m <= N; m += RT) bad |= res[m] != res[m];
-  bad = __syncthreads_or(bad);
-  if (tid == 0) *out = bad ? __builtin_nan("") : res[N];
+  if (wv == 0) {
+    const bool none = __any(bad);
+    if (lane == 0) *out = none ? __builtin_nan("") : res[N];
+  }
 }
 
 // -1/2 sum_{j>=2} (x_{l,j} - x_{l,1}) . f_{l,j} m  partials (md_pimd_x.c:4332-4345)
